@@ -19,11 +19,13 @@ dequantized once (bit-exact) plus bf16 GEMMs with the same rounding points.
 float16 x with float16 adapters (the reference's float16 X_DTYPE / LORA_DTYPE,
 ``:141-143, 745-749``) runs the NF4 GEMM's float16 form at any M, every
 rounding point float16; mixed dtypes raise ``ValueError`` (the caller's torch
-branch then serves them, as for any shape the kernels do not take).  The backward (``:761-930``) keeps the
-reference's gradients and rounding points: grad_x's NF4 product on the fused
-``grpo_nf4_grad_x`` kernel (LoRA part added in its store) below
-``GRAD_X_GEMM_MIN_ROWS`` rows for the shapes it tiles, otherwise dequantize +
-bf16 GEMM; the rank-r products and the weight gradients are bf16 GEMMs.
+branch then serves them, as for any shape the kernels do not take).  The
+backward (``:761-930``) keeps the reference's gradients and rounding points: the
+weight dequantized transposed + one GEMM for grad_x's NF4 product, and
+``grpo_lora_backward`` for everything of rank r (x A^T, g B, both adapter
+gradients, the LoRA part added to grad_x) straight from x and grad_out.  Tensors
+those kernels do not take (``_train_kernels``), and a backward that is itself
+differentiated, run the same products as torch ops.
 """
 
 from __future__ import annotations
@@ -106,8 +108,9 @@ def _bf16_scalar(v: float) -> float:
     return _scalar_as(v, torch.bfloat16)
 
 
-# Rows of grad_out from which grad_x's NF4 product runs as dequantize + bf16
-# GEMM instead of the fused nf4_grad_x kernel.  Measured on MI355X at M = 4096
+# Where the torch ops run (see _train_kernels): rows of grad_out from which
+# grad_x's NF4 product is dequantize + bf16 GEMM instead of the fused nf4_grad_x
+# kernel.  Measured on MI355X at M = 4096
 # over the Qwen2-1.5B projection shapes: the GEMM path is 1.8x (q, o) to 4.2x
 # (gate, up) faster.  Below 1024 rows the fused kernel avoids writing and
 # re-reading the whole dequantized weight for few rows.
@@ -125,11 +128,24 @@ def fused_forward_rows(k: int) -> int:
     return 4096 if k <= 4096 else 1024
 
 
+def _train_kernels(x: torch.Tensor, lora_A: torch.Tensor, lora_B: torch.Tensor,
+                   *rows: torch.Tensor) -> bool:
+    """Whether the HIP kernels of the LoRA side take these tensors (16-byte
+    aligned rows, N and K multiples of 8, rank <= 32, one dtype; tensors without a
+    storage, as under a vmapped backward, are left to the torch ops)."""
+    if x.shape[0] == 0 or lora_B.dtype != x.dtype or not ops.lora_train_workspace_bytes(
+            x.shape[0], lora_B.shape[0], x.shape[1], lora_A.shape[0]):
+        return False
+    try:
+        return all(t.data_ptr() % 16 == 0 for t in (x, lora_A, *rows))
+    except RuntimeError:
+        return False
+
+
 class FusedLoRAFunction(torch.autograd.Function):
     """Forward = one fused NF4+LoRA kernel launch (``lora_forward.py:653-759``);
-    backward = the reference's gradients (``:761-930``): grad_x from the NF4
-    weight on the HIP kernel with the LoRA part added in its store, the
-    rank-r products as plain bf16 GEMMs (float32 accumulation)."""
+    backward = the reference's gradients (``:761-930``), float32 accumulation
+    and one rounding per result or intermediate."""
 
     @staticmethod
     def forward(ctx, x, weight_4bit, quant_state, lora_A, lora_B, scaling, bias):
@@ -145,10 +161,11 @@ class FusedLoRAFunction(torch.autograd.Function):
         if w.dtype != torch.uint8:
             w = w.view(torch.uint8)
         x_flat = x.contiguous().view(m, k)
-        out = torch.empty((m, n), device=x.device, dtype=x.dtype)
         gemm_ok = m <= fused_forward_rows(k) and ops.nf4_gemm_supported(m, n, k, r, blocksize)
         fused = gemm_ok or (dt == torch.bfloat16
                             and ops.nf4_linear_plan(m, n, k, r, 1, blocksize) is not None)
+        out = (torch.empty((m, n), device=x.device, dtype=x.dtype)
+               if fused or m == 0 or n == 0 else None)
         if m > 0 and n > 0 and not fused:
             # the largest batches: W dequantized once (bit-exact), then GEMMs
             # with the kernel's rounding points (lora_forward.py:246-257):
@@ -156,10 +173,15 @@ class FusedLoRAFunction(torch.autograd.Function):
             # y = dt(acc + u), dt = bf16 or float16
             wb = ops.nf4_dequant(w, absmax, code, n * k, blocksize, dtype=dt).view(n, k)
             acc = F.linear(x_flat, wb)
-            if bias is not None:
-                acc = acc + bias.to(acc.dtype)
-            u = F.linear(F.linear(x_flat, lora_A), lora_B)
-            out = torch.add(acc, u * _scalar_as(scaling, dt))
+            b = None if bias is None else bias.to(acc.dtype)
+            if _train_kernels(x_flat, lora_A, lora_B):
+                out = ops.lora_forward_add(acc, x_flat, lora_A.contiguous(), lora_B.contiguous(),
+                                           scaling, None if b is None else b.contiguous())
+            else:
+                if b is not None:
+                    acc = acc + b
+                u = F.linear(F.linear(x_flat, lora_A), lora_B)
+                out = torch.add(acc, u * _scalar_as(scaling, dt))
         elif m > 0 and n > 0:
             ops.nf4_lora_linear(x_flat, w, absmax, code, blocksize, n, bias=bias,
                                 lora_a=lora_A, lora_b=lora_B, scaling=float(scaling), out=out)
@@ -177,7 +199,26 @@ class FusedLoRAFunction(torch.autograd.Function):
         g = grad_out.contiguous().view(m, n)
         if g.dtype != dt:
             g = g.to(dt)
-        grad_bias = g.sum(dim=0) if ctx.has_bias else None  # lora_forward.py:790
+        grad_bias = (g.sum(dim=0) if ctx.has_bias and ctx.needs_input_grad[6]
+                     else None)  # lora_forward.py:790
+        if not torch.is_grad_enabled() and _train_kernels(x_flat, lora_A, lora_B, g):
+            # At 256 rows of 1024 x 1024: 616 us for a layer's four projections
+            # forward and backward against 831 with nf4_grad_x (39 us per call)
+            # and the torch ops below; at 2092 rows of 1536 x 1536 532 against 945.
+            need_x, need_a, need_b = (ctx.needs_input_grad[i] for i in (0, 3, 4))
+            gx = None
+            if need_x:
+                if ops.nf4_dequant_t_supported(w, n, k, ctx.blocksize):
+                    gx = torch.matmul(g, ops.nf4_dequant_t(w, absmax, code, n, k, ctx.blocksize,
+                                                           dtype=dt).t())
+                else:
+                    gx = torch.matmul(g, ops.nf4_dequant(w, absmax, code, n * k, ctx.blocksize,
+                                                         dtype=dt).view(n, k))
+            grad_A, grad_B = ops.lora_backward(x_flat, g, lora_A.contiguous(),
+                                               lora_B.contiguous(), ctx.scaling, grad_x=gx,
+                                               want_a=need_a, want_b=need_b)
+            return (None if gx is None else gx.view(ctx.x_shape), None, None, grad_A, grad_B,
+                    None, grad_bias)
         # scaled_grad = dt(g * dt(scaling)) (:836-837); grad_intermediate,
         # grad_x_lora, xA, grad_B, grad_A: dt GEMMs, float32 accumulation (:839-928)
         sg = g * _scalar_as(ctx.scaling, dt)
