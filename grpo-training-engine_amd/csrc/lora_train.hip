@@ -1,37 +1,36 @@
-// The rank-r side of the NF4 + LoRA linear in training for gfx950: the
-// products x A^T and (g s) B, the adapters' gradients, and the LoRA term's
-// addition to a product of the base weight.  Restates the LoRA parts of
-// _lora_forward_kernel (src/triton_kernels/lora_forward.py:210-257) and of
-// FusedLoRAFunction.backward (:761-930); every rounding point is the 16-bit
-// type's (bf16 or float16), sums are float32:
+// The NF4 + LoRA linear for training batches on gfx950, forward and backward.
+// Restates _lora_forward_kernel (src/triton_kernels/lora_forward.py:107-260) and
+// FusedLoRAFunction.backward (:761-930); every rounding point is the 16-bit type's
+// (bf16 or float16), sums are float32:
 //   xa = dt(x A^T)                    gi = dt(dt(g * dt(s)) B)
 //   grad_A = dt(gi^T x)               grad_B = dt(dt(g * dt(s))^T xa)
-//   grad_x = dt(dt(g W) + dt(gi A))   y = dt(dt(x W^T [+ bias]) + dt(dt(t B^T) * dt(s)))
+//   grad_x = dt(dt(g W) + dt(gi A))   y = dt(dt(dt(x W^T) [+ bias]) + dt(dt(t B^T) * dt(s)))
 //
-// All of them are bound by one read of x and g (M x K and M x N 16-bit values);
-// the r <= 32 columns on the other side make the arithmetic small, so every
-// product is MFMA tiles fed straight from global memory in the row-major
-// layout the caller has: no transposed or scaled copies are written.
-//  * lora_rows_kernel (contraction over the row, x A^T and (g s) B): a
-//    workgroup owns 16 or 32 rows, its 8 waves take 64-column steps round-robin
-//    and meet in LDS.
+// The weight is decoded once per call, not once per row tile: at 512 rows and more
+// the two passes over N x K 16-bit values cost less than the decode repeated.
+// The products of rank r are bound by one read of x and g (M x K and M x N
+// 16-bit values), so they are MFMA tiles fed straight from global memory in the
+// row-major layout the caller has: no transposed or scaled copies are written.
+//  * train_prep_kernel: what the products need, in one launch of independent
+//    workgroups. x A^T and (g s) B (contraction over the row): a workgroup owns 16
+//    rows, its 8 waves take 64-column steps round-robin and meet in LDS. The
+//    weight in 16 bits, row-major or transposed. A transposed with its ranks
+//    padded to 32.
+//  * gemm16 (gemm16.hip): x W^T and g W with the LoRA term in the epilogue.
 //  * lora_wgrad_kernel (contraction over rows m): a lane loads 8 rows x 8
 //    columns and transposes pairs with v_perm, so eight MFMAs cover 128 columns x
 //    32 rows per wave step; the row range is cut into slices that leave float32
-//    partial sums, added in slice order by lora_sum_kernel (or by the add kernel's
-//    extra workgroups).
-//  * lora_add_kernel: the M x N product is read and rewritten once, the rank-r
-//    product on MFMAs with the wide operand in the A position, so a lane holds 16
-//    consecutive columns of one row (two 16-byte accesses).
+//    partial sums, added in slice order by lora_sum_kernel.
 // Measured at 8192 rows, N = K = 3584, r = 16 (bf16; x and g are 58.7 MB each):
-// rows 25.8 us and weight gradients 24.0 us (4.5 and 4.9 TB/s of x and g), add 33
-// us (3.6 TB/s), against about 300 us for the same results as torch products,
-// which wrote scaled, transposed and added copies of g and x (327 us of strided
-// copies, 268 us of adds and 490 us of rank-r GEMMs over the four projections of
-// a layer: 2199 us forward and backward, 1382 with these kernels).
+// backward's preparation 32 us (x, g and the weight: 4.6 TB/s), weight gradients
+// 24 us (4.9 TB/s) + sums 6, forward's preparation 21 us, the two GEMMs 183 and 180
+// us. Forward and backward of q, k, v, o: 2199 us as torch products over the
+// dequantized weight (scaled, transposed and added copies 595 us, rank-r GEMMs
+// 490), 1382 with library GEMMs between these kernels and a pass over the result
+// for the LoRA term (23-48 us each), 1222 with the term in the GEMM's epilogue.
 #include <algorithm>
 
-#include "common.hpp"
+#include "gemm16.hpp"
 #include "nf4_decode.hpp"
 
 using namespace grpo;
@@ -40,34 +39,67 @@ namespace {
 
 constexpr int LT_MAX_R = 32;
 
-// ------------------------------------------------- dequantize, transposed --
+// ------------------------------------------------------------ dequantize --
 
-// WT[k][n] = dt(code[q(n, k)] * absmax): the [K, N] form of nf4_dequant_vec's
-// output (bound by its 2-byte writes: 10.2 us at 3584 x 3584, 2.5 TB/s written;
-// nf4_dequant_vec takes 10.8).  The transposed weight makes grad_x = g W a product
-// of two K-contiguous operands, which the GEMM library runs in 144 us at 8192 rows
-// where the row-major weight takes 168.  A workgroup decodes 64 rows n x 128 columns k (a thread: one row, 32
-// nibbles of one absmax block) and turns the tile over in LDS.
-constexpr int DT_N = 64, DT_K = 128, DT_LD = DT_N + 8;
+struct DequantJob {
+  const uint8_t* w;
+  const float* absmax;
+  const float* code16;
+  uint16_t* out;  // [N][K], or [K][N] transposed
+  int N, K, bs_shift;
+  int blocks;     // workgroups
+};
+
+__device__ __forceinline__ void load_code(const float* code16, float (&code)[16]) {
+#pragma unroll
+  for (int j = 0; j < 16; ++j) code[j] = load_uniform(code16 + j);
+}
+
+// Row-major: a thread decodes 8 nibbles at a time, so a wave stores 1 KiB runs.
+constexpr int DQ_PER = 8 * 512 * 4;  // values per workgroup
 
 template <bool F16>
-__global__ void __launch_bounds__(256) nf4_dequant_t_kernel(const uint8_t* __restrict__ w,
-                                                            const float* __restrict__ absmax,
-                                                            const float* __restrict__ code16,
-                                                            uint16_t* __restrict__ out, int N,
-                                                            int K, int bs_shift) {
-  __shared__ __align__(16) uint16_t t[DT_K * DT_LD];
-  const int tid = threadIdx.x;
-  const int n0 = blockIdx.y * DT_N, k0 = blockIdx.x * DT_K;
-  {
-    const int nl = tid & 63, kl = 32 * (tid >> 6);
-    const int n = min(n0 + nl, N - 1), k = min(k0 + kl, K - 32);
-    const int64_t e = (int64_t)n * K + k;
-    const uint4 wv = *reinterpret_cast<const uint4*>(w + e / 2);
-    const float a = absmax[e >> bs_shift];
-    float code[16];
+__device__ __forceinline__ void dequant_rows(const DequantJob& j, int b) {
+  float code[16];
+  load_code(j.code16, code);
+  const int64_t total = (int64_t)j.N * j.K;  // a multiple of 32
+  int64_t e[4];
+  uint32_t wv[4];
+  float a[4];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) code[j] = code16[j];
+  for (int i = 0; i < 4; ++i) {
+    e[i] = (int64_t)b * DQ_PER + 8 * (threadIdx.x + 512 * i);
+    const int64_t ec = min(e[i], total - 8);
+    wv[i] = *reinterpret_cast<const uint32_t*>(j.w + ec / 2);
+    a[i] = j.absmax[ec >> j.bs_shift];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint4 v = decode8(wv[i], make_lut<F16>(code, a[i]));  // [0,2,4,6,1,3,5,7]
+    if (e[i] < total)
+      *reinterpret_cast<uint4*>(j.out + e[i]) =
+          make_uint4(perm(v.z, v.x, 0x05040100u), perm(v.z, v.x, 0x07060302u),
+                     perm(v.w, v.y, 0x05040100u), perm(v.w, v.y, 0x07060302u));
+  }
+}
+
+// Transposed, out[k][n] = dt(code[q(n, k)] * absmax): a workgroup decodes 128
+// rows n x 128 columns k (a thread: one row, 32 nibbles of one absmax block) and
+// turns the tile over in LDS.
+constexpr int DT = 128, DT_LD = DT + 8;
+
+template <bool F16>
+__device__ __forceinline__ void dequant_tile_t(const DequantJob& j, int b, uint16_t* t) {
+  const int kt = (j.K + DT - 1) / DT;
+  const int tid = threadIdx.x, n0 = (b / kt) * DT, k0 = (b % kt) * DT;
+  {
+    const int nl = tid & (DT - 1), kl = 32 * (tid / DT);
+    const int n = min(n0 + nl, j.N - 1), k = min(k0 + kl, j.K - 32);
+    const int64_t e = (int64_t)n * j.K + k;
+    const uint4 wv = *reinterpret_cast<const uint4*>(j.w + e / 2);
+    const float a = j.absmax[e >> j.bs_shift];
+    float code[16];
+    load_code(j.code16, code);
     const Lut lut = make_lut<F16>(code, a);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -82,13 +114,19 @@ __global__ void __launch_bounds__(256) nf4_dequant_t_kernel(const uint8_t* __res
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < DT_K * DT_N / 8 / 256; ++i) {
-    const int c = tid + 256 * i, kl = c >> 3, nl = 8 * (c & 7);
+  for (int i = 0; i < DT * DT / 8 / 512; ++i) {
+    const int c = tid + 512 * i, kl = c / (DT / 8), nl = 8 * (c % (DT / 8));
     const int k = k0 + kl, n = n0 + nl;
-    if (k < K && n < N)  // N % 8 == 0
-      *reinterpret_cast<uint4*>(out + (int64_t)k * N + n) =
+    if (k < j.K && n < j.N)  // N % 8 == 0
+      *reinterpret_cast<uint4*>(j.out + (int64_t)k * j.N + n) =
           *reinterpret_cast<const uint4*>(t + kl * DT_LD + nl);
   }
+}
+
+template <bool F16>
+__global__ void __launch_bounds__(512) nf4_dequant_t_kernel(DequantJob j) {
+  __shared__ __align__(16) uint16_t t[DT * DT_LD];
+  dequant_tile_t<F16>(j, blockIdx.x, t);
 }
 
 // ------------------------------------------------------------ x A^T, g B --
@@ -102,10 +140,16 @@ struct RowsJob {
   uint16_t* cols;       // [16 TC][Mp] (rows m >= M zero) or null
 };
 
-struct RowsArgs {
+// One launch: workgroups [0, rows) run job 0, the next `rows` job 1 (a job
+// without src: none), then dequant.blocks, then those that transpose A.
+struct PrepArgs {
   RowsJob job[2];  // job 0: x A^T, job 1: dt(g s) B
-  int M, Mp, r;
+  int M, Mp, r, rows;
   float scaling;
+  DequantJob dequant;
+  const uint16_t* la;  // A [r][K]
+  uint16_t* at;        // [K][32] (ranks >= r zero)
+  int K;
 };
 
 template <bool F16>
@@ -122,14 +166,13 @@ __device__ __forceinline__ uint4 keep(bool on, uint4 v) {
   return make_uint4(on ? v.x : 0u, on ? v.y : 0u, on ? v.z : 0u, on ? v.w : 0u);
 }
 
-// One job's product over the columns c0 + 16 lg .. + 15 of this lane's rows.
-template <int TC, bool F16, int RT, bool BT>
-__device__ __forceinline__ void rows_product(const RowsJob& j, const RowsArgs& p, int m0, int wave,
-                                             int ln, int lg, f32x4_t (&acc)[RT][TC]) {
+// One job's product for rows m0 .. m0 + 15: wave w takes the 64-column steps w,
+// w + 8, ...; lane (row ln, group lg) the columns c0 + 16 lg .. + 15.
+template <int TC, bool F16, bool BT>
+__device__ __forceinline__ void rows_product(const RowsJob& j, const PrepArgs& p, int m0, int wave,
+                                             int ln, int lg, f32x4_t (&acc)[TC]) {
   const float sc = BT ? round_e<F16>(p.scaling) : 1.f;
-  const uint16_t* xr[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) xr[t] = j.src + (int64_t)min(m0 + 16 * t + ln, p.M - 1) * j.ld;
+  const uint16_t* const xr = j.src + (int64_t)min(m0 + ln, p.M - 1) * j.ld;
   int rk[TC];  // ranks >= r repeat rank r - 1; their results are not used
 #pragma unroll
   for (int tc = 0; tc < TC; ++tc) rk[tc] = min(16 * tc + ln, p.r - 1);
@@ -139,6 +182,7 @@ __device__ __forceinline__ void rows_product(const RowsJob& j, const RowsArgs& p
       const int c = c0 + 16 * lg + 8 * h;
       const bool on = c < j.C;  // C % 8 == 0
       const int cc = on ? c : 0;
+      uint4 a = keep(on, *reinterpret_cast<const uint4*>(xr + cc));
       uint4 b[TC];
 #pragma unroll
       for (int tc = 0; tc < TC; ++tc) {
@@ -154,59 +198,74 @@ __device__ __forceinline__ void rows_product(const RowsJob& j, const RowsArgs& p
         }
         b[tc] = keep(on, b[tc]);
       }
+      if (BT) a = scale8<F16>(a, sc);
 #pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        uint4 a = keep(on, *reinterpret_cast<const uint4*>(xr[t] + cc));
-        if (BT) a = scale8<F16>(a, sc);
-#pragma unroll
-        for (int tc = 0; tc < TC; ++tc) acc[t][tc] = mfma16x16x32_e<F16>(a, b[tc], acc[t][tc]);
-      }
+      for (int tc = 0; tc < TC; ++tc) acc[tc] = mfma16x16x32_e<F16>(a, b[tc], acc[tc]);
     }
   }
 }
 
-template <int TC, bool F16, int RT>
-__global__ void __launch_bounds__(512) lora_rows_kernel(RowsArgs p) {
+template <int TC, bool F16>
+__device__ __forceinline__ void rows_tile(const PrepArgs& p, int b, float* red) {
   constexpr int LD = 16 * TC + 1;
-  __shared__ float red[8][16 * RT][LD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 15, lg = lane >> 4;
-  const int m0 = blockIdx.x * 16 * RT;
-  const bool bt = blockIdx.y != 0;
+  const bool bt = b >= p.rows;
   const RowsJob j = bt ? p.job[1] : p.job[0];
   if (!j.src) return;
-  f32x4_t acc[RT][TC];
+  const int m0 = 16 * (bt ? b - p.rows : b);
+  f32x4_t acc[TC];
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
-#pragma unroll
-    for (int tc = 0; tc < TC; ++tc) acc[t][tc] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int tc = 0; tc < TC; ++tc) acc[tc] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if (bt)
-    rows_product<TC, F16, RT, true>(j, p, m0, wave, ln, lg, acc);
+    rows_product<TC, F16, true>(j, p, m0, wave, ln, lg, acc);
   else
-    rows_product<TC, F16, RT, false>(j, p, m0, wave, ln, lg, acc);
+    rows_product<TC, F16, false>(j, p, m0, wave, ln, lg, acc);
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int tc = 0; tc < TC; ++tc)
 #pragma unroll
-    for (int tc = 0; tc < TC; ++tc)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) red[wave][16 * t + 4 * lg + q][16 * tc + ln] = acc[t][tc][q];
+    for (int q = 0; q < 4; ++q) red[(16 * wave + 4 * lg + q) * LD + 16 * tc + ln] = acc[tc][q];
   __syncthreads();
-  // the eight waves' sums in wave order; consecutive threads: consecutive rows
-  // of one rank, so the transposed form leaves in runs
-  for (int i = tid; i < 16 * RT * 32; i += 512) {
-    const int row = i & (16 * RT - 1), rank = i / (16 * RT), m = m0 + row;
-    uint16_t v = 0;
-    if (rank < p.r && m < p.M) {
-      float s = red[0][row][rank];
+  // one value per thread, the eight waves' sums in wave order; consecutive
+  // threads: consecutive rows of one rank, so the transposed form leaves in runs
+  const int row = tid & 15, rank = tid >> 4, m = m0 + row;
+  uint16_t v = 0;
+  if (rank < p.r && m < p.M) {
+    float s = red[row * LD + rank];
 #pragma unroll
-      for (int w = 1; w < 8; ++w) s += red[w][row][rank];
-      v = f2e<F16>(s);
-    }
-    if (m < p.Mp) {
-      if (j.rows) j.rows[(int64_t)m * 32 + rank] = v;
-      if (j.cols && rank < 16 * TC) j.cols[(int64_t)rank * p.Mp + m] = v;
-    }
+    for (int w = 1; w < 8; ++w) s += red[(16 * w + row) * LD + rank];
+    v = f2e<F16>(s);
   }
+  if (j.rows) j.rows[(int64_t)m * 32 + rank] = v;  // m < Mp: Mp % 16 == 0
+  if (j.cols && rank < 16 * TC) j.cols[(int64_t)rank * p.Mp + m] = v;
+}
+
+template <int TC, bool F16, bool TR>
+__global__ void __launch_bounds__(512) train_prep_kernel(PrepArgs p) {
+  __shared__ __align__(16) char lds[TR ? DT * DT_LD * 2 : 8 * 16 * (16 * TC + 1) * 4];
+  static_assert(8 * 16 * (16 * TC + 1) * 4 <= DT * DT_LD * 2, "both uses fit");
+  int b = blockIdx.x;
+  if (b < 2 * p.rows) {
+    rows_tile<TC, F16>(p, b, reinterpret_cast<float*>(lds));
+    return;
+  }
+  b -= 2 * p.rows;
+  if (b < p.dequant.blocks) {
+    if (TR)
+      dequant_tile_t<F16>(p.dequant, b, reinterpret_cast<uint16_t*>(lds));
+    else
+      dequant_rows<F16>(p.dequant, b);
+    return;
+  }
+  // thread (column k, ranks 8 c .. 8 c + 7)
+  const int i = (b - p.dequant.blocks) * 512 + threadIdx.x, k = i >> 2, c = 8 * (i & 3);
+  if (k >= p.K) return;
+  uint32_t v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) v[q] = c + q < p.r ? p.la[(int64_t)(c + q) * p.K + k] : 0u;
+  *reinterpret_cast<uint4*>(p.at + (int64_t)k * 32 + c) =
+      make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16),
+                 v[6] | (v[7] << 16));
 }
 
 // ------------------------------------------------- gradients of A and B --
@@ -325,15 +384,15 @@ struct SumArgs {
 
 // Four values per thread, slices in order.
 template <bool F16>
-__device__ __forceinline__ void sum_slices(const SumArgs& p, int64_t i) {
-  int64_t e = 4 * i;
+__global__ void __launch_bounds__(256) lora_sum_kernel(SumArgs p) {
+  int64_t e = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
   const bool isb = e < p.nb;
   if (!isb) e -= p.nb;
   const int64_t n = isb ? p.nb : p.na;
   if (e >= n) return;
   const float* src = (isb ? p.pb : p.pa) + e;
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int k = 0; k < p.S; ++k) {
+  float4 s = *reinterpret_cast<const float4*>(src);
+  for (int k = 1; k < p.S; ++k) {
     const float4 v = *reinterpret_cast<const float4*>(src + k * n);
     s.x += v.x;
     s.y += v.y;
@@ -342,94 +401,6 @@ __device__ __forceinline__ void sum_slices(const SumArgs& p, int64_t i) {
   }
   *reinterpret_cast<uint2*>((isb ? p.gb : p.ga) + e) =
       make_uint2(pack_e2<F16>(s.x, s.y), pack_e2<F16>(s.z, s.w));
-}
-
-// ------------------------------------------------- adding the LoRA term --
-
-struct AddArgs {
-  const uint16_t* t;    // [M][32] rows of t or gi, ranks >= r zero
-  const uint16_t* low;  // FWD: B [C][r]; else A [r][C]
-  const uint16_t* bias; // FWD: [C] or null
-  const uint16_t* src;  // [M][C] the base product
-  uint16_t* out;        // [M][C] (may be src)
-  int64_t lds, ldo;
-  int M, C, r;
-  float scaling;
-  int rows;             // rows per workgroup (a multiple of 16)
-  int tiles_c, blocks;  // workgroups of the add; the rest run sum_slices
-};
-
-template <bool FWD, bool F16>
-__device__ __forceinline__ void add_tile(const AddArgs& p, int bx) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ln = lane & 15, lg = lane >> 4;
-  const int c0 = (bx % p.tiles_c) * 256 + 64 * wave, m0 = (bx / p.tiles_c) * p.rows;
-  // MFMA row i of tile j is column c0 + 16 (i / 4) + 4 j + i % 4: a lane ends
-  // with columns c0 + 16 lg .. + 15 of row m0 + ln
-  uint4 a[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int col = min(c0 + 16 * (ln >> 2) + 4 * j + (ln & 3), p.C - 1);
-    uint32_t v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int rank = 8 * lg + i, rr = min(rank, p.r - 1);
-      const uint16_t e = FWD ? p.low[(int64_t)col * p.r + rr] : p.low[(int64_t)rr * p.C + col];
-      v[i] = rank < p.r ? e : 0u;
-    }
-    a[j] = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16),
-                      v[6] | (v[7] << 16));
-  }
-  const int c = c0 + 16 * lg;
-  const bool on[2] = {c < p.C, c + 8 < p.C};  // C % 8 == 0
-  float bias[16];
-  if (FWD && p.bias) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) bias[i] = e2f<F16>(p.bias[min(c + i, p.C - 1)]);
-  }
-  const float sc = FWD ? round_e<F16>(p.scaling) : 1.f;
-  const int m1 = min(m0 + p.rows, p.M);
-  for (int mb = m0; mb < m1; mb += 16) {
-    const int m = mb + ln, mc = min(m, p.M - 1);
-    const uint16_t* s = p.src + (int64_t)mc * p.lds + c;
-    uint4 sv[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      sv[h] = on[h] ? *reinterpret_cast<const uint4*>(s + 8 * h) : make_uint4(0, 0, 0, 0);
-    const uint4 tv = *reinterpret_cast<const uint4*>(p.t + (int64_t)mc * 32 + 8 * lg);
-    uint32_t o[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4_t u = mfma16x16x32_e<F16>(a[j], tv, f32x4_t{0.f, 0.f, 0.f, 0.f});
-      float v[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int e = 4 * j + q;
-        v[q] = e2f<F16>((uint16_t)(word(sv[e >> 3], (e >> 1) & 3) >> (16 * (e & 1))));
-        float uq = round_e<F16>(u[q]);
-        if (FWD) {
-          if (p.bias) v[q] = round_e<F16>(v[q] + bias[e]);
-          uq = round_e<F16>(uq * sc);
-        }
-        v[q] += uq;
-      }
-      o[2 * j] = pack_e2<F16>(v[0], v[1]);
-      o[2 * j + 1] = pack_e2<F16>(v[2], v[3]);
-    }
-    if (m < p.M) {
-      uint16_t* d = p.out + (int64_t)m * p.ldo + c;
-      if (on[0]) *reinterpret_cast<uint4*>(d) = make_uint4(o[0], o[1], o[2], o[3]);
-      if (on[1]) *reinterpret_cast<uint4*>(d + 8) = make_uint4(o[4], o[5], o[6], o[7]);
-    }
-  }
-}
-
-template <bool FWD, bool F16>
-__global__ void __launch_bounds__(256) lora_add_kernel(AddArgs p, SumArgs s) {
-  if ((int)blockIdx.x < p.blocks)
-    add_tile<FWD, F16>(p, blockIdx.x);
-  else
-    sum_slices<F16>(s, (int64_t)(blockIdx.x - p.blocks) * 256 + threadIdx.x);
 }
 
 // ----------------------------------------------------------------- host --
@@ -445,8 +416,10 @@ int wgrad_slices(int M, int N, int K) {
   return (int)cdiv(steps, cdiv(steps, s));
 }
 
-struct TrainWs {  // byte offsets into the workspace
-  size_t rows, xat, git, pb, pa, total;
+// Workspace of either direction (byte offsets): the 16-bit weight, t or gi by
+// rows, x A^T and gi by columns, A by columns, the partial sums.
+struct TrainWs {
+  size_t w, rows, xat, git, at, pb, pa, total;
 };
 
 TrainWs train_ws(int M, int N, int K, int r) {
@@ -459,117 +432,187 @@ TrainWs train_ws(int M, int N, int K, int r) {
     o += (n + 255) / 256 * 256;
     return at;
   };
+  w.w = take((size_t)N * K * 2);
   w.rows = take(Mp * 32 * 2);
   w.xat = take(R * Mp * 2);
   w.git = take(R * Mp * 2);
+  w.at = take((size_t)K * 32 * 2);
   w.pb = take(S > 1 ? (size_t)S * N * r * 4 : 0);
   w.pa = take(S > 1 ? (size_t)S * K * r * 4 : 0);
   w.total = o;
   return w;
 }
 
-template <bool F16>
-int launch_rows(const RowsArgs& a, int jobs, hipStream_t st) {
-  // 32 rows per workgroup once 16-row workgroups would pass four per CU
-  const bool wide = cdiv(a.Mp, 16) * jobs > 1024;
-  const dim3 grid((unsigned)cdiv(a.Mp, wide ? 32 : 16), (unsigned)jobs);
-  if (a.r > 16) {
-    if (wide) lora_rows_kernel<2, F16, 2><<<grid, 512, 0, st>>>(a);
-    else lora_rows_kernel<2, F16, 1><<<grid, 512, 0, st>>>(a);
-  } else {
-    if (wide) lora_rows_kernel<1, F16, 2><<<grid, 512, 0, st>>>(a);
-    else lora_rows_kernel<1, F16, 1><<<grid, 512, 0, st>>>(a);
-  }
-  return launch_check("lora_rows");
+template <bool F16, bool TR>
+int launch_prep(const PrepArgs& a, hipStream_t st) {
+  const unsigned grid = 2u * a.rows + a.dequant.blocks + (a.at ? (unsigned)cdiv(a.K, 128) : 0u);
+  if (a.r > 16) train_prep_kernel<2, F16, TR><<<grid, 512, 0, st>>>(a);
+  else train_prep_kernel<1, F16, TR><<<grid, 512, 0, st>>>(a);
+  return launch_check("train_prep");
 }
 
-AddArgs add_args(const uint16_t* t, const void* low, const void* bias, const void* src,
-                 int64_t lds, void* out, int64_t ldo, int M, int C, int r, float scaling) {
-  AddArgs a{};
-  a.t = t;
-  a.low = static_cast<const uint16_t*>(low);
-  a.bias = static_cast<const uint16_t*>(bias);
-  a.src = static_cast<const uint16_t*>(src);
-  a.out = static_cast<uint16_t*>(out);
-  a.lds = lds;
-  a.ldo = ldo;
-  a.M = M;
-  a.C = C;
-  a.r = r;
-  a.scaling = scaling;
-  a.tiles_c = (int)cdiv(C, 256);
-  // 64 rows per workgroup while that leaves fewer than 2048 of them
-  a.rows = cdiv(M, 64) * a.tiles_c > 2048 ? 128 : 64;
-  if (cdiv(M, 64) * a.tiles_c < 512) a.rows = 16;
-  a.blocks = a.tiles_c * (int)cdiv(M, a.rows);
-  return a;
+bool train_ok(int M, int N, int K, int r, int blocksize) {
+  return M >= 1 && r >= 1 && r <= LT_MAX_R && blocksize >= 32 &&
+         (blocksize & (blocksize - 1)) == 0 && N % 32 == 0 && K % 32 == 0 &&
+         gemm16_ok(M, N, K, K, K) && gemm16_ok(M, K, N, N, N);
 }
 
-bool train_ok(int M, int N, int K, int r) {
-  return M >= 0 && N >= 8 && K >= 8 && N % 8 == 0 && K % 8 == 0 && r >= 1 && r <= LT_MAX_R;
-}
-
-int train_unsupported() {
-  set_error("shape not supported by the LoRA training kernels (N %% 8 == 0, K %% 8 == 0, "
-            "1 <= r <= 32)");
-  return GRPO_EUNSUPPORTED;
-}
+struct TrainCall {
+  const uint16_t* x;
+  int64_t ldx;
+  const uint8_t* w;
+  const float* absmax;
+  const float* code16;
+  int bs_shift;
+  const uint16_t* la;
+  const uint16_t* lb;
+  int r;
+  float scaling;
+  int M, N, K;
+  char* ws;
+  hipStream_t st;
+};
 
 template <bool F16>
-int run_backward(const uint16_t* x, int64_t ldx, const uint16_t* g, int64_t ldg,
-                 const uint16_t* la, const uint16_t* lb, int r, float scaling, int M, int N, int K,
-                 uint16_t* grad_x, int64_t ldgx, uint16_t* grad_a, uint16_t* grad_b, char* ws,
-                 hipStream_t st) {
-  const TrainWs o = train_ws(M, N, K, r);
-  const int Mp = (int)pad32(M), S = wgrad_slices(M, N, K);
-  uint16_t* const rows = reinterpret_cast<uint16_t*>(ws + o.rows);
-  uint16_t* const xat = reinterpret_cast<uint16_t*>(ws + o.xat);
-  uint16_t* const git = reinterpret_cast<uint16_t*>(ws + o.git);
-  RowsArgs ra{};
-  ra.M = M;
-  ra.Mp = Mp;
-  ra.r = r;
-  ra.scaling = scaling;
-  if (grad_b) ra.job[0] = RowsJob{x, ldx, la, K, nullptr, xat};
+int run_forward(const TrainCall& c, const uint16_t* bias, uint16_t* y, int64_t ldy) {
+  const TrainWs o = train_ws(c.M, c.N, c.K, c.r);
+  uint16_t* const wd = reinterpret_cast<uint16_t*>(c.ws + o.w);
+  uint16_t* const rows = reinterpret_cast<uint16_t*>(c.ws + o.rows);
+  PrepArgs a{};
+  a.M = c.M;
+  a.Mp = (int)pad32(c.M);
+  a.r = c.r;
+  a.job[0] = RowsJob{c.x, c.ldx, c.la, c.K, rows, nullptr};
+  a.rows = a.Mp / 16;
+  a.dequant = DequantJob{c.w, c.absmax, c.code16, wd, c.N, c.K, c.bs_shift,
+                         (int)cdiv((int64_t)c.N * c.K, DQ_PER)};
+  if (int rc = launch_prep<F16, false>(a, c.st)) return rc;
+  Gemm16 g{};
+  g.a = c.x;
+  g.lda = c.ldx;
+  g.b = wd;
+  g.ldb = c.K;
+  g.c = y;
+  g.ldc = ldy;
+  g.M = c.M;
+  g.N = c.N;
+  g.K = c.K;
+  g.t = rows;
+  g.low = c.lb;
+  g.ldl = c.r;
+  g.bias = bias;
+  g.r = c.r;
+  g.scaling = c.scaling;
+  return gemm16_launch(g, GEMM16_LORA, F16, c.st);
+}
+
+template <bool F16>
+int run_backward(const TrainCall& c, const uint16_t* grad, int64_t ldg, uint16_t* grad_x,
+                 int64_t ldgx, uint16_t* grad_a, uint16_t* grad_b) {
+  const TrainWs o = train_ws(c.M, c.N, c.K, c.r);
+  const int Mp = (int)pad32(c.M), S = wgrad_slices(c.M, c.N, c.K);
+  uint16_t* const wt = reinterpret_cast<uint16_t*>(c.ws + o.w);
+  uint16_t* const rows = reinterpret_cast<uint16_t*>(c.ws + o.rows);
+  uint16_t* const xat = reinterpret_cast<uint16_t*>(c.ws + o.xat);
+  uint16_t* const git = reinterpret_cast<uint16_t*>(c.ws + o.git);
+  uint16_t* const at = reinterpret_cast<uint16_t*>(c.ws + o.at);
+  PrepArgs a{};
+  a.M = c.M;
+  a.Mp = Mp;
+  a.r = c.r;
+  a.scaling = c.scaling;
+  a.rows = Mp / 16;
+  a.K = c.K;
+  if (grad_b) a.job[0] = RowsJob{c.x, c.ldx, c.la, c.K, nullptr, xat};
   if (grad_x || grad_a)
-    ra.job[1] = RowsJob{g, ldg, lb, N, grad_x ? rows : nullptr, grad_a ? git : nullptr};
-  if (int rc = launch_rows<F16>(ra, 2, st)) return rc;
-  SumArgs sa{};
-  if (grad_a || grad_b) {
-    WgradArgs w{};
-    w.g = g;
-    w.ldg = ldg;
-    w.x = x;
-    w.ldx = ldx;
-    w.xat = xat;
-    w.git = git;
-    w.M = M;
-    w.Mp = Mp;
-    w.N = N;
-    w.K = K;
-    w.r = r;
-    w.tn = grad_b ? (int)cdiv(N, WG_C) : 0;
-    w.scaling = scaling;
-    w.steps = (int)cdiv(Mp / 32, S);
-    w.gb = grad_b;
-    w.ga = grad_a;
-    if (S > 1) {
-      w.pb = reinterpret_cast<float*>(ws + o.pb);
-      w.pa = reinterpret_cast<float*>(ws + o.pa);
-      sa = SumArgs{w.pb, w.pa, grad_b, grad_a, grad_b ? (int64_t)N * r : 0,
-                   grad_a ? (int64_t)K * r : 0, S};
-    }
-    const dim3 grid((unsigned)(w.tn + (grad_a ? cdiv(K, WG_C) : 0)), (unsigned)S);
-    if (r > 16) lora_wgrad_kernel<2, F16><<<grid, 256, 0, st>>>(w);
-    else lora_wgrad_kernel<1, F16><<<grid, 256, 0, st>>>(w);
-    if (int rc = launch_check("lora_wgrad")) return rc;
+    a.job[1] = RowsJob{grad, ldg, c.lb, c.N, grad_x ? rows : nullptr, grad_a ? git : nullptr};
+  if (grad_x) {
+    a.dequant = DequantJob{c.w, c.absmax, c.code16, wt, c.N, c.K, c.bs_shift,
+                           (int)(cdiv(c.N, DT) * cdiv(c.K, DT))};
+    a.la = c.la;
+    a.at = at;
   }
-  const unsigned sum_blocks = (unsigned)cdiv(cdiv(sa.nb + sa.na, 4), 256);
-  AddArgs a{};
-  if (grad_x) a = add_args(rows, la, nullptr, grad_x, ldgx, grad_x, ldgx, M, K, r, 1.f);
-  if (a.blocks + sum_blocks == 0) return GRPO_OK;
-  lora_add_kernel<false, F16><<<a.blocks + sum_blocks, 256, 0, st>>>(a, sa);
-  return launch_check("lora_add");
+  if (int rc = launch_prep<F16, true>(a, c.st)) return rc;
+  if (grad_x) {
+    Gemm16 g{};
+    g.a = grad;
+    g.lda = ldg;
+    g.b = wt;
+    g.ldb = c.N;
+    g.c = grad_x;
+    g.ldc = ldgx;
+    g.M = c.M;
+    g.N = c.K;
+    g.K = c.N;
+    g.t = rows;
+    g.low = at;
+    g.ldl = 32;
+    g.r = c.r;
+    if (int rc = gemm16_launch(g, GEMM16_ADD, F16, c.st)) return rc;
+  }
+  if (!grad_a && !grad_b) return GRPO_OK;
+  WgradArgs w{};
+  w.g = grad;
+  w.ldg = ldg;
+  w.x = c.x;
+  w.ldx = c.ldx;
+  w.xat = xat;
+  w.git = git;
+  w.M = c.M;
+  w.Mp = Mp;
+  w.N = c.N;
+  w.K = c.K;
+  w.r = c.r;
+  w.tn = grad_b ? (int)cdiv(c.N, WG_C) : 0;
+  w.scaling = c.scaling;
+  w.steps = (int)cdiv(Mp / 32, S);
+  w.gb = grad_b;
+  w.ga = grad_a;
+  if (S > 1) {
+    w.pb = reinterpret_cast<float*>(c.ws + o.pb);
+    w.pa = reinterpret_cast<float*>(c.ws + o.pa);
+  }
+  const dim3 grid((unsigned)(w.tn + (grad_a ? cdiv(c.K, WG_C) : 0)), (unsigned)S);
+  if (c.r > 16) lora_wgrad_kernel<2, F16><<<grid, 256, 0, c.st>>>(w);
+  else lora_wgrad_kernel<1, F16><<<grid, 256, 0, c.st>>>(w);
+  if (int rc = launch_check("lora_wgrad")) return rc;
+  if (S == 1) return GRPO_OK;
+  const SumArgs sa{w.pb, w.pa, grad_b, grad_a, grad_b ? (int64_t)c.N * c.r : 0,
+                   grad_a ? (int64_t)c.K * c.r : 0, S};
+  lora_sum_kernel<F16><<<(unsigned)cdiv(sa.nb + sa.na, 1024), 256, 0, c.st>>>(sa);
+  return launch_check("lora_sum");
+}
+
+// The checks both directions share.
+int train_check(const void* x, int64_t ldx, const uint8_t* w, const float* absmax,
+                const float* code16, int blocksize, const void* lora_a, const void* lora_b, int r,
+                int M, int N, int K, void* workspace, size_t workspace_bytes) {
+  if (!train_ok(M, N, K, r, blocksize)) {
+    set_error("shape not supported by the NF4 + LoRA training kernels (N %% 32 == 0, K %% 32 == "
+              "0, 1 <= r <= 32, power-of-two blocksize >= 32)");
+    return GRPO_EUNSUPPORTED;
+  }
+  if (!x || !w || !absmax || !code16 || !lora_a || !lora_b || !workspace)
+    return einval("null pointer");
+  if (ldx < K || ldx % 8 || ldx >= (1 << 22) || !aligned16(x))
+    return einval("x rows must be 16-byte aligned");
+  if (!aligned16(w) || !aligned16(lora_a) || !aligned16(workspace))
+    return einval("w, lora_a and the workspace must be 16-byte aligned");
+  if (workspace_bytes < train_ws(M, N, K, r).total) {
+    set_error("workspace too small");
+    return GRPO_EWORKSPACE;
+  }
+  return GRPO_OK;
+}
+
+TrainCall train_call(const void* x, int64_t ldx, const uint8_t* w, const float* absmax,
+                     const float* code16, int blocksize, const void* lora_a, const void* lora_b,
+                     int r, float scaling, int M, int N, int K, void* workspace,
+                     grpo_stream_t stream) {
+  return TrainCall{static_cast<const uint16_t*>(x), ldx, w, absmax, code16,
+                   __builtin_ctz((unsigned)blocksize), static_cast<const uint16_t*>(lora_a),
+                   static_cast<const uint16_t*>(lora_b), r, scaling, M, N, K,
+                   static_cast<char*>(workspace), as_stream(stream)};
 }
 
 }  // namespace
@@ -586,79 +629,59 @@ extern "C" int grpo_nf4_dequant_t(const uint8_t* w, const float* absmax, const f
     return GRPO_EUNSUPPORTED;
   }
   if (!aligned16(w) || !aligned16(out)) return einval("w and out must be 16-byte aligned");
-  const dim3 grid((unsigned)cdiv(K, DT_K), (unsigned)cdiv(N, DT_N));
-  const int shift = __builtin_ctz((unsigned)blocksize);
-  hipStream_t st = as_stream(stream);
-  if (f16)
-    nf4_dequant_t_kernel<true><<<grid, 256, 0, st>>>(w, absmax, code16,
-                                                     static_cast<uint16_t*>(out), N, K, shift);
-  else
-    nf4_dequant_t_kernel<false><<<grid, 256, 0, st>>>(w, absmax, code16,
-                                                      static_cast<uint16_t*>(out), N, K, shift);
+  const DequantJob j{w, absmax, code16, static_cast<uint16_t*>(out), N, K,
+                     __builtin_ctz((unsigned)blocksize), (int)(cdiv(N, DT) * cdiv(K, DT))};
+  if (f16) nf4_dequant_t_kernel<true><<<j.blocks, 512, 0, as_stream(stream)>>>(j);
+  else nf4_dequant_t_kernel<false><<<j.blocks, 512, 0, as_stream(stream)>>>(j);
   return launch_check("nf4_dequant_t");
 }
 
-extern "C" size_t grpo_lora_train_workspace_bytes(int M, int N, int K, int r) {
-  return M > 0 && train_ok(M, N, K, r) ? train_ws(M, N, K, r).total : 0;
+extern "C" size_t grpo_nf4_lora_train_workspace_bytes(int M, int N, int K, int r, int blocksize) {
+  return train_ok(M, N, K, r, blocksize) ? train_ws(M, N, K, r).total : 0;
 }
 
-extern "C" int grpo_lora_forward_add(const void* x, int64_t ldx, const void* lora_a,
-                                     const void* lora_b, const void* bias, int r, float scaling,
-                                     void* y, int64_t ldy, int M, int N, int K, int f16,
-                                     void* workspace, size_t workspace_bytes,
-                                     grpo_stream_t stream) {
-  if (!train_ok(M, N, K, r)) return train_unsupported();
-  if (M == 0) return GRPO_OK;
-  if (!x || !lora_a || !lora_b || !y || !workspace) return einval("null pointer");
-  if (ldx < K || ldx % 8 || !aligned16(x)) return einval("x rows must be 16-byte aligned");
+extern "C" int grpo_nf4_lora_train_forward(const void* x, int64_t ldx, const uint8_t* w,
+                                           const float* absmax, const float* code16,
+                                           int blocksize, const void* bias, const void* lora_a,
+                                           const void* lora_b, int r, float scaling, void* y,
+                                           int64_t ldy, int M, int N, int K, int f16,
+                                           void* workspace, size_t workspace_bytes,
+                                           grpo_stream_t stream) {
+  if (int rc = train_check(x, ldx, w, absmax, code16, blocksize, lora_a, lora_b, r, M, N, K,
+                           workspace, workspace_bytes))
+    return rc;
+  if (!y) return einval("null pointer");
   if (ldy < N || ldy % 8 || !aligned16(y)) return einval("y rows must be 16-byte aligned");
-  if (!aligned16(lora_a) || !aligned16(workspace))
-    return einval("lora_a and workspace must be 16-byte aligned");
-  const int Mp = (int)pad32(M);
-  if (workspace_bytes < (size_t)Mp * 64) {
-    set_error("workspace too small");
-    return GRPO_EWORKSPACE;
-  }
-  uint16_t* const rows = static_cast<uint16_t*>(workspace);
-  RowsArgs ra{};
-  ra.M = M;
-  ra.Mp = Mp;
-  ra.r = r;
-  ra.job[0] = RowsJob{static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(lora_a),
-                      K, rows, nullptr};
-  hipStream_t st = as_stream(stream);
-  if (int rc = f16 ? launch_rows<true>(ra, 1, st) : launch_rows<false>(ra, 1, st)) return rc;
-  const AddArgs a = add_args(rows, lora_b, bias, y, ldy, y, ldy, M, N, r, scaling);
-  if (f16) lora_add_kernel<true, true><<<a.blocks, 256, 0, st>>>(a, SumArgs{});
-  else lora_add_kernel<true, false><<<a.blocks, 256, 0, st>>>(a, SumArgs{});
-  return launch_check("lora_add");
+  const TrainCall c = train_call(x, ldx, w, absmax, code16, blocksize, lora_a, lora_b, r, scaling,
+                                 M, N, K, workspace, stream);
+  const uint16_t* const b = static_cast<const uint16_t*>(bias);
+  uint16_t* const o = static_cast<uint16_t*>(y);
+  return f16 ? run_forward<true>(c, b, o, ldy) : run_forward<false>(c, b, o, ldy);
 }
 
-extern "C" int grpo_lora_backward(const void* x, int64_t ldx, const void* grad, int64_t ldg,
-                                  const void* lora_a, const void* lora_b, int r, float scaling,
-                                  int M, int N, int K, int f16, void* grad_x, int64_t ldgx,
-                                  void* grad_a, void* grad_b, void* workspace,
-                                  size_t workspace_bytes, grpo_stream_t stream) {
-  if (!train_ok(M, N, K, r)) return train_unsupported();
-  if (M == 0) return einval("M > 0 required");
+extern "C" int grpo_nf4_lora_train_backward(const void* x, int64_t ldx, const void* grad,
+                                            int64_t ldg, const uint8_t* w, const float* absmax,
+                                            const float* code16, int blocksize,
+                                            const void* lora_a, const void* lora_b, int r,
+                                            float scaling, int M, int N, int K, int f16,
+                                            void* grad_x, int64_t ldgx, void* grad_a,
+                                            void* grad_b, void* workspace,
+                                            size_t workspace_bytes, grpo_stream_t stream) {
+  if (int rc = train_check(x, ldx, w, absmax, code16, blocksize, lora_a, lora_b, r, M, N, K,
+                           workspace, workspace_bytes))
+    return rc;
   if (!grad_x && !grad_a && !grad_b) return GRPO_OK;
-  if (!x || !grad || !lora_a || !lora_b || !workspace) return einval("null pointer");
-  if (ldx < K || ldx % 8 || !aligned16(x)) return einval("x rows must be 16-byte aligned");
-  if (ldg < N || ldg % 8 || !aligned16(grad)) return einval("grad rows must be 16-byte aligned");
+  if (!grad) return einval("null pointer");
+  if (ldg < N || ldg % 8 || ldg >= (1 << 22) || !aligned16(grad))
+    return einval("grad rows must be 16-byte aligned");
   if (grad_x && (ldgx < K || ldgx % 8 || !aligned16(grad_x)))
     return einval("grad_x rows must be 16-byte aligned");
-  if (!aligned16(lora_a) || !aligned16(workspace) || !aligned16(grad_a) || !aligned16(grad_b))
-    return einval("lora_a, the gradients and the workspace must be 16-byte aligned");
-  if (workspace_bytes < train_ws(M, N, K, r).total) {
-    set_error("workspace too small");
-    return GRPO_EWORKSPACE;
-  }
-  auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
-  auto v = [](void* q) { return static_cast<uint16_t*>(q); };
-  hipStream_t st = as_stream(stream);
-  char* ws = static_cast<char*>(workspace);
-  return f16 ? run_backward<true>(u(x), ldx, u(grad), ldg, u(lora_a), u(lora_b), r, scaling, M, N,
-                                  K, v(grad_x), ldgx, v(grad_a), v(grad_b), ws, st)
-             : run_backward<false>(u(x), ldx, u(grad), ldg, u(lora_a), u(lora_b), r, scaling, M, N,
-                                   K, v(grad_x), ldgx, v(grad_a), v(grad_b), ws, st);
+  if (!aligned16(grad_a) || !aligned16(grad_b))
+    return einval("the adapters' gradients must be 16-byte aligned");
+  const TrainCall c = train_call(x, ldx, w, absmax, code16, blocksize, lora_a, lora_b, r, scaling,
+                                 M, N, K, workspace, stream);
+  const uint16_t* const g = static_cast<const uint16_t*>(grad);
+  auto u = [](void* q) { return static_cast<uint16_t*>(q); };
+  return f16 ? run_backward<true>(c, g, ldg, u(grad_x), ldgx, u(grad_a), u(grad_b))
+             : run_backward<false>(c, g, ldg, u(grad_x), ldgx, u(grad_a), u(grad_b));
 }

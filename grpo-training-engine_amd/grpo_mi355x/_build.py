@@ -23,7 +23,7 @@ ARCH = "gfx950"
 
 SOURCES = ("capi.hip", "nf4_linear.hip", "nf4_fold.hip", "nf4_tile.hip", "nf4_gemm.hip",
            "paged_attention.hip", "decode_ops.hip", "lm_head.hip", "sampling.hip",
-           "nf4_backward.hip", "lora_train.hip")
+           "nf4_backward.hip", "gemm16.hip", "lora_train.hip")
 
 # Flags of one source only (machine-scheduler strategies measured per source
 # on the decode step): the folded down_proj kernel is scheduled for

@@ -78,15 +78,16 @@ SIGNATURES = {
     "grpo_nf4_grad_x": (_I32, [_VP, _I64, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _VP, _I64, _VP,
                                 _I64, _VP]),
     "grpo_nf4_dequant_t": (_I32, [_VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _VP]),
-    "grpo_lora_train_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32]),
-    "grpo_lora_forward_add": (
+    "grpo_nf4_lora_train_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32, _I32]),
+    "grpo_nf4_lora_train_forward": (
         _I32,
-        [_VP, _I64, _VP, _VP, _VP, _I32, _F32, _VP, _I64, _I32, _I32, _I32, _I32, _VP, _SZ, _VP],
+        [_VP, _I64, _VP, _VP, _VP, _I32, _VP, _VP, _VP, _I32, _F32, _VP, _I64, _I32, _I32, _I32,
+         _I32, _VP, _SZ, _VP],
     ),
-    "grpo_lora_backward": (
+    "grpo_nf4_lora_train_backward": (
         _I32,
-        [_VP, _I64, _VP, _I64, _VP, _VP, _I32, _F32, _I32, _I32, _I32, _I32, _VP, _I64, _VP, _VP,
-         _VP, _SZ, _VP],
+        [_VP, _I64, _VP, _I64, _VP, _VP, _VP, _I32, _VP, _VP, _I32, _F32, _I32, _I32, _I32, _I32,
+         _VP, _I64, _VP, _VP, _VP, _SZ, _VP],
     ),
     "grpo_nf4_linear_plan": (
         _I32,

@@ -12,20 +12,18 @@ Same call surface and dispatch as the reference's
 * shape/dtype/device problems -> ``ValueError`` (``_validate_inputs``,
   ``:435-487``); rank <= 0 -> ``ValueError`` (``:670-671``).
 
-The fused forward is ``grpo_nf4_lora_linear``: the split-K kernel up to 64
-rows, the NF4 GEMM (weight decoded in the kernel, epilogue fused) beyond, and
-for the largest training batches (``fused_forward_rows``) the weight
-dequantized once (bit-exact) plus bf16 GEMMs with the same rounding points.
-float16 x with float16 adapters (the reference's float16 X_DTYPE / LORA_DTYPE,
-``:141-143, 745-749``) runs the NF4 GEMM's float16 form at any M, every
-rounding point float16; mixed dtypes raise ``ValueError`` (the caller's torch
-branch then serves them, as for any shape the kernels do not take).  The
-backward (``:761-930``) keeps the reference's gradients and rounding points: the
-weight dequantized transposed + one GEMM for grad_x's NF4 product, and
-``grpo_lora_backward`` for everything of rank r (x A^T, g B, both adapter
-gradients, the LoRA part added to grad_x) straight from x and grad_out.  Tensors
-those kernels do not take (``_train_kernels``), and a backward that is itself
-differentiated, run the same products as torch ops.
+The fused forward is ``grpo_nf4_lora_linear`` for few rows (the weight decoded
+as it is multiplied: the split-K kernel up to 64 rows, the NF4 GEMM beyond) and
+``grpo_nf4_lora_train_forward`` from ``train_min_rows`` on (the weight brought to
+16 bits in the call, then an MFMA GEMM with the epilogue in it).  float16 x
+with float16 adapters (the reference's float16 X_DTYPE / LORA_DTYPE, ``:141-143,
+745-749``) has every rounding point float16; mixed dtypes raise ``ValueError``
+(the caller's torch branch then serves them, as for any shape the kernels do not
+take).  The backward (``:761-930``) is ``grpo_nf4_lora_train_backward``: the
+reference's gradients and rounding points, grad_x as one GEMM over the weight
+transposed in 16 bits, everything of rank r straight from x and grad_out.
+Tensors the training kernels do not take (``_train_kernels``), and a backward
+that is itself differentiated, run the same products as torch ops.
 """
 
 from __future__ import annotations
@@ -118,8 +116,8 @@ GRAD_X_GEMM_MIN_ROWS = 1024
 
 
 def fused_forward_rows(k: int) -> int:
-    """Most rows for which the forward runs the fused NF4 GEMM rather than the
-    dequantized weight + hipBLASLt.  Measured on MI355X over the Qwen2-1.5B
+    """Where the training linear does not apply: most rows for which the forward
+    runs the fused NF4 GEMM rather than the dequantized weight + hipBLASLt.  Measured on MI355X over the Qwen2-1.5B
     projection shapes (r = 16): the fused GEMM is faster up to 4096 rows for
     K = 1536 (e.g. gate at 4096 rows: 217 us against 257 us) and up to 1024
     rows for down_proj's K = 8960 (96 against 84 us at 1024 rows with LoRA, 73
@@ -128,16 +126,33 @@ def fused_forward_rows(k: int) -> int:
     return 4096 if k <= 4096 else 1024
 
 
-def _train_kernels(x: torch.Tensor, lora_A: torch.Tensor, lora_B: torch.Tensor,
+def train_min_rows(k: int, dtype: torch.dtype) -> int:
+    """Rows from which the forward runs the training linear (the weight brought
+    to 16 bits in the call, then an MFMA GEMM) rather than the kernels that decode
+    the weight as they multiply.  Measured on MI355X (us, those against this,
+    N x K, r = 16, bf16): 1536 x 1536 19.4 / 19.0 at 256 rows, 24.2 / 19.2 at 512,
+    52.4 / 39.7 at 4096; 3584 x 3584 33.3 / 42.6, 45.8 / 45.4, 194.5 / 109.7;
+    8960 x 1536 35.2 / 36.4, 48.6 / 44.5, 218.5 / 148.5; a long K with few column
+    tiles later, 1536 x 8960 74.0 / 89.1 at 1024 rows, 136.6 / 106.3 at 2048.  In
+    float16 the decoding kernel does not split K: 32.9 / 17.2 (1536 x 1536) and
+    33.2 / 30.1 (8960 x 1536) at 16 rows."""
+    if dtype == torch.float16:
+        return 1
+    return 512 if k <= 4096 else 1536
+
+
+def _train_kernels(w: torch.Tensor, blocksize: int, lora_A: torch.Tensor, lora_B: torch.Tensor,
                    *rows: torch.Tensor) -> bool:
-    """Whether the HIP kernels of the LoRA side take these tensors (16-byte
-    aligned rows, N and K multiples of 8, rank <= 32, one dtype; tensors without a
-    storage, as under a vmapped backward, are left to the torch ops)."""
-    if x.shape[0] == 0 or lora_B.dtype != x.dtype or not ops.lora_train_workspace_bytes(
-            x.shape[0], lora_B.shape[0], x.shape[1], lora_A.shape[0]):
+    """Whether ``ops.nf4_lora_train_forward`` / ``_backward`` take these tensors: one
+    dtype, N and K multiples of 32, rank <= 32, a power-of-two blocksize >= 32,
+    16-byte aligned (tensors without a storage, as under a vmapped backward, are
+    left to the torch ops)."""
+    if lora_A.dtype != rows[0].dtype or lora_B.dtype != lora_A.dtype or \
+            not ops.nf4_lora_train_workspace_bytes(rows[0].shape[0], lora_B.shape[0],
+                                                   lora_A.shape[1], lora_A.shape[0], blocksize):
         return False
     try:
-        return all(t.data_ptr() % 16 == 0 for t in (x, lora_A, *rows))
+        return all(t.data_ptr() % 16 == 0 for t in (w, lora_A, *rows))
     except RuntimeError:
         return False
 
@@ -161,34 +176,39 @@ class FusedLoRAFunction(torch.autograd.Function):
         if w.dtype != torch.uint8:
             w = w.view(torch.uint8)
         x_flat = x.contiguous().view(m, k)
-        gemm_ok = m <= fused_forward_rows(k) and ops.nf4_gemm_supported(m, n, k, r, blocksize)
-        fused = gemm_ok or (dt == torch.bfloat16
-                            and ops.nf4_linear_plan(m, n, k, r, 1, blocksize) is not None)
-        out = (torch.empty((m, n), device=x.device, dtype=x.dtype)
-               if fused or m == 0 or n == 0 else None)
-        if m > 0 and n > 0 and not fused:
-            # the largest batches: W dequantized once (bit-exact), then GEMMs
-            # with the kernel's rounding points (lora_forward.py:246-257):
-            # dt(x W^T), + bias, t = dt(x A^T), u = dt(dt(t B^T) * dt(scaling)),
-            # y = dt(acc + u), dt = bf16 or float16
-            wb = ops.nf4_dequant(w, absmax, code, n * k, blocksize, dtype=dt).view(n, k)
-            acc = F.linear(x_flat, wb)
-            b = None if bias is None else bias.to(acc.dtype)
-            if _train_kernels(x_flat, lora_A, lora_B):
-                out = ops.lora_forward_add(acc, x_flat, lora_A.contiguous(), lora_B.contiguous(),
-                                           scaling, None if b is None else b.contiguous())
-            else:
-                if b is not None:
-                    acc = acc + b
-                u = F.linear(F.linear(x_flat, lora_A), lora_B)
-                out = torch.add(acc, u * _scalar_as(scaling, dt))
-        elif m > 0 and n > 0:
-            ops.nf4_lora_linear(x_flat, w, absmax, code, blocksize, n, bias=bias,
-                                lora_a=lora_A, lora_b=lora_B, scaling=float(scaling), out=out)
+        if m >= train_min_rows(k, dt) and _train_kernels(w, blocksize, lora_A, lora_B, x_flat):
+            out = ops.nf4_lora_train_forward(
+                x_flat, w, absmax, code, blocksize, lora_A.contiguous(), lora_B.contiguous(),
+                float(scaling), None if bias is None else bias.to(dt).contiguous())
+        else:
+            out = FusedLoRAFunction._forward_any(x_flat, w, absmax, code, blocksize, n, lora_A,
+                                                 lora_B, float(scaling), bias)
         ctx.save_for_backward(x_flat, lora_A, lora_B, w, absmax, code)
         ctx.blocksize, ctx.scaling, ctx.has_bias = blocksize, float(scaling), bias is not None
         ctx.x_shape = x.shape
         return out.view(x.shape[:-1] + (n,))
+
+    @staticmethod
+    def _forward_any(x_flat, w, absmax, code, blocksize, n, lora_A, lora_B, scaling, bias):
+        """Few rows, and what the training linear does not take."""
+        (m, k), r, dt = x_flat.shape, lora_A.shape[0], x_flat.dtype
+        out = torch.empty((m, n), device=x_flat.device, dtype=dt)
+        if m == 0 or n == 0:
+            return out
+        gemm_ok = m <= fused_forward_rows(k) and ops.nf4_gemm_supported(m, n, k, r, blocksize)
+        if gemm_ok or (dt == torch.bfloat16
+                       and ops.nf4_linear_plan(m, n, k, r, 1, blocksize) is not None):
+            return ops.nf4_lora_linear(x_flat, w, absmax, code, blocksize, n, bias=bias,
+                                       lora_a=lora_A, lora_b=lora_B, scaling=scaling, out=out)
+        # W dequantized once (bit-exact), then GEMMs with the kernel's rounding
+        # points (lora_forward.py:246-257): dt(x W^T), + bias, t = dt(x A^T),
+        # u = dt(dt(t B^T) * dt(scaling)), y = dt(acc + u), dt = bf16 or float16
+        wb = ops.nf4_dequant(w, absmax, code, n * k, blocksize, dtype=dt).view(n, k)
+        acc = F.linear(x_flat, wb)
+        if bias is not None:
+            acc = acc + bias.to(acc.dtype)
+        u = F.linear(F.linear(x_flat, lora_A), lora_B)
+        return torch.add(acc, u * _scalar_as(scaling, dt))
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -201,24 +221,14 @@ class FusedLoRAFunction(torch.autograd.Function):
             g = g.to(dt)
         grad_bias = (g.sum(dim=0) if ctx.has_bias and ctx.needs_input_grad[6]
                      else None)  # lora_forward.py:790
-        if not torch.is_grad_enabled() and _train_kernels(x_flat, lora_A, lora_B, g):
-            # At 256 rows of 1024 x 1024: 616 us for a layer's four projections
-            # forward and backward against 831 with nf4_grad_x (39 us per call)
-            # and the torch ops below; at 2092 rows of 1536 x 1536 532 against 945.
+        if not torch.is_grad_enabled() and m > 0 and \
+                _train_kernels(w, ctx.blocksize, lora_A, lora_B, x_flat, g):
             need_x, need_a, need_b = (ctx.needs_input_grad[i] for i in (0, 3, 4))
-            gx = None
-            if need_x:
-                if ops.nf4_dequant_t_supported(w, n, k, ctx.blocksize):
-                    gx = torch.matmul(g, ops.nf4_dequant_t(w, absmax, code, n, k, ctx.blocksize,
-                                                           dtype=dt).t())
-                else:
-                    gx = torch.matmul(g, ops.nf4_dequant(w, absmax, code, n * k, ctx.blocksize,
-                                                         dtype=dt).view(n, k))
-            grad_A, grad_B = ops.lora_backward(x_flat, g, lora_A.contiguous(),
-                                               lora_B.contiguous(), ctx.scaling, grad_x=gx,
-                                               want_a=need_a, want_b=need_b)
-            return (None if gx is None else gx.view(ctx.x_shape), None, None, grad_A, grad_B,
-                    None, grad_bias)
+            grad_x, grad_A, grad_B = ops.nf4_lora_train_backward(
+                x_flat, g, w, absmax, code, ctx.blocksize, lora_A.contiguous(),
+                lora_B.contiguous(), ctx.scaling, need_x, need_a, need_b)
+            return (None if grad_x is None else grad_x.view(ctx.x_shape), None, None, grad_A,
+                    grad_B, None, grad_bias)
         # scaled_grad = dt(g * dt(scaling)) (:836-837); grad_intermediate,
         # grad_x_lora, xA, grad_B, grad_A: dt GEMMs, float32 accumulation (:839-928)
         sg = g * _scalar_as(ctx.scaling, dt)

@@ -131,59 +131,67 @@ def nf4_dequant_t(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor
     return out
 
 
-def lora_train_workspace_bytes(m: int, n: int, k: int, r: int) -> int:
-    """Workspace of ``lora_forward_add`` / ``lora_backward`` (0: unsupported shape)."""
-    return int(_lib.library().grpo_lora_train_workspace_bytes(m, n, k, r))
+def nf4_lora_train_workspace_bytes(m: int, n: int, k: int, r: int, blocksize: int) -> int:
+    """Workspace of ``nf4_lora_train_forward`` / ``_backward`` (0: unsupported shape)."""
+    return int(_lib.library().grpo_nf4_lora_train_workspace_bytes(m, n, k, r, int(blocksize)))
 
 
-def _check_train(x, lora_a, lora_b, others):
-    _need_cuda(x, lora_a, lora_b, *others)
+def _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, others):
+    """Shape and dtype checks of the training linear; (m, n, k, r, workspace)."""
+    _need_cuda(x, packed, absmax, code, lora_a, lora_b, *others)
     m, k = x.shape
     n, r = lora_b.shape
     if lora_a.shape != (r, k):
         raise ValueError("lora_A must be [r, K] and lora_B [N, r].")
+    if x.dtype not in (torch.bfloat16, torch.float16):
+        raise ValueError(f"bfloat16 or float16 tensors required, got {x.dtype}.")
     for t in (x, lora_a, lora_b, *others):
         if t is not None and (t.dtype != x.dtype or not t.is_contiguous()):
             raise ValueError("all tensors must be contiguous and of one dtype.")
-    if x.dtype not in (torch.bfloat16, torch.float16):
-        raise ValueError(f"bfloat16 or float16 tensors required, got {x.dtype}.")
-    nbytes = lora_train_workspace_bytes(m, n, k, r)
+    _need_dtype(packed, torch.uint8, "packed weight")
+    _need_dtype(absmax, torch.float32, "absmax")
+    if packed.numel() * 2 < n * k or absmax.numel() * blocksize < n * k or code.numel() != 16:
+        raise ValueError("packed weight or absmax too short for [N, K], or not a 4-bit codebook.")
+    nbytes = nf4_lora_train_workspace_bytes(m, n, k, r, blocksize)
     return m, n, k, r, torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
 
 
-def lora_forward_add(y: torch.Tensor, x: torch.Tensor, lora_a: torch.Tensor,
-                     lora_b: torch.Tensor, scaling: float,
-                     bias: torch.Tensor | None = None) -> torch.Tensor:
-    """``y = dt(dt(y + bias) + dt(dt(dt(x A^T) B^T) * dt(scaling)))`` in place
-    (y [M, N] = the base product, bf16 or float16)."""
+def nf4_lora_train_forward(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor,
+                           code: torch.Tensor, blocksize: int, lora_a: torch.Tensor,
+                           lora_b: torch.Tensor, scaling: float,
+                           bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``y [M, N]`` of the NF4 + LoRA linear for training batches (bf16 or float16)."""
     lib = _lib.device_library()
-    m, n, k, r, ws = _check_train(x, lora_a, lora_b, (y, bias))
-    if y.shape != (m, n) or (bias is not None and bias.numel() != n):
-        raise ValueError(f"y must be [{m}, {n}] and bias [{n}].")
-    _lib.check(lib.grpo_lora_forward_add(
-        x.data_ptr(), k, lora_a.data_ptr(), lora_b.data_ptr(), _lib.ptr(bias), r, float(scaling),
-        y.data_ptr(), n, m, n, k, int(x.dtype == torch.float16), ws.data_ptr(), ws.numel(),
-        _lib.stream_handle(x.device)), "grpo_lora_forward_add")
+    m, n, k, r, ws = _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, (bias,))
+    if bias is not None and bias.numel() != n:
+        raise ValueError(f"bias must have {n} elements.")
+    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    _lib.check(lib.grpo_nf4_lora_train_forward(
+        x.data_ptr(), k, packed.data_ptr(), absmax.data_ptr(), code.data_ptr(), int(blocksize),
+        _lib.ptr(bias), lora_a.data_ptr(), lora_b.data_ptr(), r, float(scaling), y.data_ptr(), n,
+        m, n, k, int(x.dtype == torch.float16), ws.data_ptr(), ws.numel(),
+        _lib.stream_handle(x.device)), "grpo_nf4_lora_train_forward")
     return y
 
 
-def lora_backward(x: torch.Tensor, grad: torch.Tensor, lora_a: torch.Tensor,
-                  lora_b: torch.Tensor, scaling: float, grad_x: torch.Tensor | None = None,
-                  want_a: bool = True, want_b: bool = True):
-    """(grad_A, grad_B) of the LoRA pair (None where not wanted); ``grad_x`` [M, K]
-    (holding the base product's gradient) gets the LoRA part added in place."""
+def nf4_lora_train_backward(x: torch.Tensor, grad: torch.Tensor, packed: torch.Tensor,
+                            absmax: torch.Tensor, code: torch.Tensor, blocksize: int,
+                            lora_a: torch.Tensor, lora_b: torch.Tensor, scaling: float,
+                            want_x: bool = True, want_a: bool = True, want_b: bool = True):
+    """(grad_x, grad_A, grad_B) of the NF4 + LoRA linear (None where not wanted)."""
     lib = _lib.device_library()
-    m, n, k, r, ws = _check_train(x, lora_a, lora_b, (grad, grad_x))
-    if grad.shape != (m, n) or (grad_x is not None and grad_x.shape != (m, k)):
-        raise ValueError(f"grad must be [{m}, {n}] and grad_x [{m}, {k}].")
+    m, n, k, r, ws = _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, (grad,))
+    if grad.shape != (m, n):
+        raise ValueError(f"grad must be [{m}, {n}], got {tuple(grad.shape)}.")
+    gx = torch.empty_like(x) if want_x else None
     ga = torch.empty_like(lora_a) if want_a else None
     gb = torch.empty_like(lora_b) if want_b else None
-    _lib.check(lib.grpo_lora_backward(
-        x.data_ptr(), k, grad.data_ptr(), n, lora_a.data_ptr(), lora_b.data_ptr(), r,
-        float(scaling), m, n, k, int(x.dtype == torch.float16), _lib.ptr(grad_x), k,
-        _lib.ptr(ga), _lib.ptr(gb), ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device)),
-        "grpo_lora_backward")
-    return ga, gb
+    _lib.check(lib.grpo_nf4_lora_train_backward(
+        x.data_ptr(), k, grad.data_ptr(), n, packed.data_ptr(), absmax.data_ptr(),
+        code.data_ptr(), int(blocksize), lora_a.data_ptr(), lora_b.data_ptr(), r, float(scaling),
+        m, n, k, int(x.dtype == torch.float16), _lib.ptr(gx), k, _lib.ptr(ga), _lib.ptr(gb),
+        ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device)), "grpo_nf4_lora_train_backward")
+    return gx, ga, gb
 
 
 def nf4_grad_x_supported(n: int, k: int, blocksize: int) -> bool:

@@ -97,32 +97,37 @@ int grpo_nf4_grad_x(const void* grad, int64_t ldg, const uint8_t* w, const float
 int grpo_nf4_dequant_t(const uint8_t* w, const float* absmax, const float* code16, void* out,
                        int N, int K, int blocksize, int f16, grpo_stream_t stream);
 
-/* Workspace bytes of grpo_lora_forward_add and grpo_lora_backward (0: shape not
- * supported: N % 8, K % 8 != 0 or r outside [1, 32]). */
-size_t grpo_lora_train_workspace_bytes(int M, int N, int K, int r);
+/* Workspace bytes of grpo_nf4_lora_train_forward / _backward (either; 0: shape
+ * not supported: N % 32, K % 32 != 0, r outside [1, 32] or a blocksize that is
+ * not a power of two >= 32).  Holds the weight in 16 bits. */
+size_t grpo_nf4_lora_train_workspace_bytes(int M, int N, int K, int r, int blocksize);
 
-/* The LoRA term of the forward added to a finished base product, in place:
- *   y = dt(dt(y [+ bias]) + dt(dt(t B^T) * dt(scaling))), t = dt(x A^T)
- * with y [M, N] (row stride ldy) holding dt(x W^T), x [M, K], lora_a [r, K],
- * lora_b [N, r], bias [N] or NULL (_lora_forward_kernel, src/triton_kernels/
- * lora_forward.py:210-257).  Rows of x and y, lora_a and the workspace are
- * 16-byte aligned. */
-int grpo_lora_forward_add(const void* x, int64_t ldx, const void* lora_a, const void* lora_b,
-                          const void* bias, int r, float scaling, void* y, int64_t ldy, int M,
-                          int N, int K, int f16, void* workspace, size_t workspace_bytes,
-                          grpo_stream_t stream);
+/* The fused linear for training batches, _lora_forward_kernel (src/
+ * triton_kernels/lora_forward.py:107-260) as two launches: W in dt and t = dt(x
+ * A^T), then
+ *   y = dt(dt(dt(x W^T) [+ bias]) + dt(dt(t B^T) * dt(scaling)))
+ * with float32 sums; x [M, K] (row stride ldx), w/absmax/code16/blocksize as in
+ * grpo_nf4_dequant, bias [N] or NULL, lora_a [r, K], lora_b [N, r], y [M, N].
+ * Rows of x and y, w, lora_a and the workspace are 16-byte aligned. */
+int grpo_nf4_lora_train_forward(const void* x, int64_t ldx, const uint8_t* w, const float* absmax,
+                                const float* code16, int blocksize, const void* bias,
+                                const void* lora_a, const void* lora_b, int r, float scaling,
+                                void* y, int64_t ldy, int M, int N, int K, int f16,
+                                void* workspace, size_t workspace_bytes, grpo_stream_t stream);
 
-/* The LoRA side of FusedLoRAFunction.backward (lora_forward.py:836-928), each
- * result optional (NULL):
+/* FusedLoRAFunction.backward (lora_forward.py:761-930) without the bias
+ * gradient, each result optional (NULL):
  *   sg = dt(grad * dt(scaling)), gi = dt(sg B), xa = dt(x A^T)
+ *   grad_x [M, K] = dt(dt(grad W) + dt(gi A))
  *   grad_a [r, K] = dt(gi^T x), grad_b [N, r] = dt(sg^T xa)
- *   grad_x [M, K] = dt(grad_x + dt(gi A)), in place: grad_x holds dt(grad W)
- * with float32 sums.  Rows of x, grad and grad_x, lora_a, the results and the
- * workspace are 16-byte aligned. */
-int grpo_lora_backward(const void* x, int64_t ldx, const void* grad, int64_t ldg,
-                       const void* lora_a, const void* lora_b, int r, float scaling, int M, int N,
-                       int K, int f16, void* grad_x, int64_t ldgx, void* grad_a, void* grad_b,
-                       void* workspace, size_t workspace_bytes, grpo_stream_t stream);
+ * with float32 sums.  Rows of x, grad and grad_x, w, lora_a, grad_a, grad_b and
+ * the workspace are 16-byte aligned. */
+int grpo_nf4_lora_train_backward(const void* x, int64_t ldx, const void* grad, int64_t ldg,
+                                 const uint8_t* w, const float* absmax, const float* code16,
+                                 int blocksize, const void* lora_a, const void* lora_b, int r,
+                                 float scaling, int M, int N, int K, int f16, void* grad_x,
+                                 int64_t ldgx, void* grad_a, void* grad_b, void* workspace,
+                                 size_t workspace_bytes, grpo_stream_t stream);
 
 /* ------------------------------------------------ split-K NF4 linear --
  * The fast NF4 (+ LoRA) linear runs as a split-K kernel: workgroups own a

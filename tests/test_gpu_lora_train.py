@@ -1,6 +1,6 @@
-"""The LoRA side of the training step on the GPU (csrc/lora_train.hip) against
+"""The training form of the NF4 + LoRA linear on the GPU against
 float64 torch on the same rounding points: grpo_nf4_dequant_t bit for bit with
-grpo_nf4_dequant, grpo_lora_backward and grpo_lora_forward_add.
+grpo_nf4_dequant, grpo_nf4_lora_train_forward and _backward (csrc/lora_train.hip, csrc/gemm16.hip).
 
 Tolerances: every result is a float32 sum of exact products, rounded once to the
 16-bit type.  Against the float64 sum it differs by that rounding (half an ulp:
@@ -23,53 +23,49 @@ def _close(got, want, dt, what):
 
 
 def _inputs(dev, m, n, k, r, dt, seed):
+    from grpo_mi355x.core.nf4 import quantize_nf4
+
     g = torch.Generator().manual_seed(seed)
     rnd = lambda *s, sd=1.0: (torch.randn(*s, generator=g) * sd).to(dt).to(dev)
-    return (rnd(m, k), rnd(m, n, sd=0.1), rnd(r, k, sd=0.05), rnd(n, r, sd=0.05),
-            rnd(m, k), rnd(m, n), rnd(n))
+    packed, st = quantize_nf4((torch.randn(n, k, generator=g) * 0.02).to(dev),
+                              64 if k % 64 == 0 else 32)
+    return (rnd(m, k), rnd(m, n, sd=0.1), (packed.view(-1), st.absmax, st.code, st.blocksize),
+            rnd(r, k, sd=0.05), rnd(n, r, sd=0.05), rnd(n))
 
 
-@pytest.mark.parametrize("n,k", [(8, 32), (64, 128), (72, 160), (1536, 256), (200, 1536)])
+# M: one row to past each tile (64, 128, 256) and each row slicing of the adapters'
+# gradients; N, K: column tiles with remainders, 1 to 48 stages of 32 of either
+# product; ranks below, at and past a tile of 16
+@pytest.mark.parametrize("m,n,k,r", [(1, 32, 32, 1), (16, 128, 64, 16), (33, 160, 544, 8),
+                                     (127, 256, 1536, 17), (300, 1536, 96, 32),
+                                     (1050, 288, 1024, 16), (1300, 4096, 512, 5),
+                                     (8200, 1536, 512, 16), (5000, 4128, 256, 16)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-def test_dequant_t_is_the_transposed_dequant(dev, n, k, dt):
-    from grpo_mi355x.core.nf4 import quantize_nf4
+def test_training_linear(dev, m, n, k, r, dt):
     from grpo_mi355x.kernels import ops
 
-    torch.manual_seed(n + k)
-    packed, st = quantize_nf4(torch.randn(n, k, device=dev) * 0.02, 32 if k % 64 else 64)
-    args = (packed.view(-1), st.absmax, st.code)
-    want = ops.nf4_dequant(*args, n * k, st.blocksize, dtype=dt).view(n, k)
-    got = ops.nf4_dequant_t(*args, n, k, st.blocksize, dtype=dt)
-    assert torch.equal(got.view(torch.int16), want.t().contiguous().view(torch.int16))
-
-
-@pytest.mark.parametrize("m,n,k,r", [(1, 8, 8, 1), (16, 128, 64, 16), (33, 136, 520, 8),
-                                     (127, 256, 1536, 17), (300, 1536, 72, 32),
-                                     (1050, 264, 1000, 16), (8200, 1536, 512, 16)])
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-def test_lora_backward_and_forward_add(dev, m, n, k, r, dt):
-    from grpo_mi355x.kernels import ops
-
-    x, g, a, b, gx, y, bias = _inputs(dev, m, n, k, r, dt, m + n + k + r)
+    x, g, wq, a, b, bias = _inputs(dev, m, n, k, r, dt, m + n + k + r)
+    print(f"nf4_lora_train M={m} N={n} K={k} r={r} {dt}", flush=True)
+    w = ops.nf4_dequant(*wq[:3], n * k, wq[3], dtype=dt).view(n, k).double()
     s = 1.7  # not a power of two: the rounded scaling matters
     sd = float(torch.tensor(s, dtype=dt))
     rt = lambda t: t.to(dt).double()
     sg = rt(g.double() * sd)
     gi, xa = rt(sg @ b.double()), rt(x.double() @ a.double().t())
-    ga, gb = ops.lora_backward(x, g, a, b, s, grad_x=(got := gx.clone()))
+    gx, ga, gb = ops.nf4_lora_train_backward(x, g, *wq, a, b, s)
     _close(ga, gi.t() @ x.double(), dt, "grad_A")
     _close(gb, sg.t() @ xa, dt, "grad_B")
-    _close(got, gx.double() + rt(gi @ a.double()), dt, "grad_x")
+    _close(gx, rt(g.double() @ w) + rt(gi @ a.double()), dt, "grad_x")
     # each result alone is the same
-    assert torch.equal(ops.lora_backward(x, g, a, b, s, want_b=False)[0], ga)
-    assert torch.equal(ops.lora_backward(x, g, a, b, s, want_a=False)[1], gb)
-    alone = gx.clone()
-    ops.lora_backward(x, g, a, b, s, grad_x=alone, want_a=False, want_b=False)
-    assert torch.equal(alone, got)
+    for i in range(3):
+        only = ops.nf4_lora_train_backward(x, g, *wq, a, b, s, *(j == i for j in range(3)))
+        assert [o is not None for o in only] == [j == i for j in range(3)]
+        assert torch.equal(only[i], (gx, ga, gb)[i])
     u = rt(rt(xa @ b.double().t()) * sd)
+    acc = rt(x.double() @ w.t())
     for bi in (None, bias):
-        base = y.double() if bi is None else rt(y.double() + bi.double())
-        _close(ops.lora_forward_add(y.clone(), x, a, b, s, bi), base + u, dt, "y")
+        base = acc if bi is None else rt(acc + bi.double())
+        _close(ops.nf4_lora_train_forward(x, *wq, a, b, s, bi), base + u, dt, "y")
 
 
 def test_rows_past_the_end_add_nothing(dev):
@@ -77,8 +73,36 @@ def test_rows_past_the_end_add_nothing(dev):
     the last row reaches its own results only."""
     from grpo_mi355x.kernels import ops
 
-    x, g, a, b, _, _, _ = _inputs(dev, 37, 128, 128, 16, torch.bfloat16, 3)
+    x, g, wq, a, b, _ = _inputs(dev, 37, 128, 128, 16, torch.bfloat16, 3)
     g[-1, 5] = float("inf")
-    ga, gb = ops.lora_backward(x, g, a, b, 1.0)
+    gx, ga, gb = ops.nf4_lora_train_backward(x, g, *wq, a, b, 1.0)
     assert torch.isfinite(gb[torch.arange(128) != 5]).all()
     assert not torch.isfinite(gb[5]).any()
+    assert torch.isfinite(gx[:-1]).all()
+
+
+@pytest.mark.parametrize("how", ["misaligned", "create_graph", "batched"])
+def test_backward_of_what_the_kernels_do_not_take(dev, how):
+    """grad_out rows off their alignment, a differentiable and a batched backward
+    give the gradients of the kernels' path (one rounding of each product)."""
+    from grpo_mi355x.core.nf4 import Linear4bitNF4
+    from grpo_mi355x.kernels import lora_fused_forward
+
+    m, n, k, r = 1100, 256, 128, 16
+    gen = torch.Generator().manual_seed(1)
+    rnd = lambda *s, sd: (torch.randn(*s, generator=gen) * sd).bfloat16().to(dev)
+    base = Linear4bitNF4.from_weight(rnd(n, k, sd=0.02).float())
+    x, g = rnd(1, m, k, sd=1.0).requires_grad_(), rnd(1, m, n, sd=0.1)
+    a, b = rnd(r, k, sd=0.05).requires_grad_(), rnd(n, r, sd=0.05).requires_grad_()
+    y = lora_fused_forward(x, base_layer=base, lora_A=a, lora_B=b, scaling=2.0)
+    grads = lambda go, **kw: torch.autograd.grad(y, (x, a, b), go, retain_graph=True, **kw)
+    want = grads(g)
+    if how == "misaligned":
+        got = grads(torch.cat([g.new_zeros(4), g.reshape(-1)])[4:].view(1, m, n))
+    elif how == "create_graph":
+        got = grads(g, create_graph=True)
+        assert all(t.requires_grad for t in got)
+    else:
+        got = [t[1] for t in grads(torch.stack([g * 0, g]), is_grads_batched=True)]
+    for u, v in zip(got, want):
+        _close(u.detach(), v.double(), torch.bfloat16, how)
