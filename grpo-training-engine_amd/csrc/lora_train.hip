@@ -75,11 +75,8 @@ __device__ __forceinline__ void dequant_rows(const DequantJob& j, int b) {
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint4 v = decode8(wv[i], make_lut<F16>(code, a[i]));  // [0,2,4,6,1,3,5,7]
-    if (e[i] < total)
-      *reinterpret_cast<uint4*>(j.out + e[i]) =
-          make_uint4(perm(v.z, v.x, 0x05040100u), perm(v.z, v.x, 0x07060302u),
-                     perm(v.w, v.y, 0x05040100u), perm(v.w, v.y, 0x07060302u));
+    const uint4 v = interleave8(decode8(wv[i], make_lut<F16>(code, a[i])));
+    if (e[i] < total) *reinterpret_cast<uint4*>(j.out + e[i]) = v;
   }
 }
 

@@ -65,6 +65,12 @@ __device__ __forceinline__ uint4 decode8(uint32_t wd, const Lut& t) {
                     perm(Hl, Ll, 0x05010400u), perm(Hl, Ll, 0x07030602u));
 }
 
+// The decode8 order [0,2,4,6,1,3,5,7] -> natural order.
+__device__ __forceinline__ uint4 interleave8(uint4 v) {
+  return make_uint4(perm(v.z, v.x, 0x05040100u), perm(v.z, v.x, 0x07060302u),
+                    perm(v.w, v.y, 0x05040100u), perm(v.w, v.y, 0x07060302u));
+}
+
 // Eight bf16 in natural order (4 dwords) -> the decode8 order [0,2,4,6,1,3,5,7].
 __device__ __forceinline__ uint4 deinterleave8(uint4 v) {
   return make_uint4(perm(v.y, v.x, 0x05040100u), perm(v.w, v.z, 0x05040100u),

@@ -198,9 +198,26 @@ class Linear4bitNF4(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # computes in x's dtype when that is float16 (bitsandbytes' Linear4bit
         # returns the input's dtype), in bf16 otherwise
-        w = self.dequantize(torch.float16 if x.dtype == torch.float16 else torch.bfloat16)
+        dt = torch.float16 if x.dtype == torch.float16 else torch.bfloat16
+        w = self._dequantized_for(x, dt)
         bias = None if self.bias is None else self.bias.to(w.dtype)
         return F.linear(x.to(w.dtype), w, bias)
+
+    def _dequantized_for(self, x: torch.Tensor, dt: torch.dtype) -> torch.Tensor:
+        """``dequantize(dt)``, stored [in, out] where x's gradient will be asked for
+        and out >= 2 in: grad_x = g W is then a product along contiguous rows.
+        Library GEMMs, forward + backward, out 8960, in 1536 (us): 71 -> 57 at 512
+        rows, 103 -> 73 at 1024; 9216 x 2048 108 -> 89 at 1024, 190 -> 196 at 2800; the
+        other way round for a wide in (1536 x 8960: 75 -> 109 at 1024)."""
+        from ..kernels import ops
+
+        n, k, qs = self.out_features, self.in_features, self.weight.quant_state
+        if (torch.is_grad_enabled() and x.requires_grad and n >= 2 * k and 1024 <= k <= 2048
+                and x.numel() <= 2048 * k
+                and ops.nf4_dequant_t_supported(self.weight.data, n, k, qs.blocksize)):
+            return ops.nf4_dequant_t(self.weight.data.view(-1), float_absmax(qs), qs.code, n, k,
+                                     qs.blocksize, dtype=dt).t()
+        return self.dequantize(dt)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, "

@@ -106,3 +106,42 @@ def test_backward_of_what_the_kernels_do_not_take(dev, how):
         got = [t[1] for t in grads(torch.stack([g * 0, g]), is_grads_batched=True)]
     for u, v in zip(got, want):
         _close(u.detach(), v.double(), torch.bfloat16, how)
+
+
+@pytest.mark.parametrize("m", [1, 33, 2048, 2049])
+def test_linear4bit_weight_layout_with_and_without_gradient(dev, m):
+    """Linear4bitNF4 keeps the weight transposed where x's gradient is asked for (up to
+    2048 rows): the same output and gradient as over the row-major weight, up to the
+    order of the float32 sums."""
+    from grpo_mi355x.core.nf4 import Linear4bitNF4
+
+    torch.manual_seed(m)
+    lin = Linear4bitNF4.from_weight(torch.randn(2048, 1024, device=dev) * 0.02)
+    x = torch.randn(1, m, 1024, device=dev).bfloat16().requires_grad_()
+    g = torch.randn(1, m, 2048, device=dev).bfloat16()
+    w = lin.dequantize()
+    used = lin._dequantized_for(x, torch.bfloat16)
+    assert torch.equal(used, w) and used.is_contiguous() == (m > 2048)
+    assert lin._dequantized_for(x.detach(), torch.bfloat16).is_contiguous()
+    y = lin(x)
+    y.backward(g)
+    _close(y.detach(), torch.nn.functional.linear(x.detach().double(), w.double()),
+           torch.bfloat16, "y")
+    _close(x.grad, g.double() @ w.double(), torch.bfloat16, "grad_x")
+
+
+@pytest.mark.parametrize("n,k,bs", [(1, 8, 8), (3, 24, 24), (65, 128, 64), (129, 1536, 4096)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_dequant_runs_of_eight(dev, n, k, bs, dt):
+    """nf4_dequant's vector path over odd run counts and blocksizes, bit for bit with
+    the codebook product rounded by torch."""
+    from grpo_mi355x.core.nf4 import nf4_code
+    from grpo_mi355x.kernels import ops
+
+    torch.manual_seed(n)
+    packed = torch.randint(0, 256, (n * k // 2,), dtype=torch.uint8, device=dev)
+    absmax = torch.rand(-(-n * k // bs), device=dev)
+    q = torch.stack([packed >> 4, packed & 15], 1).view(-1).long()
+    want = (nf4_code(dev)[q] * absmax.repeat_interleave(bs)[:n * k]).to(dt)
+    got = ops.nf4_dequant(packed, absmax, nf4_code(dev), n * k, bs, dtype=dt)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
