@@ -118,6 +118,13 @@ SIGNATURES = {
         [_VP, _I64, _VP, _VP, _VP, _I32, _I32, _VP, _VP, _VP, _VP, _I32, _F32, _VP, _I64, _I32,
          _I32, _VP, _SZ, _VP],
     ),
+    "grpo_decode_start": (
+        _I32,
+        [_VP, _VP, _VP, _VP, _I64, _I32, _I64, _I64, _I32, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP,
+         _VP, _VP, _I32, _VP, _I64, _VP],
+    ),
+    "grpo_prefill_rows": (
+        _I32, [_VP, _I32, _I32, _VP, _I32, _I32, _VP, _VP, _VP, _VP, _I32, _VP]),
     "grpo_embedding": (_I32, [_VP, _VP, _I64, _I32, _VP, _I32, _VP]),
     "grpo_add_rmsnorm": (_I32, [_VP, _VP, _VP, _VP, _VP, _I32, _I32, _F32, _VP]),
     "grpo_rope_append": (

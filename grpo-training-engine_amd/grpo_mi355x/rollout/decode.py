@@ -800,28 +800,29 @@ class DecodeEngine:
               limits: torch.Tensor, max_new_tokens: int, eos_token_id: Optional[int] = None,
               pad_token_id: int = 0, record: bool = True):
         """Load a new batch: input tokens at ``positions`` (tokens already cached)."""
-        B = self.B
-        self.tokens.copy_(tokens.view(B))
-        self.pos.copy_(positions.view(B).to(torch.int32))
-        self.count.zero_()
-        self.limit.copy_(limits.view(B).to(torch.int32))
-        self.active.copy_(self.limit > 0)
-        self.eos.fill_(-1 if eos_token_id is None else int(eos_token_id))
-        self.pad.fill_(int(pad_token_id))
-        w = block_tables.shape[1]
-        self.block_tables.fill_(-1)
-        self.block_tables[:, :w].copy_(block_tables)
-        if record:
-            if self.generated is None or self.generated.shape[1] != max_new_tokens:
-                self.generated = torch.full((B, max_new_tokens), pad_token_id, dtype=torch.int64,
-                                            device=self.device)
-                self.graph = None  # the recorded step writes into this buffer
-                self.graph_multi = {}
-            self.generated.fill_(pad_token_id)
-        self._masks()
-        # bound on every row's position for run()'s choice of split plan (one
-        # host sync per batch)
-        self._pos_hi = int(positions.max()) if positions.numel() else 0
+        B, dev = self.B, self.device
+        i64 = lambda t: t.view(B).to(device=dev, dtype=torch.int64).contiguous()
+        tok, pos, lim = i64(tokens), i64(positions), i64(limits)
+        bt = block_tables.to(device=dev, dtype=torch.int32)
+        if bt.stride(-1) != 1:
+            bt = bt.contiguous()
+        w = bt.shape[1]
+        bt = bt.expand(B, w)
+        if record and (self.generated is None or self.generated.shape[1] != max_new_tokens):
+            self.generated = torch.empty((B, max_new_tokens), dtype=torch.int64, device=dev)
+            self.graph = None  # the recorded step writes into this buffer
+            self.graph_multi = {}
+        gen = self.generated if record else None
+        _lib.check(self.lib.grpo_decode_start(
+            tok.data_ptr(), pos.data_ptr(), lim.data_ptr(), bt.data_ptr(), bt.stride(0), w,
+            -1 if eos_token_id is None else int(eos_token_id), int(pad_token_id), B,
+            self.tokens.data_ptr(), self.pos.data_ptr(), self.count.data_ptr(),
+            self.limit.data_ptr(), self.active.data_ptr(), self.eos.data_ptr(),
+            self.pad.data_ptr(), self.append_pos.data_ptr(), self.attn_len.data_ptr(),
+            self.block_tables.data_ptr(), self.max_blocks, _lib.ptr(gen),
+            0 if gen is None else gen.shape[1], _lib.stream_handle(dev)), "decode_start")
+        self._pos_hi = None
+        self._pos_stale = True  # read from the device when run() first plans splits
 
     def capture(self):
         """Record one step into a HIP graph (after two warm-up steps on a side stream)."""
@@ -898,7 +899,10 @@ class DecodeEngine:
     # (config 4's 32-row engine: 8867 tok/s planned live against 8927).
     LIVE_WIDTH = True
     _pw: Optional[int] = None  # plan width of the launches being built (None: the table's)
+    # bound on every row's position (None: unknown); stale: after start(), until
+    # run() needs it (a host sync)
     _pos_hi: Optional[int] = None
+    _pos_stale = False
 
     def _live_width(self, ctx: int) -> int:
         """Plan width (blocks) covering contexts of up to ``ctx`` tokens."""
@@ -935,6 +939,8 @@ class DecodeEngine:
         Each replay's attention splits are planned for the contexts its steps
         can reach (every row's position advances by at most one per step)."""
         if self.graph is not None and steps >= self.MULTI_STEP:
+            if getattr(self, "_pos_stale", False):
+                self._pos_hi, self._pos_stale = int(self.pos.max()), False
             while steps >= self.MULTI_STEP:
                 pw = (self._live_width(self._pos_hi + self.MULTI_STEP)
                       if self._pos_hi is not None else None)
@@ -986,7 +992,7 @@ class DecodeEngine:
         self.generated.copy_(src.pad.view(1, 1).expand_as(self.generated))
         self.generated[:n].copy_(src.generated.index_select(0, idx))
         self._masks()
-        self._pos_hi = src._pos_hi
+        self._pos_hi, self._pos_stale = src._pos_hi, src._pos_stale
 
     def run_paged(self, sids: list, max_steps: int, chunk: Optional[int] = None,
                   check_invariants: bool = False, compact: Optional[list] = None) -> dict:
@@ -1071,7 +1077,7 @@ class DecodeEngine:
             if check_invariants:
                 pool.check_invariants()
             peak = max(peak, pool.num_blocks - pool.num_free)
-            eng._pos_hi = max(pos)
+            eng._pos_hi, eng._pos_stale = max(pos), False
             eng.run(n)
             steps += n
         for b in list(live):  # rows cut off by max_steps
@@ -1087,6 +1093,22 @@ class DecodeEngine:
         """Copy rows 0 .. len(origin) - 1 of ``eng.generated`` to this engine's rows ``origin``."""
         idx = torch.tensor(origin, dtype=torch.long, device=self.device)
         self.generated.index_copy_(0, idx, eng.generated[:len(origin)])
+
+
+def _run_chunks(eng, table: torch.Tensor, prompt: torch.Tensor, n: int) -> None:
+    """Passes of a prefill engine over ``prompt[:n]``, eng.B positions each."""
+    dev = eng.device
+    tbl = table.view(-1).to(device=dev, dtype=torch.int32).contiguous()
+    ids = prompt[:n].to(device=dev, dtype=torch.int64).contiguous()
+    if table.shape[0] != 1 or ids.shape != (n,):
+        raise RuntimeError(f"one block table row and {n} prompt tokens required, got "
+                           f"{tuple(table.shape)} and {tuple(prompt.shape)}")
+    for p in range(0, n, eng.B):
+        _lib.check(eng.lib.grpo_prefill_rows(
+            ids.data_ptr(), p, min(eng.B, n - p), tbl.data_ptr() if p == 0 else None, tbl.numel(),
+            eng.B, eng.tokens.data_ptr(), eng.append_pos.data_ptr(), eng.attn_len.data_ptr(),
+            eng.block_tables.data_ptr(), eng.max_blocks, _lib.stream_handle(dev)), "prefill_rows")
+        eng.step()
 
 
 class PrefillEngine(DecodeEngine):
@@ -1114,7 +1136,6 @@ class PrefillEngine(DecodeEngine):
         bf = dict(dtype=torch.bfloat16, device=self.device)
         self.q_rot = torch.zeros(chunk, self.Hq, self.D, **bf)
         self.attn_out = torch.zeros(chunk, self.Hq * self.D, **bf)
-        self._rows = torch.arange(chunk, dtype=torch.int32, device=self.device)
 
     def _attn_launches(self, L: dict, kc: int, vc: int, st) -> list:
         return self._attn_launches_unfused(L, kc, vc, st)
@@ -1131,18 +1152,7 @@ class PrefillEngine(DecodeEngine):
         if self.graph is None:
             self.active.zero_()  # the warm-up passes append nothing
             self.capture()
-        w = table.shape[1]
-        self.block_tables.fill_(-1)
-        self.block_tables[:, :w].copy_(table.view(1, w).expand(self.B, w))
-        none = torch.full_like(self._rows, -1)
-        for p in range(0, n, self.B):
-            c = min(self.B, n - p)
-            valid = self._rows < c
-            self.tokens.zero_()
-            self.tokens[:c].copy_(prompt[p:p + c])
-            self.append_pos.copy_(torch.where(valid, self._rows + p, none))
-            self.attn_len.copy_(torch.where(valid, self._rows + (p + 1), none + 1))
-            self.step()
+        _run_chunks(self, table, prompt, n)
 
 
 class GemmPrefillEngine:
@@ -1197,7 +1207,6 @@ class GemmPrefillEngine:
         self.attn_out = torch.zeros(B, self.Hq * D, **bf)
         self.gu = torch.zeros(B, 2 * self.I, **bf)
         self.act = torch.zeros(B, self.I, **bf)
-        self._rows = torch.arange(B, dtype=torch.int32, device=dev)
         self._keep = []
         self.layers = []
         ws = 0
@@ -1332,18 +1341,7 @@ class GemmPrefillEngine:
         whose block table row is ``table`` ([1, w] int32, its blocks reserved)."""
         if self.graph is None:
             self.capture()
-        w = table.shape[1]
-        self.block_tables.fill_(-1)
-        self.block_tables[:, :w].copy_(table.view(1, w).expand(self.B, w))
-        none = torch.full_like(self._rows, -1)
-        for p in range(0, n, self.B):
-            c = min(self.B, n - p)
-            valid = self._rows < c
-            self.tokens.zero_()
-            self.tokens[:c].copy_(prompt[p:p + c])
-            self.append_pos.copy_(torch.where(valid, self._rows + p, none))
-            self.attn_len.copy_(torch.where(valid, self._rows + (p + 1), none + 1))
-            self.step()
+        _run_chunks(self, table, prompt, n)
 
 
 def release_decode_caches(model=None) -> None:

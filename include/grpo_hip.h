@@ -850,6 +850,26 @@ int grpo_sample_advance(const void* logits, int64_t ld_logits, int M, int V, flo
                         int32_t* append_pos, int32_t* attn_len, void* workspace,
                         size_t workspace_bytes, grpo_stream_t stream);
 
+/* Load a batch into an engine's row state (DecodeEngine.start), B rows: tokens,
+ * positions (tokens already cached) and limits as int64 [B]; tables int32 [B,
+ * width] (row stride ld_tables, 0 for one row shared by all; width <=
+ * max_blocks, the rest of a row becomes -1). A row with limit <= 0 starts
+ * stopped. generated [B, gen_ld] (may be NULL) is filled with pad_id. */
+int grpo_decode_start(const int64_t* tokens_in, const int64_t* positions, const int64_t* limits,
+                      const int32_t* tables, int64_t ld_tables, int width, int64_t eos_id,
+                      int64_t pad_id, int B, int64_t* tokens, int32_t* pos, int32_t* count,
+                      int32_t* limit, uint8_t* active, int64_t* eos, int64_t* pad,
+                      int32_t* append_pos, int32_t* attn_len, int32_t* block_tables,
+                      int max_blocks, int64_t* generated, int64_t gen_ld, grpo_stream_t stream);
+
+/* Load a chunk of one prompt into a prefill engine's B rows: row i < count takes
+ * prompt[first + i] at position first + i, the others idle (slot -1, length 0);
+ * table int32 [width] (NULL: block_tables keeps its contents) becomes every
+ * row's block table, entries past width -1. */
+int grpo_prefill_rows(const int64_t* prompt, int first, int count, const int32_t* table, int width,
+                      int B, int64_t* tokens, int32_t* append_pos, int32_t* attn_len,
+                      int32_t* block_tables, int max_blocks, grpo_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
