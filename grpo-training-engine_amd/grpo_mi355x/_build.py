@@ -22,7 +22,7 @@ LIB_PATH = NATIVE_DIR / "libgrpo_hip.so"
 ARCH = "gfx950"
 
 SOURCES = ("capi.hip", "nf4_linear.hip", "nf4_fold.hip", "nf4_tile.hip", "nf4_gemm.hip",
-           "paged_attention.hip", "decode_ops.hip", "lm_head.hip", "sampling.hip",
+           "paged_attention.hip", "prefill_attention.hip", "decode_ops.hip", "lm_head.hip", "sampling.hip",
            "nf4_backward.hip", "gemm16.hip", "lora_train.hip")
 
 # Flags of one source only (machine-scheduler strategies measured per source

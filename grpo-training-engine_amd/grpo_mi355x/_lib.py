@@ -118,6 +118,12 @@ SIGNATURES = {
         [_VP, _I64, _VP, _VP, _VP, _I32, _I32, _VP, _VP, _VP, _VP, _I32, _F32, _VP, _I64, _I32,
          _I32, _VP, _SZ, _VP],
     ),
+    "grpo_paged_attn_prefill_supported": (_I32, [_I32, _I32, _I32, _I32]),
+    "grpo_paged_attn_prefill": (
+        _I32,
+        [_VP, _I64, _I64, _VP, _VP, _I64, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _F32,
+         _VP],
+    ),
     "grpo_decode_start": (
         _I32,
         [_VP, _VP, _VP, _VP, _I64, _I32, _I64, _I64, _I32, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP,

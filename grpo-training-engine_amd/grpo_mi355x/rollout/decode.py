@@ -1239,8 +1239,11 @@ class GemmPrefillEngine:
                     B, n, k, rr, nseg, self.bs)))
         # one workspace for every linear (they run one after another on one stream)
         self.ws = torch.empty(max(ws, 16), dtype=torch.uint8, device=dev)
-        self.ws_attn = ops.workspace("paged_attn_prefill", max(ops.paged_attention_workspace_bytes(
-            B, self.Hq, self.Hkv, D, pool.block_size, max_blocks), 1), dev)
+        self.attn_prefill = bool(self.lib.grpo_paged_attn_prefill_supported(
+            self.Hq, self.Hkv, D, pool.block_size))
+        self.ws_attn = ops.workspace("paged_attn_prefill", 1 if self.attn_prefill else max(
+            ops.paged_attention_workspace_bytes(B, self.Hq, self.Hkv, D, pool.block_size,
+                                                max_blocks), 1), dev)
         self.embed = model.model.embed_tokens.weight
         self.gu_fused = bool(self.lib.grpo_nf4_gate_up_silu_supported(B, self.I, H, self.bs))
         self.graph: Optional[torch.cuda.CUDAGraph] = None
@@ -1286,10 +1289,15 @@ class GemmPrefillEngine:
                 pool.block_size, self.max_blocks, B, st), "append")))
             if li == last:
                 break  # the last layer's attention and MLP feed nothing kept
-            out.append(("attention", lambda kc=kc, vc=vc: chk(lib.grpo_paged_attn_decode(
-                q, Hq * D, D, kc, vc, pool.num_blocks, bt, self.max_blocks, al, ao, 1, B, Hq,
-                Hkv, D, pool.block_size, self.max_blocks, 1.0 / math.sqrt(D), wsa, wsa_n, st),
-                "attention")))
+            if self.attn_prefill:  # the rows share one block table: row 0's
+                out.append(("attention", lambda kc=kc, vc=vc: chk(lib.grpo_paged_attn_prefill(
+                    q, Hq * D, D, kc, vc, pool.num_blocks, bt, al, ao, B, Hq, Hkv, D,
+                    pool.block_size, self.max_blocks, 1.0 / math.sqrt(D), st), "attention")))
+            else:
+                out.append(("attention", lambda kc=kc, vc=vc: chk(lib.grpo_paged_attn_decode(
+                    q, Hq * D, D, kc, vc, pool.num_blocks, bt, self.max_blocks, al, ao, 1, B, Hq,
+                    Hkv, D, pool.block_size, self.max_blocks, 1.0 / math.sqrt(D), wsa, wsa_n, st),
+                    "attention")))
             out.append(("o", lambda L=L: linear(
                 ao, Hq * D, L["o_w"], L["o_absmax"], L["o_code"], L["o_bias"], L["o_la"],
                 L["o_lb"], L["o_r"], L["o_scaling"], y, H, Hq * D)))

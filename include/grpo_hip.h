@@ -850,6 +850,19 @@ int grpo_sample_advance(const void* logits, int64_t ld_logits, int M, int V, flo
                         int32_t* append_pos, int32_t* attn_len, void* workspace,
                         size_t workspace_bytes, grpo_stream_t stream);
 
+/* Attention of a prompt chunk: M rows of one sequence, row m over its first
+ * lens[m] tokens (int32 [M]; <= 0: the row's output is 0), block_table int32
+ * [max_blocks] of that sequence; q bf16 [M, Hq, 128] (row and head strides), out
+ * bf16 [M, Hq, 128]. The scores, softmax and rounding of grpo_paged_attn_decode.
+ * Needs head_dim 128, block size 16 and 16-byte aligned rows and caches
+ * (grpo_paged_attn_prefill_supported; alignment aside). No workspace. */
+int grpo_paged_attn_prefill_supported(int Hq, int Hkv, int D, int block_size);
+int grpo_paged_attn_prefill(const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                            const void* k_cache, const void* v_cache, int64_t num_blocks,
+                            const int32_t* block_table, const int32_t* lens, void* out, int M,
+                            int Hq, int Hkv, int D, int block_size, int max_blocks, float scale,
+                            grpo_stream_t stream);
+
 /* Load a batch into an engine's row state (DecodeEngine.start), B rows: tokens,
  * positions (tokens already cached) and limits as int64 [B]; tables int32 [B,
  * width] (row stride ld_tables, 0 for one row shared by all; width <=

@@ -1,0 +1,79 @@
+"""grpo_paged_attn_prefill against the decode attention of the same rows, which is
+pinned against the oracle (tests/test_gpu_attention.py), and against float64.
+
+Both kernels hold float32 scores, sums and P (as two bf16 terms) and round once to
+bf16; they differ in the order of the sums, so a result can fall to the other
+neighbouring bf16 value: within one ulp (2^-7 of the larger), most of them equal."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dev, M, Hq, Hkv, lens, max_blocks, seed, holes=()):
+    from grpo_mi355x import _lib
+    from grpo_mi355x.kernels import ops
+
+    lib = _lib.device_library()
+    g = torch.Generator().manual_seed(seed)
+    nb = max_blocks + 3
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
+    q, k, v = rnd(M, Hq, 128), rnd(nb, Hkv, 16, 128), rnd(nb, Hkv, 16, 128)
+    table = torch.randperm(nb, generator=g)[:max_blocks].int()
+    if holes:  # ids out of range, and a block 0 that must not leak through them
+        table[table == 0] = nb - 1
+        for i, b in enumerate(holes):
+            table[b] = (-1, nb)[i % 2]
+        k[0], v[0] = float("nan"), float("nan")
+    table = table.to(dev)
+    ln = torch.tensor(lens, dtype=torch.int32, device=dev)
+    out = torch.full((M, Hq, 128), 7.0, dtype=torch.bfloat16, device=dev)
+    print(f"prefill attention M={M} Hq={Hq} Hkv={Hkv} max_blocks={max_blocks}", flush=True)
+    _lib.check(lib.grpo_paged_attn_prefill(
+        q.data_ptr(), Hq * 128, 128, k.data_ptr(), v.data_ptr(), nb, table.data_ptr(),
+        ln.data_ptr(), out.data_ptr(), M, Hq, Hkv, 128, 16, max_blocks, 1 / math.sqrt(128),
+        _lib.stream_handle(dev)), "prefill")
+    want = ops.paged_attention_decode(q, k, v, table.expand(M, max_blocks).contiguous(), ln,
+                                      1 / math.sqrt(128), out_dtype=torch.float32)
+    ops.attention_handover_check(dev)
+    return out.float(), want, (q, k, v, table)
+
+
+# rows: within, at and past a 16-row tile; contexts: within a block, at and past the 32-
+# and 64-token halves and steps, the ring of three steps, the 64-block table windows, empty and clamped ones
+@pytest.mark.parametrize("M,Hq,Hkv,first,max_blocks", [
+    (1, 1, 1, 1, 1), (17, 12, 2, 1, 2), (16, 4, 4, 17, 3), (40, 7, 1, 60, 8), (64, 28, 4, 129, 12),
+    (33, 10, 2, 200, 16), (70, 8, 1, 1, 6), (512, 12, 2, 1, 32), (100, 16, 8, 4000, 260),
+    (16, 2, 1, 1009, 64), (16, 2, 1, 1020, 70), (16, 2, 1, 2040, 130)])
+def test_prefill_attention(dev, M, Hq, Hkv, first, max_blocks):
+    lens = [first + i for i in range(M)]
+    if M > 20:
+        lens[3], lens[5], lens[-1] = 0, -4, 16 * max_blocks + 50
+    got, want, _ = _run(dev, M, Hq, Hkv, lens, max_blocks, M + Hq)
+    assert float(((got - want).abs() / want.abs().clamp(min=1e-3)).max()) <= 2.0 ** -7
+    assert float((got == want.bfloat16().float()).float().mean()) >= 0.97
+    if M > 20:
+        assert not got[3].any() and not got[5].any()
+
+
+@pytest.mark.parametrize("first,max_blocks,holes", [
+    (20, 12, (1, 6)), (1000, 80, (0, 62, 63, 64, 65, 66)), (1, 3, (0, 1, 2))])
+def test_prefill_attention_skips_invalid_blocks(dev, first, max_blocks, holes):
+    got, want, _ = _run(dev, 50, 6, 1, [first + 3 * i for i in range(50)], max_blocks, 5, holes)
+    assert torch.isfinite(got).all()
+    assert float(((got - want).abs() / want.abs().clamp(min=1e-3)).max()) <= 2.0 ** -7
+
+
+def test_prefill_attention_against_float64(dev):
+    got, _, (q, k, v, table) = _run(dev, 96, 12, 2, [100 + i for i in range(96)], 13, 9)
+    kk, vv = (t[table.long()].transpose(1, 2).reshape(-1, 2, 128).double().repeat_interleave(6, 1)
+              for t in (k, v))
+    s = torch.einsum("mhd,thd->mht", q.double(), kk) / math.sqrt(128)
+    on = torch.arange(kk.shape[0], device=dev) < torch.arange(100, 196, device=dev)[:, None]
+    p = torch.softmax(s.masked_fill(~on[:, None], -math.inf), -1)
+    want = torch.einsum("mht,thd->mhd", p, vv)
+    # one rounding to bf16: half an ulp, 2^-9, with a little for the float32 sums
+    assert float(((got - want).abs() / want.abs().clamp(min=1e-2)).max()) <= 1.05 * 2.0 ** -8
