@@ -604,6 +604,29 @@ extern "C" int grpo_nf4_tile_linear(const void* x, int64_t ldx, const uint8_t* w
   return launch_tile<TX_BF16, TE_OUT>(a, pl, as_stream(stream));
 }
 
+extern "C" int grpo_nf4_tile_linear_one(const void* x, int64_t ldx, const uint8_t* w,
+                                        const float* absmax, const float* code16, int blocksize,
+                                        const void* bias, const void* lora_a_packed,
+                                        const void* lora_b, int r, float scaling, void* y,
+                                        int64_t ldy, int M, int N, int K, grpo_stream_t stream) {
+  if (!grpo_nf4_tile_supported(M, N, K, r, 1, blocksize)) {
+    set_error("shape not supported by the one-launch linear");
+    return GRPO_EUNSUPPORTED;
+  }
+  grpo_tile_linear_t lin{};
+  lin.M = M;
+  lin.N = N;
+  lin.K = K;
+  lin.nseg = 1;
+  lin.r = r;
+  lin.seg_end[0] = N;
+  lin.lora_a[0] = lora_a_packed;
+  lin.lora_b[0] = lora_b;
+  lin.bias[0] = bias;
+  lin.scaling = scaling;
+  return grpo_nf4_tile_linear(x, ldx, w, absmax, code16, blocksize, &lin, y, ldy, stream);
+}
+
 extern "C" int grpo_nf4_tile_linear_norm(const void* h, int64_t ldh, const float* sumsq,
                                          int groups, const void* norm_weight, float eps,
                                          const uint8_t* w, const float* absmax,

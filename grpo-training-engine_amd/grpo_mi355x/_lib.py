@@ -246,6 +246,11 @@ SIGNATURES = {
     "grpo_nf4_tile_packed_lora_a_bytes": (_SZ, [_I32]),
     "grpo_nf4_tile_pack_lora_a": (_I32, [_VP, _I32, _I32, _I64, _VP, _VP]),
     "grpo_nf4_tile_linear": (_I32, [_VP, _I64, _VP, _VP, _VP, _I32, _TILE, _VP, _I64, _VP]),
+    "grpo_nf4_tile_linear_one": (
+        _I32,
+        [_VP, _I64, _VP, _VP, _VP, _I32, _VP, _VP, _VP, _I32, _F32, _VP, _I64, _I32, _I32, _I32,
+         _VP],
+    ),
     "grpo_nf4_tile_linear_norm": (
         _I32, [_VP, _I64, _VP, _I32, _VP, _F32, _VP, _VP, _VP, _I32, _TILE, _VP, _I64, _VP]),
     "grpo_nf4_tile_linear_residual": (
@@ -295,7 +300,7 @@ def _load() -> ctypes.CDLL:
 
 def library() -> ctypes.CDLL:
     """The loaded library (no device needed); ImportError if it is not built."""
-    return _load()
+    return _lib if _lib is not None else _load()
 
 
 def device_library() -> ctypes.CDLL:
@@ -305,7 +310,7 @@ def device_library() -> ctypes.CDLL:
     reference's ``except ImportError`` fallback chain behave as they do there.
     """
     global _device_ok, _device_error
-    lib = _load()
+    lib = _lib if _lib is not None else _load()
     if _device_ok is None:
         if not torch.cuda.is_available():
             _device_ok, _device_error = False, "no ROCm/HIP device visible to torch"
@@ -340,7 +345,10 @@ def check(rc: int, what: str) -> None:
 
 def stream_handle(device: torch.device | None = None) -> int:
     """hipStream_t of torch's current stream on ``device`` (as an integer)."""
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)  # no Stream object: 0.2 us of 2
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -22,7 +22,7 @@ with float16 adapters (the reference's float16 X_DTYPE / LORA_DTYPE, ``:141-143,
 take).  The backward (``:761-930``) is ``grpo_nf4_lora_train_backward``: the
 reference's gradients and rounding points, grad_x as one GEMM over the weight
 transposed in 16 bits, everything of rank r straight from x and grad_out.
-Tensors the training kernels do not take (``_train_kernels``), and a backward
+Tensors the training kernels do not take (``_train_workspace``), and a backward
 that is itself differentiated, run the same products as torch ops.
 """
 
@@ -31,14 +31,31 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 
+from ..core.nf4 import float_absmax
 from . import ops
+
+
+_HALF = (torch.bfloat16, torch.float16)
 
 
 def _validate_inputs(x: torch.Tensor, weight_4bit: torch.Tensor, quant_state,
                      lora_A: torch.Tensor, lora_B: torch.Tensor):
     """``lora_forward.py:435-487`` (same messages, same ValueError)."""
+    xs, sa, sb = x.shape, lora_A.shape, lora_B.shape
+    if len(xs) == 3 and len(sa) == 2 and len(sb) == 2 and x.is_cuda and weight_4bit.is_cuda and \
+            lora_A.is_cuda and lora_B.is_cuda and x.dtype in _HALF and lora_A.dtype in _HALF and \
+            lora_A.dtype == lora_B.dtype:
+        n, k = quant_state.shape
+        if xs[2] == k == sa[1] and sb[0] == n and sb[1] == sa[0]:
+            return xs[0] * xs[1], n, k, sa[0]
+    return _validate_each(x, weight_4bit, quant_state, lora_A, lora_B)
+
+
+def _validate_each(x, weight_4bit, quant_state, lora_A, lora_B):
+    """The checks of ``_validate_inputs`` one by one, for their messages."""
     if x.ndim != 3:
         raise ValueError(f"x must be [batch, seq_len, hidden], got {x.shape}.")
     if lora_A.ndim != 2 or lora_B.ndim != 2:
@@ -79,13 +96,14 @@ def _extract_quant_state(weight_4bit: torch.Tensor, quant_state):
     A double-quantized (nested) state's absmax is expanded to float32 once
     (``lora_forward.py:187-199``, see ``core.nf4.float_absmax``) and cached on
     the state: the base weights are frozen."""
-    from ..core.nf4 import float_absmax
-
     device = weight_4bit.device
-    if bool(getattr(quant_state, "nested", False)) and quant_state.absmax.device != device:
+    if getattr(quant_state, "nested", False) and quant_state.absmax.device != device:
         raise ValueError("nested quant_state must be on the weight's device.")
-    absmax = float_absmax(quant_state).to(device=device).contiguous()
-    code = quant_state.code.to(device=device, dtype=torch.float32).contiguous()
+    absmax, code = float_absmax(quant_state), quant_state.code
+    if absmax.device != device or not absmax.is_contiguous():
+        absmax = absmax.to(device=device).contiguous()
+    if code.device != device or code.dtype != torch.float32 or not code.is_contiguous():
+        code = code.to(device=device, dtype=torch.float32).contiguous()
     if absmax.dtype != torch.float32:
         raise ValueError(f"absmax must be float32 for a non-nested state, got {absmax.dtype}.")
     if code.numel() != 16:
@@ -106,7 +124,7 @@ def _bf16_scalar(v: float) -> float:
     return _scalar_as(v, torch.bfloat16)
 
 
-# Where the torch ops run (see _train_kernels): rows of grad_out from which
+# Where the torch ops run (see _train_workspace): rows of grad_out from which
 # grad_x's NF4 product is dequantize + bf16 GEMM instead of the fused nf4_grad_x
 # kernel.  Measured on MI355X at M = 4096
 # over the Qwen2-1.5B projection shapes: the GEMM path is 1.8x (q, o) to 4.2x
@@ -141,20 +159,78 @@ def train_min_rows(k: int, dtype: torch.dtype) -> int:
     return 512 if k <= 4096 else 1536
 
 
-def _train_kernels(w: torch.Tensor, blocksize: int, lora_A: torch.Tensor, lora_B: torch.Tensor,
-                   *rows: torch.Tensor) -> bool:
-    """Whether ``ops.nf4_lora_train_forward`` / ``_backward`` take these tensors: one
-    dtype, N and K multiples of 32, rank <= 32, a power-of-two blocksize >= 32,
-    16-byte aligned (tensors without a storage, as under a vmapped backward, are
-    left to the torch ops)."""
-    if lora_A.dtype != rows[0].dtype or lora_B.dtype != lora_A.dtype or \
-            not ops.nf4_lora_train_workspace_bytes(rows[0].shape[0], lora_B.shape[0],
-                                                   lora_A.shape[1], lora_A.shape[0], blocksize):
-        return False
+def _train_workspace(w: torch.Tensor, blocksize: int, lora_A: torch.Tensor,
+                     lora_B: torch.Tensor, *rows: torch.Tensor) -> int:
+    """Workspace bytes of the training linear for these tensors, 0 if its kernels do
+    not take them: one dtype, N and K multiples of 32, rank <= 32, a power-of-two
+    blocksize >= 32, 16-byte aligned (tensors without a storage, as under a vmapped
+    backward, are left to the torch ops)."""
+    x = rows[0]
+    if lora_A.dtype != x.dtype or lora_B.dtype != x.dtype:
+        return 0
+    r, k = lora_A.shape
+    nbytes = ops.nf4_lora_train_workspace_bytes(x.shape[0], lora_B.shape[0], k, r, blocksize)
+    if not nbytes:
+        return 0
     try:
-        return all(t.data_ptr() % 16 == 0 for t in (w, lora_A, *rows))
+        low = w.data_ptr() | lora_A.data_ptr()
+        for t in rows:
+            low |= t.data_ptr()
     except RuntimeError:
-        return False
+        return 0
+    return nbytes if low % 16 == 0 else 0
+
+
+def _run_forward(x, weight_4bit, quant_state, lora_A, lora_B, scaling, bias):
+    """The fused linear: (output, what its backward needs)."""
+    m, n, k, r = _validate_inputs(x, weight_4bit, quant_state, lora_A, lora_B)
+    if r <= 0:
+        raise ValueError(f"LoRA rank must be > 0, got {r}.")
+    dt = x.dtype
+    if lora_A.dtype != dt:
+        raise ValueError("the HIP NF4+LoRA kernels take x and the adapters in one dtype "
+                         f"(bfloat16 or float16); got x {dt}, lora {lora_A.dtype}.")
+    absmax, code, blocksize = _extract_quant_state(weight_4bit, quant_state)
+    w = weight_4bit if weight_4bit.is_contiguous() else weight_4bit.contiguous()
+    if w.dtype != torch.uint8:
+        w = w.view(-1).view(torch.uint8)
+    x_flat = (x if x.is_contiguous() else x.contiguous()).view(m, k)
+    if w.numel() * 2 < n * k or absmax.numel() * blocksize < n * k:
+        raise ValueError("packed weight or absmax too short for the quant_state's shape.")
+    if bias is not None and (not bias.is_cuda or bias.numel() != n):
+        raise ValueError(f"bias must have {n} elements on the ROCm/HIP device.")
+    nbytes = (_train_workspace(w, blocksize, lora_A, lora_B, x_flat)
+              if m >= train_min_rows(k, dt) else 0)
+    if nbytes:
+        if bias is not None and (bias.dtype != dt or not bias.is_contiguous()):
+            bias = bias.to(dt).contiguous()
+        out = ops.train_forward(x_flat, w, absmax, code, blocksize, lora_A.contiguous(),
+                                lora_B.contiguous(), scaling, bias, nbytes)
+    else:
+        out = _forward_any(x_flat, w, absmax, code, blocksize, n, lora_A, lora_B, scaling, bias)
+    return out.view(x.shape[:-1] + (n,)), (x_flat, lora_A, lora_B, w, absmax, code), blocksize
+
+
+def _forward_any(x_flat, w, absmax, code, blocksize, n, lora_A, lora_B, scaling, bias):
+    """Few rows, and what the training linear does not take."""
+    (m, k), r, dt = x_flat.shape, lora_A.shape[0], x_flat.dtype
+    out = torch.empty((m, n), device=x_flat.device, dtype=dt)
+    if m == 0 or n == 0:
+        return out
+    gemm_ok = m <= fused_forward_rows(k) and ops.nf4_gemm_supported(m, n, k, r, blocksize)
+    if gemm_ok or (dt == torch.bfloat16
+                   and ops.nf4_linear_plan(m, n, k, r, 1, blocksize) is not None):
+        return ops.nf4_lora_linear(x_flat, w, absmax, code, blocksize, n, bias=bias,
+                                   lora_a=lora_A, lora_b=lora_B, scaling=scaling, out=out)
+    # W dequantized once (bit-exact), then GEMMs with the kernel's rounding
+    # points (lora_forward.py:246-257): dt(x W^T), + bias, t = dt(x A^T),
+    # u = dt(dt(t B^T) * dt(scaling)), y = dt(acc + u), dt = bf16 or float16
+    wb = ops.nf4_dequant(w, absmax, code, n * k, blocksize, dtype=dt).view(n, k)
+    acc = F.linear(x_flat, wb)
+    if bias is not None:
+        acc = acc + bias.to(acc.dtype)
+    u = F.linear(F.linear(x_flat, lora_A), lora_B)
+    return torch.add(acc, u * _scalar_as(scaling, dt))
 
 
 class FusedLoRAFunction(torch.autograd.Function):
@@ -164,51 +240,13 @@ class FusedLoRAFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight_4bit, quant_state, lora_A, lora_B, scaling, bias):
-        m, n, k, r = _validate_inputs(x, weight_4bit, quant_state, lora_A, lora_B)
-        if r <= 0:
-            raise ValueError(f"LoRA rank must be > 0, got {r}.")
-        if lora_A.dtype != x.dtype:
-            raise ValueError("the HIP NF4+LoRA kernels take x and the adapters in one dtype "
-                             f"(bfloat16 or float16); got x {x.dtype}, lora {lora_A.dtype}.")
-        dt = x.dtype
-        absmax, code, blocksize = _extract_quant_state(weight_4bit, quant_state)
-        w = weight_4bit.contiguous().view(-1)
-        if w.dtype != torch.uint8:
-            w = w.view(torch.uint8)
-        x_flat = x.contiguous().view(m, k)
-        if m >= train_min_rows(k, dt) and _train_kernels(w, blocksize, lora_A, lora_B, x_flat):
-            out = ops.nf4_lora_train_forward(
-                x_flat, w, absmax, code, blocksize, lora_A.contiguous(), lora_B.contiguous(),
-                float(scaling), None if bias is None else bias.to(dt).contiguous())
-        else:
-            out = FusedLoRAFunction._forward_any(x_flat, w, absmax, code, blocksize, n, lora_A,
-                                                 lora_B, float(scaling), bias)
-        ctx.save_for_backward(x_flat, lora_A, lora_B, w, absmax, code)
-        ctx.blocksize, ctx.scaling, ctx.has_bias = blocksize, float(scaling), bias is not None
+        scaling = float(scaling)
+        out, saved, blocksize = _run_forward(x, weight_4bit, quant_state, lora_A, lora_B, scaling,
+                                             bias)
+        ctx.save_for_backward(*saved)
+        ctx.blocksize, ctx.scaling, ctx.has_bias = blocksize, scaling, bias is not None
         ctx.x_shape = x.shape
-        return out.view(x.shape[:-1] + (n,))
-
-    @staticmethod
-    def _forward_any(x_flat, w, absmax, code, blocksize, n, lora_A, lora_B, scaling, bias):
-        """Few rows, and what the training linear does not take."""
-        (m, k), r, dt = x_flat.shape, lora_A.shape[0], x_flat.dtype
-        out = torch.empty((m, n), device=x_flat.device, dtype=dt)
-        if m == 0 or n == 0:
-            return out
-        gemm_ok = m <= fused_forward_rows(k) and ops.nf4_gemm_supported(m, n, k, r, blocksize)
-        if gemm_ok or (dt == torch.bfloat16
-                       and ops.nf4_linear_plan(m, n, k, r, 1, blocksize) is not None):
-            return ops.nf4_lora_linear(x_flat, w, absmax, code, blocksize, n, bias=bias,
-                                       lora_a=lora_A, lora_b=lora_B, scaling=scaling, out=out)
-        # W dequantized once (bit-exact), then GEMMs with the kernel's rounding
-        # points (lora_forward.py:246-257): dt(x W^T), + bias, t = dt(x A^T),
-        # u = dt(dt(t B^T) * dt(scaling)), y = dt(acc + u), dt = bf16 or float16
-        wb = ops.nf4_dequant(w, absmax, code, n * k, blocksize, dtype=dt).view(n, k)
-        acc = F.linear(x_flat, wb)
-        if bias is not None:
-            acc = acc + bias.to(acc.dtype)
-        u = F.linear(F.linear(x_flat, lora_A), lora_B)
-        return torch.add(acc, u * _scalar_as(scaling, dt))
+        return out
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -221,12 +259,13 @@ class FusedLoRAFunction(torch.autograd.Function):
             g = g.to(dt)
         grad_bias = (g.sum(dim=0) if ctx.has_bias and ctx.needs_input_grad[6]
                      else None)  # lora_forward.py:790
-        if not torch.is_grad_enabled() and m > 0 and \
-                _train_kernels(w, ctx.blocksize, lora_A, lora_B, x_flat, g):
-            need_x, need_a, need_b = (ctx.needs_input_grad[i] for i in (0, 3, 4))
-            grad_x, grad_A, grad_B = ops.nf4_lora_train_backward(
+        nbytes = (_train_workspace(w, ctx.blocksize, lora_A, lora_B, x_flat, g)
+                  if m > 0 and not torch.is_grad_enabled() else 0)
+        if nbytes:
+            need = ctx.needs_input_grad
+            grad_x, grad_A, grad_B = ops.train_backward(
                 x_flat, g, w, absmax, code, ctx.blocksize, lora_A.contiguous(),
-                lora_B.contiguous(), ctx.scaling, need_x, need_a, need_b)
+                lora_B.contiguous(), ctx.scaling, need[0], need[3], need[4], nbytes)
             return (None if grad_x is None else grad_x.view(ctx.x_shape), None, None, grad_A,
                     grad_B, None, grad_bias)
         # scaled_grad = dt(g * dt(scaling)) (:836-837); grad_intermediate,
@@ -263,7 +302,8 @@ def lora_fused_forward(x: torch.Tensor, base_layer=None, lora_A=None, lora_B=Non
         dropout = getattr(lora_layer, "lora_dropout", None)
     if base_layer is None or lora_A is None or lora_B is None or scaling is None:
         raise ValueError("Provide lora_layer or base_layer/lora_A/lora_B/scaling for fused LoRA.")
-    dropout_p = getattr(dropout, "p", 0.0) if dropout is not None else 0.0
+    dropout_p = (0.0 if dropout is None or type(dropout) is torch.nn.Identity
+                 else getattr(dropout, "p", 0.0))
     if dropout_p and dropout_p > 0.0:
         raise ValueError("Dropout is not supported in lora_fused_forward.")
 
@@ -273,9 +313,14 @@ def lora_fused_forward(x: torch.Tensor, base_layer=None, lora_A=None, lora_B=Non
 
     if (not prefer_base_layer and weight_4bit is not None
             and getattr(weight_4bit, "quant_state", None) is not None):
-        return FusedLoRAFunction.apply(x, weight_4bit, weight_4bit.quant_state, lora_A_weight,
-                                       lora_B_weight, float(scaling),
-                                       getattr(base_layer, "bias", None))
+        args = (x, weight_4bit, weight_4bit.quant_state, lora_A_weight, lora_B_weight,
+                float(scaling), getattr(base_layer, "bias", None))
+        # With nothing to record (no grad mode, no forward-mode level, no transform)
+        # the autograd function's own bookkeeping, 5 us of a decode call's 25, is left out.
+        if not torch.is_grad_enabled() and fwAD._current_level < 0 and \
+                not torch._C._are_functorch_transforms_active():
+            return _run_forward(*args)[0]
+        return FusedLoRAFunction.apply(*args)
 
     # Adapter branch (lora_forward.py:986-1037): base layer + the two adapter
     # products, each rounded to the adapter dtype, scaled, cast, added.

@@ -7,6 +7,8 @@ These validate shapes/dtypes on the host (``ValueError``, like the reference's
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from .. import _lib
@@ -133,11 +135,11 @@ def nf4_dequant_t(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor
 
 def nf4_lora_train_workspace_bytes(m: int, n: int, k: int, r: int, blocksize: int) -> int:
     """Workspace of ``nf4_lora_train_forward`` / ``_backward`` (0: unsupported shape)."""
-    return int(_lib.library().grpo_nf4_lora_train_workspace_bytes(m, n, k, r, int(blocksize)))
+    return _lib.library().grpo_nf4_lora_train_workspace_bytes(m, n, k, r, blocksize)
 
 
-def _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, others):
-    """Shape and dtype checks of the training linear; (m, n, k, r, workspace)."""
+def _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, others) -> int:
+    """Shape and dtype checks of the training linear; its workspace bytes."""
     _need_cuda(x, packed, absmax, code, lora_a, lora_b, *others)
     m, k = x.shape
     n, r = lora_b.shape
@@ -152,8 +154,41 @@ def _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, others):
     _need_dtype(absmax, torch.float32, "absmax")
     if packed.numel() * 2 < n * k or absmax.numel() * blocksize < n * k or code.numel() != 16:
         raise ValueError("packed weight or absmax too short for [N, K], or not a 4-bit codebook.")
-    nbytes = nf4_lora_train_workspace_bytes(m, n, k, r, blocksize)
-    return m, n, k, r, torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
+    return nf4_lora_train_workspace_bytes(m, n, k, r, int(blocksize))
+
+
+def train_forward(x, packed, absmax, code, blocksize, lora_a, lora_b, scaling, bias, nbytes):
+    """``nf4_lora_train_forward`` of checked arguments (``nbytes``: their workspace)."""
+    (m, k), (n, r), dev = x.shape, lora_b.shape, x.device
+    y = torch.empty((m, n), dtype=x.dtype, device=dev)
+    ws = torch.empty(nbytes or 16, dtype=torch.uint8, device=dev)
+    rc = _lib.device_library().grpo_nf4_lora_train_forward(
+        x.data_ptr(), k, packed.data_ptr(), absmax.data_ptr(), code.data_ptr(), blocksize,
+        None if bias is None else bias.data_ptr(), lora_a.data_ptr(), lora_b.data_ptr(), r,
+        scaling, y.data_ptr(), n, m, n, k, x.dtype == torch.float16, ws.data_ptr(), nbytes,
+        _lib.stream_handle(dev))
+    if rc:
+        _lib.check(rc, "grpo_nf4_lora_train_forward")
+    return y
+
+
+def train_backward(x, grad, packed, absmax, code, blocksize, lora_a, lora_b, scaling, want_x,
+                   want_a, want_b, nbytes):
+    """``nf4_lora_train_backward`` of checked arguments (``nbytes``: their workspace)."""
+    (m, k), (n, r), dev = x.shape, lora_b.shape, x.device
+    gx = torch.empty_like(x) if want_x else None
+    ga = torch.empty_like(lora_a) if want_a else None
+    gb = torch.empty_like(lora_b) if want_b else None
+    ws = torch.empty(nbytes or 16, dtype=torch.uint8, device=dev)
+    rc = _lib.device_library().grpo_nf4_lora_train_backward(
+        x.data_ptr(), k, grad.data_ptr(), n, packed.data_ptr(), absmax.data_ptr(),
+        code.data_ptr(), blocksize, lora_a.data_ptr(), lora_b.data_ptr(), r, scaling, m, n, k,
+        x.dtype == torch.float16, None if gx is None else gx.data_ptr(), k,
+        None if ga is None else ga.data_ptr(), None if gb is None else gb.data_ptr(),
+        ws.data_ptr(), nbytes, _lib.stream_handle(dev))
+    if rc:
+        _lib.check(rc, "grpo_nf4_lora_train_backward")
+    return gx, ga, gb
 
 
 def nf4_lora_train_forward(x: torch.Tensor, packed: torch.Tensor, absmax: torch.Tensor,
@@ -161,17 +196,12 @@ def nf4_lora_train_forward(x: torch.Tensor, packed: torch.Tensor, absmax: torch.
                            lora_b: torch.Tensor, scaling: float,
                            bias: torch.Tensor | None = None) -> torch.Tensor:
     """``y [M, N]`` of the NF4 + LoRA linear for training batches (bf16 or float16)."""
-    lib = _lib.device_library()
-    m, n, k, r, ws = _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, (bias,))
-    if bias is not None and bias.numel() != n:
-        raise ValueError(f"bias must have {n} elements.")
-    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    _lib.check(lib.grpo_nf4_lora_train_forward(
-        x.data_ptr(), k, packed.data_ptr(), absmax.data_ptr(), code.data_ptr(), int(blocksize),
-        _lib.ptr(bias), lora_a.data_ptr(), lora_b.data_ptr(), r, float(scaling), y.data_ptr(), n,
-        m, n, k, int(x.dtype == torch.float16), ws.data_ptr(), ws.numel(),
-        _lib.stream_handle(x.device)), "grpo_nf4_lora_train_forward")
-    return y
+    _lib.device_library()
+    nbytes = _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, (bias,))
+    if bias is not None and bias.numel() != lora_b.shape[0]:
+        raise ValueError(f"bias must have {lora_b.shape[0]} elements.")
+    return train_forward(x, packed, absmax, code, int(blocksize), lora_a, lora_b, float(scaling),
+                         bias, nbytes)
 
 
 def nf4_lora_train_backward(x: torch.Tensor, grad: torch.Tensor, packed: torch.Tensor,
@@ -179,19 +209,13 @@ def nf4_lora_train_backward(x: torch.Tensor, grad: torch.Tensor, packed: torch.T
                             lora_a: torch.Tensor, lora_b: torch.Tensor, scaling: float,
                             want_x: bool = True, want_a: bool = True, want_b: bool = True):
     """(grad_x, grad_A, grad_B) of the NF4 + LoRA linear (None where not wanted)."""
-    lib = _lib.device_library()
-    m, n, k, r, ws = _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, (grad,))
-    if grad.shape != (m, n):
-        raise ValueError(f"grad must be [{m}, {n}], got {tuple(grad.shape)}.")
-    gx = torch.empty_like(x) if want_x else None
-    ga = torch.empty_like(lora_a) if want_a else None
-    gb = torch.empty_like(lora_b) if want_b else None
-    _lib.check(lib.grpo_nf4_lora_train_backward(
-        x.data_ptr(), k, grad.data_ptr(), n, packed.data_ptr(), absmax.data_ptr(),
-        code.data_ptr(), int(blocksize), lora_a.data_ptr(), lora_b.data_ptr(), r, float(scaling),
-        m, n, k, int(x.dtype == torch.float16), _lib.ptr(gx), k, _lib.ptr(ga), _lib.ptr(gb),
-        ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device)), "grpo_nf4_lora_train_backward")
-    return gx, ga, gb
+    _lib.device_library()
+    nbytes = _check_train(x, packed, absmax, code, blocksize, lora_a, lora_b, (grad,))
+    if grad.shape != (x.shape[0], lora_b.shape[0]):
+        raise ValueError(f"grad must be [{x.shape[0]}, {lora_b.shape[0]}], got "
+                         f"{tuple(grad.shape)}.")
+    return train_backward(x, grad, packed, absmax, code, int(blocksize), lora_a, lora_b,
+                          float(scaling), want_x, want_a, want_b, nbytes)
 
 
 def nf4_grad_x_supported(n: int, k: int, blocksize: int) -> bool:
@@ -245,13 +269,16 @@ def nf4_lora_linear(x2d: torch.Tensor, packed: torch.Tensor, absmax: torch.Tenso
     any M (``y`` float16).
     """
     lib = _lib.device_library()
-    _need_cuda(x2d, packed, absmax, code, bias, lora_a, lora_b)
+    if not (x2d.is_cuda and packed.is_cuda and absmax.is_cuda and code.is_cuda):
+        raise ValueError("all tensors must be on the ROCm/HIP device.")
+    _need_cuda(bias, lora_a, lora_b)
     if x2d.ndim != 2:
         raise ValueError(f"x must be 2-D [M, K], got {tuple(x2d.shape)}.")
     if x2d.dtype == torch.float16:
         return _nf4_lora_linear_f16(lib, x2d, packed, absmax, code, blocksize, n, bias, lora_a,
                                     lora_b, scaling, out)
-    _need_dtype(x2d, torch.bfloat16, "x")
+    bf = torch.bfloat16
+    _need_dtype(x2d, bf, "x")
     m, k = x2d.shape
     if x2d.stride(1) != 1:
         x2d = x2d.contiguous()
@@ -260,45 +287,39 @@ def nf4_lora_linear(x2d: torch.Tensor, packed: torch.Tensor, absmax: torch.Tenso
         r = lora_a.shape[0]
         if lora_a.shape != (r, k) or lora_b is None or lora_b.shape != (n, r):
             raise ValueError("lora_A must be [r, K] and lora_B [N, r].")
-        _need_dtype(lora_a, torch.bfloat16, "lora_A")
-        _need_dtype(lora_b, torch.bfloat16, "lora_B")
+        if lora_a.dtype != bf or lora_b.dtype != bf:
+            _need_dtype(lora_a, bf, "lora_A")
+            _need_dtype(lora_b, bf, "lora_B")
         lora_a, lora_b = lora_a.contiguous(), lora_b.contiguous()
     if bias is not None:
         if bias.numel() != n:
             raise ValueError(f"bias must have {n} elements.")
-        bias = bias.to(torch.bfloat16).contiguous()
+        if bias.dtype != bf or not bias.is_contiguous():
+            bias = bias.to(bf).contiguous()
     if packed.numel() * 2 < n * k:
         raise ValueError("packed weight smaller than N*K/2 bytes.")
+    dev, ldx, xp, wp = x2d.device, x2d.stride(0), x2d.data_ptr(), packed.data_ptr()
     if out is None:
-        out = torch.empty((m, n), dtype=torch.bfloat16, device=x2d.device)
-    elif out.shape != (m, n) or out.stride(1) != 1 or out.dtype != torch.bfloat16:
+        out = torch.empty((m, n), dtype=bf, device=dev)
+    elif out.shape != (m, n) or out.stride(1) != 1 or out.dtype != bf:
         raise ValueError("out must be a bf16 [M, N] tensor with unit column stride.")
-    if (m <= TILE_MAX_ROWS and x2d.stride(0) % 8 == 0 and x2d.data_ptr() % 16 == 0
-            and packed.data_ptr() % 16 == 0 and out.data_ptr() % 2 == 0
-            and lib.grpo_nf4_tile_supported(m, n, k, r, 1, int(blocksize))):
+    bp, st = _lib.ptr(bias), _lib.stream_handle(dev)
+    if m <= TILE_MAX_ROWS and ldx % 8 == 0 and xp % 16 == 0 and wp % 16 == 0 and \
+            lib.grpo_nf4_tile_supported(m, n, k, r, 1, int(blocksize)):
         # decode batches: the one-launch tile linear (LoRA A in its packed
         # order, built once per A version)
-        d = _lib.TileLinear()
-        d.M, d.N, d.K, d.nseg, d.r = m, n, k, 1, r
-        d.seg_end[0] = n
-        d.bias[0] = _lib.ptr(bias)
-        if r > 0:
-            d.lora_a[0] = packed_lora_a(lora_a).data_ptr()
-            d.lora_b[0] = lora_b.data_ptr()
-        d.scaling = float(scaling)
-        rc = lib.grpo_nf4_tile_linear(x2d.data_ptr(), x2d.stride(0), packed.data_ptr(),
-                                      absmax.data_ptr(), code.data_ptr(), int(blocksize),
-                                      ctypes_byref(d), out.data_ptr(), out.stride(0),
-                                      _lib.stream_handle(x2d.device))
+        rc = lib.grpo_nf4_tile_linear_one(
+            xp, ldx, wp, absmax.data_ptr(), code.data_ptr(), int(blocksize), bp,
+            packed_lora_a(lora_a).data_ptr() if r > 0 else None, _lib.ptr(lora_b), r,
+            float(scaling), out.data_ptr(), out.stride(0), m, n, k, st)
         _lib.check(rc, "grpo_nf4_tile_linear")
         return out
     nbytes = int(lib.grpo_nf4_lora_linear_workspace_bytes(m, n, k, r, 1, int(blocksize)))
-    ws = workspace("nf4_linear", nbytes, x2d.device)
+    ws = workspace("nf4_linear", nbytes, dev)
     rc = lib.grpo_nf4_lora_linear(
-        x2d.data_ptr(), x2d.stride(0), packed.data_ptr(), absmax.data_ptr(), code.data_ptr(),
-        int(blocksize), _lib.ptr(bias), _lib.ptr(lora_a), _lib.ptr(lora_b), r, float(scaling),
-        out.data_ptr(), out.stride(0), m, n, k, _lib.ptr(ws), 0 if ws is None else ws.numel(),
-        _lib.stream_handle(x2d.device))
+        xp, ldx, wp, absmax.data_ptr(), code.data_ptr(), int(blocksize), bp, _lib.ptr(lora_a),
+        _lib.ptr(lora_b), r, float(scaling), out.data_ptr(), out.stride(0), m, n, k, _lib.ptr(ws),
+        0 if ws is None else ws.numel(), st)
     _lib.check(rc, "grpo_nf4_lora_linear")
     return out
 
@@ -486,26 +507,37 @@ def nf4_linear_plan(m: int, n: int, k: int, r: int, nseg: int,
 
 # ----------------------------------------------------------- paged KV ---
 
-def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
-    if k_cache.ndim != 4 or v_cache.ndim != 4:
+_BF16, _I32 = torch.bfloat16, torch.int32
+
+
+def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor) -> torch.Size:
+    shape = k_cache.shape
+    if len(shape) != 4 or v_cache.ndim != 4:
         raise ValueError("k_cache/v_cache must be [num_blocks, heads, block, head_dim].")
-    if k_cache.shape != v_cache.shape:
+    if shape != v_cache.shape:
         raise ValueError("k_cache and v_cache must have identical shapes.")
-    _need_dtype(k_cache, torch.bfloat16, "k_cache")
-    _need_dtype(v_cache, torch.bfloat16, "v_cache")
+    if k_cache.dtype != _BF16 or v_cache.dtype != _BF16:
+        _need_dtype(k_cache, _BF16, "k_cache")
+        _need_dtype(v_cache, _BF16, "v_cache")
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise ValueError("k_cache/v_cache must be contiguous.")
+    return shape
 
 
-def _check_tables(block_tables: torch.Tensor, context_lens: torch.Tensor, b: int) -> None:
-    if block_tables.ndim != 2 or block_tables.shape[0] != b:
+def _check_tables(block_tables: torch.Tensor, context_lens: torch.Tensor, b: int):
+    """(row stride, max_blocks) of checked tables."""
+    shape = block_tables.shape
+    if len(shape) != 2 or shape[0] != b:
         raise ValueError("block_tables must be [batch, max_blocks].")
-    if context_lens.ndim != 1 or context_lens.shape[0] != b:
+    if context_lens.shape != (b,):
         raise ValueError("context_lens must be [batch].")
-    _need_dtype(block_tables, torch.int32, "block_tables")
-    _need_dtype(context_lens, torch.int32, "context_lens")
-    if block_tables.stride(1) != 1 or not context_lens.is_contiguous():
+    if block_tables.dtype != _I32 or context_lens.dtype != _I32:
+        _need_dtype(block_tables, _I32, "block_tables")
+        _need_dtype(context_lens, _I32, "context_lens")
+    row, col = block_tables.stride()
+    if col != 1 or not context_lens.is_contiguous():
         raise ValueError("block_tables rows and context_lens must be contiguous.")
+    return row, shape[1]
 
 
 def paged_kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Tensor,
@@ -513,22 +545,25 @@ def paged_kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Ten
                     context_lens: torch.Tensor) -> None:
     """Write ``k_new/v_new [B, Hkv, D]`` at slot ``context_lens[b]`` of each sequence."""
     lib = _lib.device_library()
-    _need_cuda(k_new, v_new, k_cache, v_cache, block_tables, context_lens)
-    _check_cache(k_cache, v_cache)
-    nb, hkv, bs, d = k_cache.shape
-    if k_new.shape != v_new.shape or k_new.ndim != 3 or k_new.shape[1:] != (hkv, d):
+    if not (k_new.is_cuda and v_new.is_cuda and k_cache.is_cuda and v_cache.is_cuda
+            and block_tables.is_cuda and context_lens.is_cuda):
+        raise ValueError("all tensors must be on the ROCm/HIP device.")
+    nb, hkv, bs, d = _check_cache(k_cache, v_cache)
+    shape = k_new.shape
+    if shape != v_new.shape or len(shape) != 3 or shape[1:] != (hkv, d):
         raise ValueError(f"k_new/v_new must be [B, {hkv}, {d}].")
-    b = k_new.shape[0]
-    _check_tables(block_tables, context_lens, b)
-    k_new = k_new.to(torch.bfloat16)
-    v_new = v_new.to(torch.bfloat16)
-    if k_new.stride(2) != 1 or k_new.stride() != v_new.stride():
+    b = shape[0]
+    row, max_blocks = _check_tables(block_tables, context_lens, b)
+    k_new = k_new.to(_BF16)
+    v_new = v_new.to(_BF16)
+    st = k_new.stride()
+    if st[2] != 1 or st != v_new.stride():
         k_new, v_new = k_new.contiguous(), v_new.contiguous()
+        st = k_new.stride()
     rc = lib.grpo_paged_kv_append(
-        k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1), k_cache.data_ptr(),
-        v_cache.data_ptr(), nb, block_tables.data_ptr(), block_tables.stride(0),
-        context_lens.data_ptr(), b, hkv, d, bs, block_tables.shape[1],
-        _lib.stream_handle(k_cache.device))
+        k_new.data_ptr(), v_new.data_ptr(), st[0], st[1], k_cache.data_ptr(),
+        v_cache.data_ptr(), nb, block_tables.data_ptr(), row, context_lens.data_ptr(), b, hkv, d,
+        bs, max_blocks, _lib.stream_handle(k_cache.device))
     _lib.check(rc, "grpo_paged_kv_append")
 
 
@@ -545,14 +580,20 @@ _attn_merge: dict = {}
 ATTN_ONE_LAUNCH = True
 
 
-def _attn_merge_state(lib, device, b: int, hkv: int):
-    need = max(int(lib.grpo_paged_attn_merge_counter_bytes(b, hkv)) // 4, 1)
-    key = device if isinstance(device, torch.device) else torch.device(device)
-    st = _attn_merge.get(key)
+@functools.lru_cache(maxsize=1024)
+def _attn_plan(b: int, hq: int, hkv: int, d: int, bs: int, max_blocks: int) -> tuple[int, int]:
+    """(workspace bytes, merge counters) of an attention call of this shape."""
+    lib = _lib.library()
+    return (int(lib.grpo_paged_attn_workspace_bytes(b, hq, hkv, d, bs, max_blocks)),
+            max(int(lib.grpo_paged_attn_merge_counter_bytes(b, hkv)) // 4, 1))
+
+
+def _attn_merge_state(device, need: int):
+    st = _attn_merge.get(device)
     if st is None or st[0].numel() < need:
-        err = st[1] if st is not None else torch.zeros(1, dtype=torch.int32, device=key)
-        st = (torch.zeros(need, dtype=torch.int32, device=key), err)
-        _attn_merge[key] = st
+        err = st[1] if st is not None else torch.zeros(1, dtype=torch.int32, device=device)
+        st = (torch.zeros(need, dtype=torch.int32, device=device), err)
+        _attn_merge[device] = st
     return st
 
 
@@ -594,45 +635,43 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     library's per-GPU scratch array, no workspace, split + merge launches);
     ``out`` must then be given for the call to allocate nothing at all."""
     lib = _lib.device_library()
-    _need_cuda(q, k_cache, v_cache, block_tables, context_lens)
-    _check_cache(k_cache, v_cache)
-    nb, hkv, bs, d = k_cache.shape
-    if q.ndim != 3 or q.shape[2] != d:
+    if not (q.is_cuda and k_cache.is_cuda and v_cache.is_cuda and block_tables.is_cuda
+            and context_lens.is_cuda):
+        raise ValueError("all tensors must be on the ROCm/HIP device.")
+    nb, hkv, bs, d = _check_cache(k_cache, v_cache)
+    shape, dev = q.shape, q.device
+    if len(shape) != 3 or shape[2] != d:
         raise ValueError(f"q must be [B, Hq, {d}].")
-    b, hq, _ = q.shape
+    b, hq, _ = shape
     if hq % hkv != 0:
         raise ValueError(f"query heads ({hq}) must be a multiple of KV heads ({hkv}).")
-    _check_tables(block_tables, context_lens, b)
-    q = q.to(torch.bfloat16)
-    if q.stride(2) != 1:
+    row, max_blocks = _check_tables(block_tables, context_lens, b)
+    q = q.to(_BF16)
+    qsb, qsh, qsd = q.stride()
+    if qsd != 1:
         q = q.contiguous()
-    if out_dtype not in (torch.float32, torch.bfloat16):
+        qsb, qsh, _ = q.stride()
+    if out_dtype not in (torch.float32, _BF16):
         raise ValueError("out_dtype must be float32 or bfloat16.")
     if out is None:
-        out = torch.empty((b, hq, d), dtype=out_dtype, device=q.device)
+        out = torch.empty(shape, dtype=out_dtype, device=dev)
     elif out.shape != (b, hq, d) or not out.is_contiguous() or out.dtype != out_dtype:
         raise ValueError("out must be a contiguous [B, Hq, D] tensor of out_dtype.")
-    max_blocks = block_tables.shape[1]
+    st = _lib.stream_handle(dev)
+    args = (q.data_ptr(), qsb, qsh, k_cache.data_ptr(), v_cache.data_ptr(), nb,
+            block_tables.data_ptr(), row, context_lens.data_ptr(), out.data_ptr(),
+            1 if out_dtype == _BF16 else 0, b, hq, hkv, d, bs, max_blocks, float(scale))
     if no_alloc:
-        rc = lib.grpo_paged_attn_decode_noalloc(
-            q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), nb,
-            block_tables.data_ptr(), block_tables.stride(0), context_lens.data_ptr(),
-            out.data_ptr(), 1 if out_dtype == torch.bfloat16 else 0, b, hq, hkv, d, bs,
-            max_blocks, float(scale), _lib.stream_handle(q.device))
-        _lib.check(rc, "grpo_paged_attn_decode_noalloc")
+        _lib.check(lib.grpo_paged_attn_decode_noalloc(*args, st),
+                   "grpo_paged_attn_decode_noalloc")
         return out
-    nbytes = int(lib.grpo_paged_attn_workspace_bytes(b, hq, hkv, d, bs, max_blocks))
-    ws = workspace("paged_attn", nbytes, q.device)
-    args = (q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), nb,
-            block_tables.data_ptr(), block_tables.stride(0), context_lens.data_ptr(),
-            out.data_ptr(), 1 if out_dtype == torch.bfloat16 else 0, b, hq, hkv, d, bs,
-            max_blocks, float(scale), _lib.ptr(ws), 0 if ws is None else ws.numel())
+    nbytes, counters = _attn_plan(b, hq, hkv, d, bs, max_blocks)
+    ws = workspace("paged_attn", nbytes, dev)
+    args += (_lib.ptr(ws), 0 if ws is None else ws.numel())
     if ATTN_ONE_LAUNCH:
-        cnt, err = _attn_merge_state(lib, q.device, b, hkv)
-        rc = lib.grpo_paged_attn_decode_merged(*args, cnt.data_ptr(), err.data_ptr(),
-                                               _lib.stream_handle(q.device))
-        _lib.check(rc, "grpo_paged_attn_decode_merged")
+        cnt, err = _attn_merge_state(dev, counters)
+        _lib.check(lib.grpo_paged_attn_decode_merged(*args, cnt.data_ptr(), err.data_ptr(), st),
+                   "grpo_paged_attn_decode_merged")
     else:
-        rc = lib.grpo_paged_attn_decode(*args, _lib.stream_handle(q.device))
-        _lib.check(rc, "grpo_paged_attn_decode")
+        _lib.check(lib.grpo_paged_attn_decode(*args, st), "grpo_paged_attn_decode")
     return out

@@ -236,6 +236,13 @@ int grpo_nf4_tile_linear(const void* x, int64_t ldx, const uint8_t* w, const flo
                          const float* code16, int blocksize, const grpo_tile_linear_t* lin,
                          void* y, int64_t ldy, grpo_stream_t stream);
 
+/* grpo_nf4_tile_linear of one segment without a descriptor; GRPO_EUNSUPPORTED
+ * for shapes that grpo_nf4_tile_supported refuses. */
+int grpo_nf4_tile_linear_one(const void* x, int64_t ldx, const uint8_t* w, const float* absmax,
+                             const float* code16, int blocksize, const void* bias,
+                             const void* lora_a_packed, const void* lora_b, int r, float scaling,
+                             void* y, int64_t ldy, int M, int N, int K, grpo_stream_t stream);
+
 /* grpo_nf4_tile_linear with x = RMSNorm(h) = bf16(bf16(h * inv) * norm_weight),
  * inv = 1 / sqrt(sum_g sumsq[m, g] / K + eps) (groups: a multiple of 4, <= 256
  * partial sums of h^2 per row, as grpo_nf4_linear_residual /

@@ -145,3 +145,50 @@ def test_dequant_runs_of_eight(dev, n, k, bs, dt):
     want = (nf4_code(dev)[q] * absmax.repeat_interleave(bs)[:n * k]).to(dt)
     got = ops.nf4_dequant(packed, absmax, nf4_code(dev), n * k, bs, dtype=dt)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_no_grad_call_is_the_recorded_one(dev):
+    """Without grad mode the autograd function is passed by: the same output, and a
+    forward-mode level, a transform or grad mode still goes through it; arguments
+    the kernels must not see stay refused."""
+    from grpo_mi355x.core.lora import ManualLoRALayer
+    from grpo_mi355x.core.nf4 import Linear4bitNF4
+    from grpo_mi355x.kernels import lora_forward as L, lora_fused_forward
+
+    torch.manual_seed(0)
+    base = Linear4bitNF4.from_weight(torch.randn(256, 512, device=dev) * 0.02,
+                                     torch.randn(256, device=dev))
+    layer = ManualLoRALayer(base).to(dev).bfloat16()
+    torch.nn.init.normal_(layer.lora_B.weight, std=0.05)
+    called, apply = [], L.FusedLoRAFunction.apply
+    for m in (8, 100, 600):
+        x = torch.randn(1, m, 512, device=dev).bfloat16()
+        want = lora_fused_forward(x, lora_layer=layer)
+        assert want.grad_fn is not None
+        with torch.no_grad():
+            got = lora_fused_forward(x, lora_layer=layer)
+        assert got.grad_fn is None and torch.equal(got, want.detach())
+    L.FusedLoRAFunction.apply = staticmethod(lambda *a: called.append(1) or apply(*a))
+    try:
+        with torch.no_grad():
+            lora_fused_forward(x, lora_layer=layer)
+            assert not called
+            with torch.autograd.forward_ad.dual_level():
+                lora_fused_forward(x, lora_layer=layer)
+            assert len(called) == 1
+    finally:
+        L.FusedLoRAFunction.apply = apply
+    with torch.no_grad():
+        for bad in (torch.zeros(255, device=dev), torch.zeros(256)):
+            base.bias = torch.nn.Parameter(bad, requires_grad=False)
+            with pytest.raises(ValueError):
+                lora_fused_forward(x, lora_layer=layer)
+        base.bias = None
+        full, base.weight.quant_state.absmax = base.weight.quant_state.absmax, \
+            base.weight.quant_state.absmax[:-1]
+        with pytest.raises(ValueError):
+            lora_fused_forward(x, lora_layer=layer)
+        base.weight.quant_state.absmax = full
+        # vmap: no storage to hand to a kernel; the layer's torch branch serves it
+        y = torch.vmap(lambda t: layer(t))(torch.stack([x, 2 * x]))
+        assert y.shape == (2, 1, 600, 256)
