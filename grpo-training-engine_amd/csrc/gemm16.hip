@@ -16,9 +16,7 @@
 //    first half the second half's operands are read, then comes the step's one
 //    barrier (the next stage has landed), and during the second half the
 //    next stage's operands are read and the stage three ahead is fetched, one
-//    load after each row of MFMAs. The loads are volatile asm without results, and
-//    every wait for them is explicit: the compiler, which does not tell the ring's
-//    stages apart, would wait for all of them before each operand read.
+//    load after each row of MFMAs (loads and waits: lds_dma.hpp).
 //  * Tiles go to the XCDs in eight equal runs, in groups of a few rows of tiles,
 //    so that the tiles that run together on an XCD share operands in its L2.
 //
@@ -31,6 +29,7 @@
 // 1024 x 1024 5.4 us (19.3). The library's products need one more pass over C for
 // each of bias, LoRA term and sum.
 #include "gemm16.hpp"
+#include "lds_dma.hpp"
 
 #include <algorithm>
 
@@ -45,19 +44,6 @@ struct Args {
   int MT, NT;
   bool lowvec;  // 16-byte loads of low's rows
 };
-
-// 16 bytes per lane from base + voff to the wave's 1 KiB at LDS address lds.
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds),
-               "v"(voff), "s"(base)
-               : "memory");
-}
-
-// Wait until at most N vector memory operations are outstanding.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
 
 // RM x RN tiles of 16 x 16 per wave, WM x WN waves, GROUP rows of tiles.
 template <bool F16, Gemm16Mode MODE, int RM, int RN, int WM, int WN, int GROUP>
@@ -98,7 +84,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm16_kernel(Args p) {
   }
   const int nst = g.K / 32;
   const uint32_t lbase =
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds + wave * LD * PIECE * 2;
+      lds_address(lds) + wave * LD * PIECE * 2;
   // stages past the end repeat the last one into slots that are not multiplied
   auto fetch = [&](int st, int i) __attribute__((always_inline)) {
     dma16(lbase + (st % RING) * (ST * 2) + i * PIECE * 2, voff[i],

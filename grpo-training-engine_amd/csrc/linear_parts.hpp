@@ -65,7 +65,7 @@ struct GemmPlan {
   size_t part_bytes, tpart_bytes;
 };
 bool nf4_gemm_ok(int M, int N, int K, int r, int blocksize);
-GemmPlan nf4_gemm_plan(int M, int K, int r, int nseg, const int* seg_end);
+GemmPlan nf4_gemm_plan(int M, int K, int r, int blocksize, int nseg, const int* seg_end);
 // The MLP's gate|up projection + SiLU*up on the NF4 GEMM (more than 64 rows):
 // act[M, I] = bf16(bf16(silu(x Wg^T)) * bf16(x Wu^T)), W = [2I, K] stacked.
 bool nf4_gemm_silu_ok(int M, int I, int K, int blocksize);

@@ -32,9 +32,13 @@
 //    tiles, column tile by column tile, are cut into 8 equal runs and run x
 //    goes to the ids = x mod 8, so the row tiles of a column tile read its
 //    weights through one L2 and every XCD gets the same number of tiles.
+//
+// bf16 with K % 128 == 0, r <= 16 and blocksize >= 64 runs nf4_gemm_k2 (below) instead,
+// which was no slower at any of 45 measured shapes of 128 .. 2048 rows.
 #include <algorithm>
 #include <type_traits>
 
+#include "lds_dma.hpp"
 #include "linear_parts.hpp"
 #include "nf4_decode.hpp"
 
@@ -470,6 +474,563 @@ __global__ void __launch_bounds__(256) nf4_finish_rows(LinParts o, uint16_t* __r
   }
 }
 
+// ------------------------------------------------- K in steps of 128, bf16 --
+//
+// The same linear for K % 128 == 0 and r <= 16 on the ring of gemm16.hip: x comes to LDS
+// by global_load_lds in stages of 32 K values, four in flight, and the weight is
+// decoded once per workgroup (not once per 32-column wave) into LDS, in the piece order
+// its operand reads want.
+//  * Superstage = 128 K values = four stages. Its packed bytes (16 rows x 64 bytes per
+//    1 KiB piece), absmax (one per row and stage) and LoRA A rows come to LDS too,
+//    into a ring of three: the one being decoded, the next and the one being fetched.
+//  * Step st multiplies stage st, decodes stage st + 2 (a thread: 8 or 16 nibbles of
+//    one row, whose codebook is built once per stage, or per two where the absmax
+//    block has 64 values or more), fetches stage st + 3 of x and a quarter of the
+//    superstage after next. The decoded stages alternate between two LDS slots: the
+//    slot written in step st was read before its barrier. Every wait counts loads.
+//  * LoRA: x A^T is one more MFMA column of the tile, its rows shared out among the
+//    waves; t passes through LDS once and its product with B is one MFMA per tile.
+//  * SILU: the four column tiles of a wave are gate, gate, up, up of the same 32
+//    columns, so a lane ends with both factors of 8 activation columns.
+//  * KS = 2: two K groups of waves, each with rings of its own, halve the chain of
+//    steps of a small launch; they exchange halves of their sums through LDS.
+// Bound by the vector ALUs' decode beside the MFMAs (about 90 vector instructions per
+// stage and wave against 16 MFMAs of 16 cycles on the 128 x 128 tile), and below one
+// workgroup per CU by the chain of a step (LDS, decode, barrier: 0.32 us per 64 K
+// values at 64 x 64). Against nf4_gemm_mfma, us at 511 rows: 2048 x 1536, r 16: 28.2 ->
+// 13.9; 1536 x 1536, r 16: 24.1 -> 13.3; gate|up 2 x 8960 x 1536: 64.6 -> 51.9; 1536 x
+// 8960: 37.5 -> 36.6; 4608 x 3584, r 16: 55.5 -> 45.1; at 2048 rows: 39.2 -> 27.1, 38.2
+// -> 25.9, 177.7 -> 155.3, 111.6 -> 91.5, 158.1 -> 136.4.
+struct K2Args {
+  const uint16_t* x;
+  int64_t ldx;
+  const uint8_t* w;
+  const float* absmax;
+  const float* code16;
+  int bs_shift;
+  int nseg;
+  int seg_end[MAXSEG];
+  int seg_tile[MAXSEG + 1];
+  const uint16_t* bias[MAXSEG];
+  const uint16_t* la[MAXSEG];
+  const uint16_t* lb[MAXSEG];
+  int r;
+  float scaling;
+  uint16_t* y;
+  int64_t ldy;
+  int M, K;
+  int MT, NT;
+  int nss;  // superstages
+  int kst;  // superstages per K slice (gridDim.y slices)
+  bool yvec, lbvec;  // 16-byte stores of y, 16-byte loads of LoRA B
+  float* part;  // K slices: part[slice][m][n] (slice stride psl, row stride ldp)
+  int64_t ldp, psl;
+  float* tpart;  // LoRA t partials [slice][16] at segment stride tseg
+  int64_t tsl, tseg;
+  int silu_I;
+};
+
+enum K2Mode { K2_OUT, K2_PART, K2_SILU };
+
+template <K2Mode MODE, bool LORA, int RM, int RN, int WM, int WN, int KS>
+struct K2Shape {
+  static constexpr int BM = 16 * RM * WM, BN = 16 * RN * WN, W = WM * WN, T = 64 * W;
+  static constexpr int TA = BM / 16, TB = BN / 16;     // pieces of a stage of x, of the weight
+  static constexpr int LDA = TA / W, LDX = LDA + LORA; // x, x and LoRA A loads per wave and step
+  static constexpr int EW = TB / W, EA = 1, E = EW + EA;  // other loads per wave and superstage
+  static constexpr int TPR = T / BN;                   // threads per weight row
+  static constexpr int ST = (TA + LORA) * 1024, SB = TB * 1024;  // bytes of a stage
+  static constexpr int RAW = TB * 1024 + 8 * BN;       // a superstage's packed bytes, absmax
+  static constexpr int XS = 4 * ST, BS = 2 * SB, LDS = XS + BS + 3 * RAW;  // of a K group
+  // exchange of two K groups: sums from 0, t sums from XT, then t
+  static constexpr int XT = W * RM * RN * 1024;
+  static constexpr int TS = XT + (LORA ? 2 * W * (RM / WN > 0 ? RM / WN : 1) * 1024 : 0);
+  static_assert(KS == 1 || (KS == 2 && TS + (LORA ? BM * 64 : 0) <= 2 * LDS), "exchange");
+  static constexpr int ex(int j) { return ((j & 3) + 1) * E / 4 - (j & 3) * E / 4; }
+  static_assert(TA % W == 0 && TB % W == 0 && (!LORA || W == 4) && BN / 32 <= W && TPR >= 1 && 4 % TPR == 0, "");
+};
+
+template <K2Mode MODE, bool LORA, int RM, int RN, int WM, int WN, int KS>
+__global__ void __launch_bounds__(64 * WM * WN * KS, 2) nf4_gemm_k2(K2Args p) {
+  using S = K2Shape<MODE, LORA, RM, RN, WM, WN, KS>;
+  constexpr int BN = S::BN, W = S::W, RH = RM / 2, NIB = 32 / S::TPR;
+  constexpr bool SILU = MODE == K2_SILU;
+  static_assert(!SILU || (RN == 4 && !LORA), "gate, gate, up, up");
+  extern __shared__ __align__(16) char smem0[];
+  // K group of this wave, thread and wave in the group
+  const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / S::T);
+  const int tid = threadIdx.x % S::T, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  char* const smem = smem0 + grp * S::LDS;
+  const int ln = lane & 15, lg = lane >> 4;
+  const int bx = blockIdx.x, run = bx & 7, T = p.MT * p.NT;
+  const int t = ((run * T) >> 3) + (bx >> 3);
+  if (t >= (((run + 1) * T) >> 3)) return;  // past the end of this run
+  const int nt = t / p.MT, mt = t - nt * p.MT;
+  const int seg = (nt >= p.seg_tile[1]) + (nt >= p.seg_tile[2]) + (nt >= p.seg_tile[3]);
+  const int c0 = seg > 0 ? sel4(p.seg_end[0], p.seg_end[1], p.seg_end[2], p.seg_end[3],
+                                seg - 1) : 0;
+  const int N = sel4(p.seg_end[0], p.seg_end[1], p.seg_end[2], p.seg_end[3], seg) - c0;
+  const uint16_t* const sbias = sel4(p.bias[0], p.bias[1], p.bias[2], p.bias[3], seg);
+  const uint16_t* const sla = sel4(p.la[0], p.la[1], p.la[2], p.la[3], seg);
+  const uint16_t* const slb = sel4(p.lb[0], p.lb[1], p.lb[2], p.lb[3], seg);
+  const int lt = nt - sel4(p.seg_tile[0], p.seg_tile[1], p.seg_tile[2], p.seg_tile[3], seg);
+  const int m0 = mt * S::BM, n0 = lt * (SILU ? BN / 2 : BN);
+
+  // weight row (of the whole stacked weight) of row i of piece pb
+  auto wrow = [&](int pb, int i) __attribute__((always_inline)) {
+    const int g = pb / RN, j = pb % RN;
+    if (SILU) {
+      const int a = n0 + 32 * g + 8 * (i >> 2) + 4 * (j & 1) + (i & 3);
+      return (j >> 1) * p.silu_I + min(a, p.silu_I - 1);
+    }
+    return c0 + min(n0 + 16 * RN * g + 4 * RN * (i >> 2) + 4 * j + (i & 3), N - 1);
+  };
+  // superstages of this workgroup, of this group (the second's may be none: its loads
+  // then repeat valid ones)
+  const int wss0 = blockIdx.y * p.kst, wnss = min(p.nss, wss0 + p.kst) - wss0;
+  const int lss = KS == 1 ? wnss : (wnss + 1) >> 1;  // of the longer group
+  const int nst = 4 * (grp == 0 ? lss : wnss - lss), last = max(nst, 4) - 1;
+  const int64_t k0 = 128 * (int64_t)min(wss0 + grp * lss, p.nss - 1);
+  const uint32_t lb0 = lds_address(smem);
+
+  // x: this wave's pieces of a stage
+  const int prow = lane >> 2, pch = (lane & 3) ^ ((prow >> 1) & 3);
+  const char* const xb = reinterpret_cast<const char*>(p.x + (int64_t)m0 * p.ldx + k0);
+  uint32_t xoff[S::LDA];
+#pragma unroll
+  for (int i = 0; i < S::LDA; ++i)
+    xoff[i] = min(16 * (wave * S::LDA + i) + prow, p.M - 1 - m0) * (uint32_t)(2 * p.ldx) + 16 * pch;
+  auto fetch_x = [&](int st, int i) __attribute__((always_inline)) {
+    dma16(lb0 + (st & 3) * S::ST + (wave * S::LDA + i) * 1024, xoff[i],
+          xb + 64 * (int64_t)min(st, last));
+  };
+  // packed weight: piece e W + wave, 16 rows x 64 bytes, chunk ^ (row / 4 % 4)
+  const int wch = (lane & 3) ^ ((prow >> 2) & 3);
+  uint32_t woff[S::EW];
+#pragma unroll
+  for (int e = 0; e < S::EW; ++e)
+    woff[e] = (uint32_t)wrow(e * W + wave, prow) * (uint32_t)(p.K / 2) + 16 * wch;
+  const char* const wb = reinterpret_cast<const char*>(p.w) + k0 / 2;
+  // LoRA A of a stage: this wave's 256 bytes (4 rows), ranks >= r repeat rank r - 1
+  const int lrow = 4 * wave + (lane >> 4), lch = ((lane >> 2) & 3) ^ ((lrow >> 1) & 3);
+  const uint32_t loff =
+      LORA ? min(lrow, p.r - 1) * (uint32_t)(2 * p.K) + 16 * lch + 4 * (lane & 3) : 0;
+  const char* const lab = reinterpret_cast<const char*>(sla) + 2 * k0;
+  auto fetch_l = [&](int st) __attribute__((always_inline)) {
+    if (LORA)
+      dma4(lb0 + (st & 3) * S::ST + S::TA * 1024 + wave * 256, loff,
+           lab + 64 * (int64_t)min(st, last));
+  };
+  // absmax: 64 values of the superstage's half id % 2, rows 64 (id / 2) + lane of the
+  // piece order (id = wave, modulo what there is)
+  const int aid = wave % (BN / 32), arho = 64 * (aid >> 1) + lane;
+  const uint32_t aidx = (uint32_t)wrow(arho >> 4, arho & 15) * (uint32_t)p.K + (uint32_t)k0 +
+                        64 * (aid & 1);
+  constexpr int OA = S::TB * 1024;  // absmax in a raw slot: [half][row]
+  auto fetch_raw = [&](int ss, int e) __attribute__((always_inline)) {
+    const uint32_t slot = lb0 + S::XS + S::BS + (ss % 3) * S::RAW;
+    const int sc = min(ss, last >> 2);
+    if (e < S::EW)
+      dma16(slot + (e * W + wave) * 1024, woff[e], wb + 64 * (int64_t)sc);
+    else
+      dma4(slot + OA + ((aid & 1) * BN + 64 * (aid >> 1)) * 4,
+           ((aidx + 128u * sc) >> p.bs_shift) * 4, p.absmax);
+  };
+  // the extra loads of phase j: raw loads [j E / 4, (j + 1) E / 4) of superstage ss
+  auto extras = [&](int ss, auto jc) __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+#pragma unroll
+    for (int e = j * S::E / 4; e < (j + 1) * S::E / 4; ++e) fetch_raw(ss, e);
+  };
+
+  float code[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) code[j] = load_uniform(p.code16 + j);
+  const int rho = tid / S::TPR, sub = tid % S::TPR, dr = rho & 15;
+  const int wread = (rho >> 4) * 1024 + dr * 64 + (16 / S::TPR) * sub, wsw = (dr >> 2) & 3;
+  char* const bw = smem + S::XS + (rho >> 4) * 1024 + dr * 64;
+  Lut lut;
+  uint32_t raw[NIB / 8];
+  float am = 0.f;
+  // packed nibbles and absmax of stage d (j = d % 4) of this thread
+  auto take = [&](int d, int j) __attribute__((always_inline)) {
+    const char* const slot = smem + S::XS + S::BS + ((d >> 2) % 3) * S::RAW;
+    const char* const q = slot + wread + 16 * (j ^ wsw);
+    if constexpr (NIB == 16) {
+      const uint2 v = *reinterpret_cast<const uint2*>(q);
+      raw[0] = v.x;
+      raw[1] = v.y;
+    } else if constexpr (NIB == 32) {
+      const uint4 v = *reinterpret_cast<const uint4*>(q);
+      raw[0] = v.x;
+      raw[1] = v.y;
+      raw[2] = v.z;
+      raw[3] = v.w;
+    } else {
+      raw[0] = *reinterpret_cast<const uint32_t*>(q);
+    }
+    if (!(j & 1)) am = *reinterpret_cast<const float*>(slot + OA + ((j >> 1) * BN + rho) * 4);
+  };
+  auto decode = [&](int d, int j) __attribute__((always_inline)) {
+    if (!(j & 1)) lut = make_lut(code, am);  // an absmax block is two stages at least
+#pragma unroll
+    for (int c = 0; c < NIB / 8; ++c) {
+      const int ch = sub * (NIB / 8) + c;
+      *reinterpret_cast<uint4*>(bw + (d & 1) * S::SB + 16 * (ch ^ ((dr >> 1) & 3))) =
+          interleave8(decode8(raw[c], lut));
+    }
+  };
+
+  // ---- prologue: superstages 0 and 1, stages 0 .. 2 of x, the first half of
+  // superstage 2 (in the order the steps before step 0 would have used)
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+#pragma unroll
+  for (int e = 0; e < S::E; ++e) fetch_raw(0, e);
+#pragma unroll
+  for (int e = 0; e < S::E; ++e) fetch_raw(1, e);
+#pragma unroll
+  for (int st = 0; st < 3; ++st) {
+#pragma unroll
+    for (int i = 0; i < S::LDA; ++i) fetch_x(st, i);
+    fetch_l(st);
+    if (st == 1) extras(2, I0{});
+    if (st == 2) extras(2, I1{});
+  }
+  constexpr int PRE = 3 * S::LDX + S::ex(0) + S::ex(1);  // loads after the raw ones
+  wait_vm<PRE + S::E>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  take(0, 0);
+  decode(0, 0);
+  take(1, 1);
+  decode(1, 1);
+
+  const int wm = wave / WN, wn = wave % WN;
+  const int off = ln * 64 + 16 * (lg ^ ((ln >> 1) & 3));
+  const char* const la = smem + wm * RM * 1024 + off;
+  const char* const lbp = smem + S::XS + wn * RN * 1024 + off;
+  f32x4_t acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int RT = RM / WN > 0 ? RM / WN : 1;  // row tiles of t per wave
+  f32x4_t tacc[LORA ? RT : 1];
+#pragma unroll
+  for (int i = 0; i < (LORA ? RT : 1); ++i) tacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  uint4 a0[RH], a1[RH], b0[RN], b1[RN], l0 = make_uint4(0, 0, 0, 0), l1 = l0;
+  auto read = [&](const char* q, auto& x) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(x) / 16); ++i)
+      x[i] = *reinterpret_cast<const uint4*>(q + i * 1024);
+  };
+  auto read_l = [&](int st, uint4& l) __attribute__((always_inline)) {
+    if (LORA)
+      l = *reinterpret_cast<const uint4*>(smem + (st & 3) * S::ST + S::TA * 1024 + off);
+  };
+  // x A^T of row tile i (static) in the wave that has it
+  auto mul_t = [&](int i, const uint4& a, const uint4& l) __attribute__((always_inline)) {
+    if (LORA && i / RT == wn) tacc[i % RT] = mfma16x16x32(l, a, tacc[i % RT]);
+  };
+  wait_vm_lds<PRE - S::LDX>();  // stage 0 of x, and this wave's decoded values
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read(lbp, b0);
+  read(la, a0);
+  read_l(0, l0);
+
+  // step st, j = (st + 2) % 4 the phase of the stage that it decodes
+  auto step = [&](int st, auto jc, uint4 (&bc)[RN], uint4& lc, uint4 (&bn)[RN], uint4& lnx)
+                  __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    take(st + 2, j);
+    read(la + (st & 3) * S::ST + RH * 1024, a1);
+#pragma unroll
+    for (int i = 0; i < RH; ++i) {
+#pragma unroll
+      for (int q = 0; q < RN; ++q) acc[i][q] = mfma16x16x32(bc[q], a0[i], acc[i][q]);
+      mul_t(i, a0[i], lc);
+    }
+    // stage st + 1 of x has landed, and every wave's LDS work is done: its reads of
+    // the slots written next, its decoded values of stage st + 1
+    wait_vm_lds<S::ex(j + 2) + S::LDX + S::ex(j + 3)>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(lbp + ((st + 1) & 1) * S::SB, bn);
+    read(la + ((st + 1) & 3) * S::ST, a0);
+    read_l(st + 1, lnx);
+    decode(st + 2, j);
+#pragma unroll
+    for (int i = 0; i < RH; ++i) {
+#pragma unroll
+      for (int q = 0; q < RN; ++q) acc[RH + i][q] = mfma16x16x32(bc[q], a1[i], acc[RH + i][q]);
+      mul_t(RH + i, a1[i], lc);
+    }
+#pragma unroll
+    for (int i = 0; i < S::LDA; ++i) fetch_x(st + 3, i);
+    fetch_l(st + 3);
+    extras(((st + 2) >> 2) + 2, jc);
+  };
+  for (int st = 0; st < nst; st += 4) {
+    step(st, I2{}, b0, l0, b1, l1);
+    step(st + 1, I3{}, b1, l1, b0, l0);
+    step(st + 2, I0{}, b0, l0, b1, l1);
+    step(st + 3, I1{}, b1, l1, b0, l0);
+  }
+  if (KS > 1 && nst < 4 * lss)  // the longer group's last four barriers
+#pragma unroll
+    for (int i = 0; i < 4; ++i) __builtin_amdgcn_s_barrier();
+  wait_vm<0>();
+  if (LORA) {  // ranks >= r, which repeat rank r - 1, must not reach a product with 0
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (4 * lg + e >= p.r) tacc[i][e] = 0.f;
+  }
+
+  // Row tiles that this wave finishes: with two K groups half of them, whose other
+  // partial sum comes through LDS from the same wave of the other group.
+  constexpr int NR = KS == 1 ? RM : RH;
+  const int rt0 = wm * RM + (KS == 1 ? 0 : grp * RH);
+  f32x4_t fin[NR][RN];
+  uint16_t* const ts = reinterpret_cast<uint16_t*>(smem0 + (KS == 1 ? 0 : S::TS));
+  if constexpr (KS == 1) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+      for (int q = 0; q < RN; ++q) fin[i][q] = acc[i][q];
+    if (LORA) __syncthreads();  // every wave is past its last read of the rings
+  } else {
+    f32x4_t* const xs = reinterpret_cast<f32x4_t*>(smem0) + lane;
+    f32x4_t* const xt = reinterpret_cast<f32x4_t*>(smem0 + S::XT) + lane;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RH; ++i)
+#pragma unroll
+      for (int q = 0; q < RN; ++q) {
+        xs[((grp * W + wave) * RH * RN + i * RN + q) * 64] = grp == 0 ? acc[RH + i][q] : acc[i][q];
+        fin[i][q] = grp == 0 ? acc[i][q] : acc[RH + i][q];
+      }
+    if (LORA)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) xt[((grp * W + wave) * RT + i) * 64] = tacc[i];
+    __syncthreads();
+    const int og = 1 - grp;
+#pragma unroll
+    for (int i = 0; i < RH; ++i)
+#pragma unroll
+      for (int q = 0; q < RN; ++q) fin[i][q] += xs[((og * W + wave) * RH * RN + i * RN + q) * 64];
+    if (LORA)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) tacc[i] += xt[((og * W + wave) * RT + i) * 64];
+  }
+
+  const int nl = n0 + wn * 16 * RN + 4 * RN * lg;  // this lane's first column
+  if constexpr (MODE == K2_PART) {
+    float* const pp = p.part + blockIdx.y * p.psl + c0;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int m = m0 + (rt0 + i) * 16 + ln;
+      if (m >= p.M) continue;
+#pragma unroll
+      for (int q = 0; q < RN; ++q)
+        if (nl + 4 * q < N)  // N % 16 == 0
+          *reinterpret_cast<float4*>(pp + (int64_t)m * p.ldp + nl + 4 * q) =
+              make_float4(fin[i][q][0], fin[i][q][1], fin[i][q][2], fin[i][q][3]);
+    }
+    if (LORA && lt == 0 && grp == 0) {
+      float* const tp = p.tpart + blockIdx.y * p.tsl + seg * p.tseg;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const int m = m0 + (wm * RM + wn * RT + i) * 16 + ln;
+        if (wn * RT + i < RM && m < p.M)
+          *reinterpret_cast<float4*>(tp + (int64_t)m * 16 + 4 * lg) =
+              make_float4(tacc[i][0], tacc[i][1], tacc[i][2], tacc[i][3]);
+      }
+    }
+  } else if constexpr (SILU) {
+    const int a = n0 + 32 * wn + 8 * lg;  // act columns a .. a + 7
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int m = m0 + (rt0 + i) * 16 + ln;
+      uint32_t o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float r2[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int e = 2 * q + h;
+          const float gv = round_bf(fin[i][e >> 2][e & 3]);
+          const float uv = round_bf(fin[i][2 + (e >> 2)][e & 3]);
+          r2[h] = round_bf(gv * (1.f / (1.f + expf(-gv)))) * uv;  // as silu_mul_kernel
+        }
+        o[q] = pack_bf2(r2[0], r2[1]);
+      }
+      if (m < p.M && a < p.silu_I) {  // I % 8 == 0
+        uint16_t* const d = p.y + (int64_t)m * p.ldy + a;
+        if (p.yvec) {
+          *reinterpret_cast<uint4*>(d) = make_uint4(o[0], o[1], o[2], o[3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) d[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    }
+  } else {
+    uint4 low[RN];
+    if (LORA) {
+      // t [BM][32], ranks >= 16 zero
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        if (grp == 0 && wn * RT + i < RM) {
+          uint16_t* d = ts + ((wm * RM + wn * RT + i) * 16 + ln) * 32 + 4 * lg;
+          *reinterpret_cast<uint2*>(d) = make_uint2(pack_bf2(tacc[i][0], tacc[i][1]),
+                                                    pack_bf2(tacc[i][2], tacc[i][3]));
+          *reinterpret_cast<uint2*>(d + 16) = make_uint2(0, 0);
+        }
+#pragma unroll
+      for (int q = 0; q < RN; ++q) {
+        const int col = min(n0 + wn * 16 * RN + 4 * RN * (ln >> 2) + 4 * q + (ln & 3), N - 1);
+        const uint16_t* br = slb + (int64_t)col * p.r;
+        low[q] = make_uint4(0, 0, 0, 0);
+        if (p.lbvec) {
+          if (8 * lg < p.r) low[q] = *reinterpret_cast<const uint4*>(br + 8 * lg);
+        } else {
+          uint32_t v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = 8 * lg + e < p.r ? br[8 * lg + e] : 0u;
+          low[q] = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16),
+                              v[6] | (v[7] << 16));
+        }
+      }
+      __syncthreads();
+    }
+    float bias[4 * RN];
+    if (sbias) {
+#pragma unroll
+      for (int e = 0; e < 4 * RN; ++e) bias[e] = bf2f(sbias[min(nl + e, N - 1)]);
+    }
+    const float sc = round_bf(p.scaling);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int row = (rt0 + i) * 16 + ln, m = m0 + row;
+      uint4 tv;
+      if (LORA) tv = *reinterpret_cast<const uint4*>(ts + row * 32 + 8 * lg);
+      uint32_t o[2 * RN];
+#pragma unroll
+      for (int q = 0; q < RN; ++q) {
+        f32x4_t u{0.f, 0.f, 0.f, 0.f};
+        if (LORA) u = mfma16x16x32(low[q], tv, u);
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = round_bf(fin[i][q][e]);
+          if (sbias) v[e] = round_bf(v[e] + bias[4 * q + e]);
+          if (LORA) v[e] = round_bf(v[e] + round_bf(round_bf(u[e]) * sc));
+        }
+        o[2 * q] = pack_bf2(v[0], v[1]);
+        o[2 * q + 1] = pack_bf2(v[2], v[3]);
+      }
+      if (m < p.M) {
+        uint16_t* const d = p.y + (int64_t)m * p.ldy + c0 + nl;
+        if (p.yvec) {  // segment ends % 8 == 0
+#pragma unroll
+          for (int h = 0; h < RN / 2; ++h)
+            if (nl + 8 * h < N)
+              *reinterpret_cast<uint4*>(d + 8 * h) =
+                  make_uint4(o[4 * h], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4 * RN; ++e)
+            if (nl + e < N) d[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    }
+  }
+}
+
+// Tiles of nf4_gemm_k2 (ks K groups) and their time model in us, fitted to 430 measured
+// shapes of 128 .. 2048 rows (r.m.s. error 6 %; the tile it picks is within 7 % of the
+// best one measured, and within 2 % in 40 of 45 shapes): a round of workgroups costs
+// `fixed` and, per step, `step` alone on a CU, `more` for each further one that fits
+// (occ, occ_l with LoRA), `lora` with LoRA.
+struct K2Tile {
+  int bm, bn, ks, occ, occ_l;
+  double fixed, step, more, lora;
+};
+constexpr K2Tile K2_TILE[] = {{256, 256, 1, 1, 1, 10.2, 0.75, 0.0, 0.0},
+                              {128, 128, 1, 2, 2, 3.9, 0.38, 0.21, 0.06},
+                              {64, 128, 2, 1, 1, 3.4, 0.47, 0.0, 0.02},
+                              {64, 64, 2, 2, 1, 1.8, 0.32, 0.22, 0.04},
+                              {128, 128, 2, 1, 1, 5.1, 0.58, 0.0, 0.05}};
+// Which tiles a form is built for.
+constexpr bool k2_has(int tile, K2Mode mode, bool lora) {
+  return tile == 0 ? !lora && mode != K2_PART : (mode != K2_SILU || tile == 1 || tile == 4);
+}
+
+// The tile for the segments' columns (SILU: I columns of half a tile each) in S K
+// slices of kss superstages, and its time in us. A split also writes float32 partial
+// sums, reads them back and launches the finish (3.2 us; 1.4 us per million sums, with
+// LoRA 3.3 us per million outputs).
+int k2_tile(int M, int nseg, const int* seg_end, int kss, int S, bool lora, K2Mode mode,
+            double* us) {
+  int best = -1;
+  for (int i = 0; i < 5; ++i) {
+    if (!k2_has(i, mode, lora)) continue;
+    const K2Tile& c = K2_TILE[i];
+    int64_t nt = 0;
+    for (int s = 0, start = 0; s < nseg; start = seg_end[s], ++s)
+      nt += cdiv(seg_end[s] - start, mode == K2_SILU ? c.bn / 2 : c.bn);
+    const int64_t tiles = cdiv(M, c.bm) * nt * S;
+    const int occ = lora ? c.occ_l : c.occ;
+    auto round = [&](int64_t per_cu) {
+      return c.fixed + 4 * (double)cdiv(kss, c.ks) *
+                           (c.step + (lora ? c.lora : 0.0) + (double)(per_cu - 1) * c.more);
+    };
+    const int64_t full = tiles / (256 * occ), rem = tiles % (256 * occ);
+    double t = 3.5 + (double)full * round(occ) + (rem ? round(cdiv(rem, 256)) : 0.0);
+    if (S > 1) {
+      const double outs = (double)M * seg_end[nseg - 1];
+      t += 3.2 + outs * (S * 1.4e-6 + (lora ? 3.3e-6 : 0.0));
+    }
+    if (best < 0 || t < *us) best = i, *us = t;
+  }
+  return best;
+}
+
+bool k2_shape(int K, int r, int64_t wrows, int blocksize) {
+  return K % 128 == 0 && r <= 16 && blocksize >= 64 && wrows * K < (1ll << 32);
+}
+
+template <K2Mode MODE, bool LORA, int RM, int RN, int WM, int WN, int KS>
+int k2_go(const K2Args& a, unsigned slices, hipStream_t st) {
+  using S = K2Shape<MODE, LORA, RM, RN, WM, WN, KS>;
+  static_assert(KS * S::LDS <= 160 * 1024, "LDS");
+  constexpr auto kern = nf4_gemm_k2<MODE, LORA, RM, RN, WM, WN, KS>;
+  if (int rc = allow_dynamic_lds<kern, KS * S::LDS>()) return rc;
+  kern<<<dim3(8u * (unsigned)cdiv((int64_t)a.MT * a.NT, 8), slices), KS * S::T, KS * S::LDS,
+         st>>>(a);
+  return launch_check("nf4_gemm_k2");
+}
+
+template <K2Mode MODE, bool LORA>
+int k2_pick(const K2Args& a, int tile, unsigned slices, hipStream_t st) {
+  if constexpr (k2_has(0, MODE, LORA))
+    if (tile == 0) return k2_go<MODE, LORA, 8, 4, 2, 4, 1>(a, slices, st);
+  if constexpr (k2_has(2, MODE, LORA))
+    if (tile == 2) return k2_go<MODE, LORA, 2, 4, 2, 2, 2>(a, slices, st);
+  if constexpr (k2_has(3, MODE, LORA))
+    if (tile == 3) return k2_go<MODE, LORA, 2, 2, 2, 2, 2>(a, slices, st);
+  if (tile == 4) return k2_go<MODE, LORA, 4, 4, 2, 2, 2>(a, slices, st);
+  return k2_go<MODE, LORA, 4, 4, 2, 2, 1>(a, slices, st);
+}
+
 bool pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 
 
@@ -486,7 +1047,7 @@ bool nf4_gemm_ok(int M, int N, int K, int r, int blocksize) {
   return gemm_ok(M, N, K, r, blocksize);
 }
 
-GemmPlan nf4_gemm_plan(int M, int K, int r, int nseg, const int* seg_end) {
+GemmPlan nf4_gemm_plan(int M, int K, int r, int blocksize, int nseg, const int* seg_end) {
   const int nst = (int)cdiv(K, GM_KS);
   GemmPlan pl{1, nst, 0, 0};
   const int64_t mt = cdiv(M, GM_BM);
@@ -497,12 +1058,32 @@ GemmPlan nf4_gemm_plan(int M, int K, int r, int nseg, const int* seg_end) {
     split_ok = split_ok && seg_end[s] % 16 == 0;
   }
   if (!split_ok || nst < 6) return pl;
+  const int N = seg_end[nseg - 1];
+  if (k2_shape(K, r, N, blocksize)) {
+    // The ring kernel (nf4_gemm_k2): the slice count of the least estimated time, of one
+    // N-column segment, so that a size query without the segments gives the same.
+    double best = 0.0;
+    for (int S = 1; S <= std::min(MAX_SLICES, nst / 3); ++S) {
+      const int kst = (int)cdiv(nst, S), slices = (int)cdiv(nst, kst);
+      double t = 0.0;
+      k2_tile(M, 1, &N, kst, slices, r > 0, slices > 1 ? K2_PART : K2_OUT, &t);
+      if (S == 1 || t < best) {
+        best = t;
+        pl.S = slices;
+        pl.kst = kst;
+      }
+    }
+    if (pl.S > 1) {
+      pl.part_bytes = (size_t)pl.S * M * N * 4;
+      pl.tpart_bytes = r > 0 ? (size_t)pl.S * nseg * M * 16 * 4 : 0;
+    }
+    return pl;
+  }
   // Time model (us) of S K slices, from measurements on MI355X: a workgroup
   // stage (128 K values) takes about 2.2 us whatever the tile count (its loads'
   // latency), 512 workgroups run at once; a split adds the float32 partial
   // sums (written and read back, ~4 TB/s), the finish launch and, with LoRA,
   // the finish's per-output rank sums (~2 ns per 1000 outputs).
-  const int N = seg_end[nseg - 1];
   const double outs = (double)M * N;
   auto est = [&](int S, int* kst, int* slices) {
     *kst = (int)cdiv(nst, S);
@@ -605,6 +1186,50 @@ int nf4_gemm_launch(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t wr
     a.tsl = split->tsl;
     a.tseg = split->tseg;
   }
+  if (!f16 && wrow0 == 0 && k2_shape(K, r, N, blocksize) && ldx < (1 << 22)) {
+    K2Args k{};
+    k.x = x;
+    k.ldx = ldx;
+    k.w = w;
+    k.absmax = absmax;
+    k.code16 = code16;
+    k.bs_shift = a.bs_shift;
+    k.nseg = sg.nseg;
+    k.r = r;
+    k.scaling = scaling;
+    k.y = y;
+    k.ldy = ldy;
+    k.M = M;
+    k.K = K;
+    k.nss = a.nst;
+    k.kst = a.kst;
+    k.lbvec = a.lbvec;
+    k.yvec = a.yvec;
+    k.part = a.part;
+    k.ldp = a.ldp;
+    k.psl = a.psl;
+    k.tpart = a.tpart;
+    k.tsl = a.tsl;
+    k.tseg = a.tseg;
+    double us = 0.0;
+    const int tile = k2_tile(M, sg.nseg, sg.seg_end, k.kst, (int)slices, r > 0,
+                             slices > 1 ? K2_PART : K2_OUT, &us);
+    k.MT = (int)cdiv(M, K2_TILE[tile].bm);
+    for (int s = 0; s < MAXSEG; ++s) {
+      k.seg_end[s] = a.seg_end[s];
+      k.bias[s] = a.bias[s];
+      k.la[s] = a.la[s];
+      k.lb[s] = a.lb[s];
+      k.seg_tile[s] = k.NT;
+      if (s < sg.nseg)
+        k.NT += (int)cdiv(sg.seg_end[s] - (s > 0 ? sg.seg_end[s - 1] : 0), K2_TILE[tile].bn);
+    }
+    for (int s = sg.nseg; s <= MAXSEG; ++s) k.seg_tile[s] = k.NT;
+    if (slices > 1)
+      return r > 0 ? k2_pick<K2_PART, true>(k, tile, slices, st)
+                   : k2_pick<K2_PART, false>(k, tile, slices, st);
+    return r > 0 ? k2_pick<K2_OUT, true>(k, tile, 1, st) : k2_pick<K2_OUT, false>(k, tile, 1, st);
+  }
   const dim3 grid(8u * (unsigned)cdiv((int64_t)a.MT * a.NT, 8), slices);
   const int tc = r > 16 ? 2 : (r > 0 ? 1 : 0);
   int rc = GRPO_OK;
@@ -675,6 +1300,33 @@ int nf4_gemm_silu_launch(const uint16_t* x, int64_t ldx, const uint8_t* w, const
   a.yvec = aligned16(act) && lda % 8 == 0;
   a.nst = a.kst = (int)cdiv(K, GM_KS);
   a.silu_I = I;
+  if (k2_shape(K, 0, 2 * (int64_t)I, blocksize) && ldx < (1 << 22)) {
+    K2Args k{};
+    k.x = x;
+    k.ldx = ldx;
+    k.w = w;
+    k.absmax = absmax;
+    k.code16 = code16;
+    k.bs_shift = a.bs_shift;
+    k.nseg = 1;
+    k.y = act;
+    k.ldy = lda;
+    k.M = M;
+    k.K = K;
+    k.nss = k.kst = a.nst;
+    k.silu_I = I;
+    k.yvec = a.yvec;
+    double us = 0.0;
+    const int tile = k2_tile(M, 1, &I, k.nss, 1, false, K2_SILU, &us);
+    k.MT = (int)cdiv(M, K2_TILE[tile].bm);
+    k.NT = (int)cdiv(I, K2_TILE[tile].bn / 2);
+    for (int s = 0; s < MAXSEG; ++s) {
+      k.seg_end[s] = 2 * I;
+      k.seg_tile[s] = s == 0 ? 0 : k.NT;
+    }
+    k.seg_tile[MAXSEG] = k.NT;
+    return k2_pick<K2_SILU, false>(k, tile, 1, st);
+  }
   const dim3 grid(8u * (unsigned)cdiv((int64_t)a.MT * a.NT, 8));
   constexpr auto kern = nf4_gemm_mfma<0, false, true>;
   if (int rc = allow_dynamic_lds<kern, (int)GM_LDS>()) return rc;

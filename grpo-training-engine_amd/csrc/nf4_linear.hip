@@ -1958,7 +1958,7 @@ int run_linear(const GenArgs& g, void* workspace, size_t workspace_bytes, hipStr
     // Few tiles and a long K: the K slices write float32 partial sums (LinParts
     // layout over all segments) and nf4_finish applies the epilogue.
     // A workspace smaller than the plan's partial sums runs the linear unsplit.
-    GemmPlan pl = nf4_gemm_plan(g.M, g.K, g.r, g.nseg, g.seg_end);
+    GemmPlan pl = nf4_gemm_plan(g.M, g.K, g.r, g.blocksize, g.nseg, g.seg_end);
     if (pl.S > 1 && (!workspace || workspace_bytes < align256(pl.part_bytes) + pl.tpart_bytes))
       pl.S = 1;
     GemmSplit sp{};
@@ -2018,10 +2018,10 @@ size_t workspace_bytes_for(int M, int N, int K, int r, int nseg, int blocksize,
     if (seg_end) {
       for (int s = 0, start = 0; s < nseg; start = seg_end[s], ++s)
         if (!nf4_gemm_ok(M, seg_end[s] - start, K, r, blocksize)) return 0;
-      pl = nf4_gemm_plan(M, K, r, nseg, seg_end);
+      pl = nf4_gemm_plan(M, K, r, blocksize, nseg, seg_end);
     } else {
       if (!nf4_gemm_ok(M, N, K, r, blocksize)) return 0;
-      pl = nf4_gemm_plan(M, K, r, 1, &N);
+      pl = nf4_gemm_plan(M, K, r, blocksize, 1, &N);
       pl.tpart_bytes = r > 0 ? (size_t)pl.S * nseg * M * 16 * 4 : 0;
     }
     return pl.S > 1 ? align256(pl.part_bytes) + pl.tpart_bytes : 0;

@@ -27,7 +27,7 @@
 // 28.0 for the decode kernel and its merge; after 2000 tokens 33 us.
 #include <algorithm>
 
-#include "common.hpp"
+#include "lds_dma.hpp"
 
 using namespace grpo;
 
@@ -52,12 +52,6 @@ struct PrefillArgs {
   float scale;
 };
 
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds),
-               "v"(voff), "s"(base)
-               : "memory");
-}
-
 // Largest value of each row of 16 lanes, of the first row for the whole wave (the
 // rows hold the same values): DPP moves, no LDS round trips.
 __device__ __forceinline__ int max16(int v) {
@@ -68,11 +62,6 @@ __device__ __forceinline__ int max16(int v) {
   STEP_MAX(0x140);  // row_mirror
 #undef STEP_MAX
   return __builtin_amdgcn_readfirstlane(v);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
 __device__ __forceinline__ uint32_t word(const uint4& v, int i) {
@@ -118,7 +107,7 @@ __global__ void __launch_bounds__(64 * CS * HW) prefill_attn_kernel(PrefillArgs 
   const int most = max16(len), least = -max16(m < p.M ? -len : -cap);
   const int nblk = (most + PBS - 1) / PBS, nstep = (most + STEP - 1) / STEP;
   const int row4 = lane >> 4, slot = lane & 15;
-  const uint32_t lbase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const uint32_t lbase = lds_address(lds);
   // Piece pc of a step: tokens 4 (pc % 8) .. + 3 of K (pc / 8 even) or V of part pc / 16.
   // Blocks past the rows' contexts read the last one (its tokens are masked).
   uint32_t voff[LD];
