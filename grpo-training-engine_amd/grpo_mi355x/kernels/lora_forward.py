@@ -14,7 +14,7 @@ Same call surface and dispatch as the reference's
 
 The fused forward is ``grpo_nf4_lora_linear`` for few rows (the weight decoded
 as it is multiplied: the split-K kernel up to 64 rows, the NF4 GEMM beyond) and
-``grpo_nf4_lora_train_forward`` from ``train_min_rows`` on (the weight brought to
+``grpo_nf4_lora_train_forward`` where ``train_forward_pays`` (the weight brought to
 16 bits in the call, then an MFMA GEMM with the epilogue in it).  float16 x
 with float16 adapters (the reference's float16 X_DTYPE / LORA_DTYPE, ``:141-143,
 745-749``) has every rounding point float16; mixed dtypes raise ``ValueError``
@@ -144,19 +144,23 @@ def fused_forward_rows(k: int) -> int:
     return 4096 if k <= 4096 else 1024
 
 
-def train_min_rows(k: int, dtype: torch.dtype) -> int:
-    """Rows from which the forward runs the training linear (the weight brought
-    to 16 bits in the call, then an MFMA GEMM) rather than the kernels that decode
-    the weight as they multiply.  Measured on MI355X (us, those against this,
-    N x K, r = 16, bf16): 1536 x 1536 19.4 / 19.0 at 256 rows, 24.2 / 19.2 at 512,
-    52.4 / 39.7 at 4096; 3584 x 3584 33.3 / 42.6, 45.8 / 45.4, 194.5 / 109.7;
-    8960 x 1536 35.2 / 36.4, 48.6 / 44.5, 218.5 / 148.5; a long K with few column
-    tiles later, 1536 x 8960 74.0 / 89.1 at 1024 rows, 136.6 / 106.3 at 2048.  In
-    float16 the decoding kernel does not split K: 32.9 / 17.2 (1536 x 1536) and
+def train_forward_pays(m: int, n: int, k: int, r: int, blocksize: int,
+                       dtype: torch.dtype) -> bool:
+    """Whether the forward runs the training linear (the weight brought to 16 bits in
+    the call, then an MFMA GEMM) rather than the kernels that decode the weight as they
+    multiply.  Decoding costs the NF4 GEMM a share of every tile, so what counts is M N.
+    Measured on MI355X (us, those against this, N x K at M rows, r = 16, bf16, the NF4
+    GEMM's ring kernel): 1536 x 1536 26.5 / 30.4 at 2048, 44.9 / 38.8 at 4096; 3584 x
+    3584 49.2 / 52.3 at 1024, 91.4 / 79.8 at 2048; 8960 x 1536 41.7 / 45.1 at 512, 65.2 /
+    54.8 at 1024; 256 x 1536 15.5 / 19.1 at 4096.  Shapes its older kernel takes cross
+    earlier: 24.2 / 19.2 at 512 rows of 1536 x 1536, 136.6 / 106.3 at 2048 of 1536 x
+    8960.  In float16 the decoding kernel does not split K: 32.9 / 17.2 (1536 x 1536) and
     33.2 / 30.1 (8960 x 1536) at 16 rows."""
     if dtype == torch.float16:
-        return 1
-    return 512 if k <= 4096 else 1536
+        return True
+    if k % 128 == 0 and r <= 16 and blocksize >= 64 and m <= fused_forward_rows(k):
+        return m * n >= 5_000_000
+    return m >= (512 if k <= 4096 else 1024)
 
 
 def _train_workspace(w: torch.Tensor, blocksize: int, lora_A: torch.Tensor,
@@ -200,7 +204,7 @@ def _run_forward(x, weight_4bit, quant_state, lora_A, lora_B, scaling, bias):
     if bias is not None and (not bias.is_cuda or bias.numel() != n):
         raise ValueError(f"bias must have {n} elements on the ROCm/HIP device.")
     nbytes = (_train_workspace(w, blocksize, lora_A, lora_B, x_flat)
-              if m >= train_min_rows(k, dt) else 0)
+              if train_forward_pays(m, n, k, r, blocksize, dt) else 0)
     if nbytes:
         if bias is not None and (bias.dtype != dt or not bias.is_contiguous()):
             bias = bias.to(dt).contiguous()
