@@ -55,7 +55,6 @@ constexpr size_t SMP_LDS = (size_t)SMP_KEYS * 4;
 constexpr float EXP_MIN_X = -86.0f;
 constexpr int SMP_U = 8;  // 16-byte group loads in flight per thread in the row passes
 constexpr int SMP_CMAX = SMP_KEYS / 2;                // entries of the compacted bins
-constexpr int SMP_EPT = (SMP_CMAX + SMP_T - 1) / SMP_T;  // entries per thread at most
 static_assert(SMP_KEYS % SMP_T == 0 && SMP_KEYS % 4 == 0, "bins must split evenly");
 
 // Per-row workspace.
@@ -141,68 +140,86 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+// v of the lane that DPP control CTRL names, 0 where it names none.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ uint64_t dpp0(uint64_t v) {
+  return dpp0<CTRL>((uint32_t)v) | ((uint64_t)dpp0<CTRL>((uint32_t)(v >> 32)) << 32);
+}
+// Inclusive prefix over each row of 16 lanes, and over the wave: shifts by 1, 2, 4, 8
+// within the rows, then lane 15 of rows 0 and 2 to the rows after them, then lane 31 to
+// the upper half.
+template <typename T, typename F>
+__device__ __forceinline__ T row_prefix(T v, F&& op) {
+  v = op(v, dpp0<0x111>(v));
+  v = op(v, dpp0<0x112>(v));
+  v = op(v, dpp0<0x114>(v));
+  return op(v, dpp0<0x118>(v));
+}
+template <typename T, typename F>
+__device__ __forceinline__ T wave_prefix(T v, F&& op) {
+  v = row_prefix(v, op);
+  const T below = dpp0<0x142>(v);
+  v = op(v, (threadIdx.x & 16) ? below : 0);
+  const T half = dpp0<0x143>(v);
+  return op(v, (threadIdx.x & 32) ? half : 0);
+}
+struct Add {
+  template <typename T>
+  __device__ __forceinline__ T operator()(T a, T b) const { return a + b; }
+};
+struct Max {
+  __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return max(a, b); }
+};
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int lane) {
+  return lane_value((uint32_t)v, lane) | ((uint64_t)lane_value((uint32_t)(v >> 32), lane) << 32);
 }
 
-// Block-wide sum / max over NW waves through one LDS slot per wave.  Every
+// Block-wide sum / max over NW <= 16 waves through one LDS slot per wave.  Every
 // thread gets the result; the trailing barrier lets the slots be reused.
+template <int NW, typename T, typename F>
+__device__ __forceinline__ T block_reduce(T v, T* slots, F&& op) {
+  const int lane = threadIdx.x & 63;
+  v = wave_prefix(v, op);
+  if (lane == 63) slots[threadIdx.x >> 6] = v;
+  __syncthreads();
+  const T s = lane < NW ? slots[lane] : 0;
+  __syncthreads();
+  return lane_value(row_prefix(s, op), 15);
+}
 template <int NW, typename T>
 __device__ __forceinline__ T block_sum(T v, T* slots) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) slots[threadIdx.x >> 6] = v;
-  __syncthreads();
-  T s = 0;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) s += slots[w];
-  __syncthreads();
-  return s;
+  return block_reduce<NW>(v, slots, Add());
 }
 template <int NW>
 __device__ __forceinline__ uint32_t block_max(uint32_t v, uint32_t* slots) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor(v, o));
-  if ((threadIdx.x & 63) == 0) slots[threadIdx.x >> 6] = v;
-  __syncthreads();
-  uint32_t s = 0;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) s = max(s, slots[w]);
-  __syncthreads();
-  return s;
+  return block_reduce<NW>(v, slots, Max());
 }
 
-// Exclusive prefix over the block (thread order) of a (u64, u32) pair.
+// Exclusive prefix over a block of SMP_T threads (thread order) of a (u64, u32) pair.
+static_assert(SMP_T == 1024, "sixteen waves: one row of lanes scans their sums");
 __device__ __forceinline__ void block_excl_scan(uint64_t& a, uint32_t& b, uint64_t* sa,
                                                 uint32_t* sb) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint64_t ia = a;
-  uint32_t ib = b;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint64_t ta = __shfl_up(ia, o);
-    const uint32_t tb = __shfl_up(ib, o);
-    if (lane >= o) {
-      ia += ta;
-      ib += tb;
-    }
-  }
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint64_t ia = wave_prefix(a, Add());
+  const uint32_t ib = wave_prefix(b, Add());
   if (lane == 63) {
     sa[wave] = ia;
     sb[wave] = ib;
   }
   __syncthreads();
-  uint64_t pa = 0;
-  uint32_t pb = 0;
-  for (int w = 0; w < wave; ++w) {
-    pa += sa[w];
-    pb += sb[w];
-  }
+  const uint64_t va = row_prefix(sa[lane & 15], Add());
+  const uint32_t vb = row_prefix(sb[lane & 15], Add());
   __syncthreads();
-  a = pa + ia - a;
-  b = pb + ib - b;
+  a = ia - a + (wave ? lane_value(va, wave - 1) : 0);
+  b = ib - b + (wave ? lane_value(vb, wave - 1) : 0);
 }
 
 // Calls f(group index, its 16 bytes) for the groups first, first + stride, ...
@@ -235,10 +252,11 @@ __device__ __forceinline__ void keys_of(const uint4& v, float inv_t, uint32_t (&
 __device__ __forceinline__ bool row_stopped(const SampleArgs& a, int m) {
   return a.tokens != nullptr && !a.active[m];
 }
+// (One load per lane: a loop over the slices waits for each, 4 us for 32 of them.)
+static_assert(SMP_SMAX <= 64, "a lane per slice");
 __device__ __forceinline__ uint32_t row_max_key(const SampleArgs& a, const RowWs& w) {
-  uint32_t k = 0;
-  for (int i = 0; i < a.S; ++i) k = max(k, w.slice_max[i]);
-  return k;
+  const int lane = threadIdx.x & 63;
+  return lane_value(wave_prefix(lane < a.S ? w.slice_max[lane] : 0u, Max()), 63);
 }
 
 // K0: the slice's maximum key.
@@ -338,6 +356,10 @@ __device__ __forceinline__ uint64_t prob62(uint32_t w) {
 // taking bins t, t + 1024, ... (the populated bins cluster near the top of the
 // window); the ordered prefixes run over contiguous ranges, thread t taking
 // bins [34t, 34t + 34).  Everything after the first read lives in LDS.
+// Bound by latency on one CU per row: e is computed again in each pass, in rolled loops
+// (kept in registers over unrolled ones it spilled and ran 17000 lines of code once).
+// 8 rows x 151936: 19.9 -> 15.9 us, the five launches 44.0 -> 34.6 with prefixes by DPP
+// and the per-slice results read a lane each.
 __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
   touch_kernargs<sizeof(SampleArgs)>();
   extern __shared__ uint32_t lds[];  // [SMP_KEYS] packed (count, p or q) words
@@ -412,34 +434,24 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
           }
       }
       __syncthreads();
-      const uint32_t ept = (N + SMP_T - 1) / SMP_T;  // entries per thread (<= SMP_EPT)
-      const uint32_t k0 = tid * ept;
-      float ev[SMP_EPT];
+      const uint32_t ept = (N + SMP_T - 1) / SMP_T;  // entries per thread
+      const uint32_t k0 = tid * ept, k1 = min(N, k0 + ept);
       // A: e per entry, Z
       fresh();
       uint64_t zc = 0;
-#pragma unroll
-      for (int i = 0; i < SMP_EPT; ++i) {
-        const uint32_t k = k0 + i;
-        ev[i] = 0.0f;
-        if (i < (int)ept && k < N) {
-          ev[i] = e_of(cbin[k]);
-          zc += (uint64_t)ccnt[k] * to_fixed(ev[i], TWO44);
-        }
-      }
+#pragma unroll 1
+      for (uint32_t k = k0; k < k1; ++k)
+        zc += (uint64_t)ccnt[k] * to_fixed(e_of(cbin[k]), TWO44);
       const float zcf = (float)block_sum<SMP_T / 64>(zc, s64) * TWO_M44;
       // B, C: p per entry; running sum in sorted order; the cut (as an entry index)
       uint64_t mass = 0;
       uint32_t ntok = 0;
-#pragma unroll
-      for (int i = 0; i < SMP_EPT; ++i) {
-        const uint32_t k = k0 + i;
-        if (i < (int)ept && k < N) {
-          const uint16_t pb = f2bf(ev[i] / zcf);
-          cprob[k] = pb;
-          mass += (uint64_t)ccnt[k] * to_fixed(bf2f(pb), TWO62);
-          ntok += ccnt[k];
-        }
+#pragma unroll 1
+      for (uint32_t k = k0; k < k1; ++k) {
+        const uint16_t pb = f2bf(e_of(cbin[k]) / zcf);
+        cprob[k] = pb;
+        mass += (uint64_t)ccnt[k] * to_fixed(bf2f(pb), TWO62);
+        ntok += ccnt[k];
       }
       uint64_t cum = mass;
       uint32_t above = ntok;
@@ -458,7 +470,7 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
             s_cut[2] = 0;
           }
         } else if ((int64_t)cum <= a.keep && (int64_t)(cum + mass) > a.keep) {
-          for (uint32_t k = k0; k < min(N, k0 + ept); ++k) {  // this thread holds the crossing
+          for (uint32_t k = k0; k < k1; ++k) {  // this thread holds the crossing
             const uint32_t ck = ccnt[k];
             const uint64_t pk = to_fixed(bf2f(cprob[k]), TWO62);
             const uint64_t end = cum + (uint64_t)ck * pk;
@@ -483,23 +495,17 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
       };
       // D: Z' over the kept entries
       uint64_t zkc = 0;
-#pragma unroll
-      for (int i = 0; i < SMP_EPT; ++i) {
-        const uint32_t k = k0 + i;
-        if (i < (int)ept && k < N) zkc += kept_e(k) * to_fixed(ev[i], TWO44);
-      }
+#pragma unroll 1
+      for (uint32_t k = k0; k < k1; ++k) zkc += kept_e(k) * to_fixed(e_of(cbin[k]), TWO44);
       const float zkcf = (float)block_sum<SMP_T / 64>(zkc, s64) * TWO_M44;
       // E, F: q per kept entry; kept mass in sorted order; W; the draw
       uint64_t w = 0;
-#pragma unroll
-      for (int i = 0; i < SMP_EPT; ++i) {
-        const uint32_t k = k0 + i;
-        if (i < (int)ept && k < N) {
-          const uint64_t n = kept_e(k);
-          const uint16_t qb = n ? f2bf(ev[i] / zkcf) : (uint16_t)0;
-          cprob[k] = qb;
-          w += n * to_fixed(bf2f(qb), TWO62);
-        }
+#pragma unroll 1
+      for (uint32_t k = k0; k < k1; ++k) {
+        const uint64_t n = kept_e(k);
+        const uint16_t qb = n ? f2bf(e_of(cbin[k]) / zkcf) : (uint16_t)0;
+        cprob[k] = qb;
+        w += n * to_fixed(bf2f(qb), TWO62);
       }
       uint64_t wpre = w;
       block_excl_scan(wpre, unused, s64, s32);
@@ -516,7 +522,7 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
       const uint64_t t = __umul64hi(r, W);
       if (t >= wpre && t < wpre + w) {  // t lies in this thread's entries
         uint64_t acc = wpre;
-        for (uint32_t k = k0; k < min(N, k0 + ept); ++k) {
+        for (uint32_t k = k0; k < k1; ++k) {
           const uint64_t n = kept_e(k);
           if (!n) continue;
           const uint64_t q62 = to_fixed(bf2f(cprob[k]), TWO62);
@@ -541,22 +547,20 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
   // A (balanced): Z = sum count * e over the bins (2^-44 units)
   uint64_t z = 0;
   fresh();
-#pragma unroll
+#pragma unroll 2
   for (int j = 0; j < SMP_KPT; ++j) {
     const int bin = tid + j * SMP_T;
     const uint32_t c = lds[bin];
     if (c) z += (uint64_t)c * to_fixed(e_of(bin), TWO44);
-    if (j & 1) __builtin_amdgcn_sched_barrier(0);  // two exp chains at a time
   }
   const float zf = (float)block_sum<SMP_T / 64>(z, s64) * TWO_M44;
   // B (balanced): p = bf16(e / Z) packed beside the count
   fresh();
-#pragma unroll
+#pragma unroll 2
   for (int j = 0; j < SMP_KPT; ++j) {
     const int bin = tid + j * SMP_T;
     const uint32_t c = lds[bin];
     if (c) lds[bin] = c | ((uint32_t)f2bf(e_of(bin) / zf) << 18);
-    if (j & 1) __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
   // C (contiguous): running sum of p in sorted order; the cut
@@ -564,12 +568,11 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
   {
     uint64_t mass = 0;
     uint32_t ntok = 0;
-#pragma unroll
+#pragma unroll 2
     for (int j = 0; j < SMP_KPT; ++j) {
       const uint32_t w = lds[b0 + j];
       mass += (uint64_t)cnt_of(w) * prob62(w);
       ntok += cnt_of(w);
-      if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
     }
     uint64_t cum = mass;
     uint32_t above = ntok;
@@ -614,33 +617,30 @@ __global__ void __launch_bounds__(SMP_T) smp_scan_kernel(SampleArgs a) {
   // D (balanced): Z' = sum kept * e
   uint64_t zk = 0;
   fresh();
-#pragma unroll
+#pragma unroll 2
   for (int j = 0; j < SMP_KPT; ++j) {
     const int bin = tid + j * SMP_T;
     const uint64_t n = kept((uint32_t)bin, cnt_of(lds[bin]));
     if (n) zk += n * to_fixed(e_of(bin), TWO44);
-    if (j & 1) __builtin_amdgcn_sched_barrier(0);
   }
   const float zkf = (float)block_sum<SMP_T / 64>(zk, s64) * TWO_M44;
   // E (balanced): q = bf16(e / Z') of the kept bins in place of p (0 elsewhere)
   fresh();
-#pragma unroll
+#pragma unroll 2
   for (int j = 0; j < SMP_KPT; ++j) {
     const int bin = tid + j * SMP_T;
     const uint32_t c = cnt_of(lds[bin]);
     const uint32_t qb = kept((uint32_t)bin, c) ? f2bf(e_of(bin) / zkf) : 0u;
     lds[bin] = c | (qb << 18);
-    if (j & 1) __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
   // F (contiguous): the kept mass in sorted order, W, and the draw
   {
     uint64_t w = 0;
-#pragma unroll
+#pragma unroll 2
     for (int j = 0; j < SMP_KPT; ++j) {
       const uint32_t v = lds[b0 + j];
       w += kept((uint32_t)(b0 + j), cnt_of(v)) * prob62(v);
-      if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
     }
     uint64_t wpre = w;
     uint32_t unused = 0;
@@ -721,15 +721,11 @@ __global__ void __launch_bounds__(SMP_T) smp_pick_kernel(SampleArgs a) {
   const RowWs& ws = a.ws[m];
   const uint32_t key = (uint32_t)ws.sel_key;
   int64_t rank = ws.sel_rank;
-  int hold = a.S - 1;
-  for (int s = 0; s < a.S; ++s) {
-    const int64_t c = ws.slice_cnt[s];
-    if (rank < c) {
-      hold = s;
-      break;
-    }
-    rank -= c;
-  }
+  const int lane = tid & 63;
+  const uint32_t upto = wave_prefix(lane < a.S ? ws.slice_cnt[lane] : 0u, Add());
+  const uint64_t past = __ballot(rank < (int64_t)upto);  // slices that end past the rank
+  const int hold = past ? __builtin_ctzll(past) : a.S - 1;
+  if (hold > 0) rank -= lane_value(upto, hold - 1);
   if (tid == 0) s_token = -1;
   __syncthreads();
   const uint16_t* row = a.logits + (int64_t)m * a.ld;
