@@ -189,9 +189,10 @@ class Linear4bitNF4(nn.Module):
         dequantization."""
         from ..kernels.ops import nf4_dequant
 
-        qs = self.weight.quant_state
+        weight = self.weight
+        qs = weight.quant_state
         n = self.out_features * self.in_features
-        w = nf4_dequant(self.weight.data.view(-1), float_absmax(qs), qs.code, n, qs.blocksize,
+        w = nf4_dequant(weight.data.view(-1), float_absmax(qs), qs.code, n, qs.blocksize,
                         dtype=dtype)
         return w.view(self.out_features, self.in_features)
 
@@ -209,14 +210,16 @@ class Linear4bitNF4(nn.Module):
         Library GEMMs, forward + backward, out 8960, in 1536 (us): 71 -> 57 at 512
         rows, 103 -> 73 at 1024; 9216 x 2048 108 -> 89 at 1024, 190 -> 196 at 2800; the
         other way round for a wide in (1536 x 8960: 75 -> 109 at 1024)."""
-        from ..kernels import ops
+        n, k = self.out_features, self.in_features
+        if (n >= 2 * k and 1024 <= k <= 2048 and x.requires_grad and torch.is_grad_enabled()
+                and x.numel() <= 2048 * k):
+            from ..kernels import ops
 
-        n, k, qs = self.out_features, self.in_features, self.weight.quant_state
-        if (torch.is_grad_enabled() and x.requires_grad and n >= 2 * k and 1024 <= k <= 2048
-                and x.numel() <= 2048 * k
-                and ops.nf4_dequant_t_supported(self.weight.data, n, k, qs.blocksize)):
-            return ops.nf4_dequant_t(self.weight.data.view(-1), float_absmax(qs), qs.code, n, k,
-                                     qs.blocksize, dtype=dt).t()
+            weight = self.weight
+            qs, packed = weight.quant_state, weight.data
+            if ops.nf4_dequant_t_supported(packed, n, k, qs.blocksize):
+                return ops.nf4_dequant_t(packed.view(-1), float_absmax(qs), qs.code, n, k,
+                                         qs.blocksize, dtype=dt).t()
         return self.dequantize(dt)
 
     def extra_repr(self) -> str:

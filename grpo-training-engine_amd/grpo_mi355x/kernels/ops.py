@@ -55,6 +55,16 @@ def _need_dtype(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
         raise ValueError(f"{name} must be {dtype}, got {t.dtype}.")
 
 
+def _need_nf4(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor) -> None:
+    """The device and types of a packed weight, its float32 absmax and its codebook."""
+    if not (packed.is_cuda and absmax.is_cuda and code.is_cuda and packed.dtype == torch.uint8
+            and absmax.dtype == torch.float32 and code.dtype == torch.float32):
+        _need_cuda(packed, absmax, code)
+        _need_dtype(packed, torch.uint8, "packed weight")
+        _need_dtype(absmax, torch.float32, "absmax")
+        _need_dtype(code, torch.float32, "code")
+
+
 # --------------------------------------------------------------- NF4 ---
 
 def nf4_absmax_expand(absmax_q: torch.Tensor, code2: torch.Tensor, absmax2: torch.Tensor,
@@ -88,10 +98,7 @@ def nf4_dequant(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor, 
     if dtype not in (torch.bfloat16, torch.float16):
         raise ValueError(f"dequantization to bfloat16 or float16, got {dtype}.")
     lib = _lib.device_library()
-    _need_cuda(packed, absmax, code)
-    _need_dtype(packed, torch.uint8, "packed weight")
-    _need_dtype(absmax, torch.float32, "absmax")
-    _need_dtype(code, torch.float32, "code")
+    _need_nf4(packed, absmax, code)
     if packed.numel() * 2 < numel:
         raise ValueError(f"packed weight holds {packed.numel() * 2} nibbles, need {numel}.")
     if absmax.numel() * blocksize < numel:
@@ -119,13 +126,15 @@ def nf4_dequant_t_supported(packed: torch.Tensor, n: int, k: int, blocksize: int
 def nf4_dequant_t(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor, n: int, k: int,
                   blocksize: int, dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """``nf4_dequant`` of W [n, k], stored transposed: a contiguous [k, n] tensor."""
+    if dtype not in (torch.bfloat16, torch.float16):
+        raise ValueError(f"dequantization to bfloat16 or float16, got {dtype}.")
     lib = _lib.device_library()
-    _need_cuda(packed, absmax, code)
-    _need_dtype(absmax, torch.float32, "absmax")
+    _need_nf4(packed, absmax, code)
     if packed.numel() * 2 < n * k or absmax.numel() * blocksize < n * k:
         raise ValueError("packed weight or absmax too short for [n, k].")
     if code.numel() != 16:
         raise ValueError("code must have 16 entries.")
+    packed, absmax, code = packed.contiguous(), absmax.contiguous(), code.contiguous()
     out = torch.empty((k, n), dtype=dtype, device=packed.device)
     _lib.check(lib.grpo_nf4_dequant_t(
         packed.data_ptr(), absmax.data_ptr(), code.data_ptr(), out.data_ptr(), n, k, blocksize,

@@ -192,3 +192,21 @@ def test_no_grad_call_is_the_recorded_one(dev):
         # vmap: no storage to hand to a kernel; the layer's torch branch serves it
         y = torch.vmap(lambda t: layer(t))(torch.stack([x, 2 * x]))
         assert y.shape == (2, 1, 600, 256)
+
+
+def test_transposed_dequant_of_strided_scales(dev):
+    """The weight kept transposed for a gradient holds the values of dequantize() also
+    for strided absmax and codebook, and what dequantize() refuses stays refused."""
+    from grpo_mi355x.core.nf4 import Linear4bitNF4
+
+    torch.manual_seed(3)
+    layer = Linear4bitNF4.from_weight(torch.randn(2048, 1024, device=dev) * 0.02)
+    x = torch.randn(1, 40, 1024, device=dev).bfloat16().requires_grad_()
+    qs, want = layer.weight.quant_state, layer.dequantize()
+    every2 = lambda t: torch.stack([t, t + 1], 1).view(-1)[::2]
+    qs.absmax, qs.code = every2(qs.absmax), every2(qs.code)
+    w = layer._dequantized_for(x, torch.bfloat16)
+    assert not w.is_contiguous() and torch.equal(w, want)  # stored [in, out]
+    qs.code = qs.code.double()
+    with pytest.raises(ValueError):
+        layer(x)
