@@ -62,6 +62,20 @@ __global__ void __launch_bounds__(ROW_T) embedding_kernel(const int64_t* __restr
   for (int i = threadIdx.x; i < H; i += ROW_T) out[(int64_t)b * H + i] = ok ? src[i] : 0;
 }
 
+// ... in 16-byte pieces (H % 8 == 0, aligned rows): 64 rows of 3584 8.2 -> 4.7 us, bound by
+// the launch and two dependent loads.
+__global__ void __launch_bounds__(ROW_T) embedding_vec_kernel(const int64_t* __restrict__ ids,
+                                                              const uint16_t* __restrict__ table,
+                                                              int64_t V, int H,
+                                                              uint16_t* __restrict__ out) {
+  const int b = blockIdx.x;
+  const int64_t id = ids[b];
+  const bool ok = id >= 0 && id < V;
+  const uint4* const src = reinterpret_cast<const uint4*>(table + (ok ? id : 0) * (int64_t)H);
+  uint4* const dst = reinterpret_cast<uint4*>(out + (int64_t)b * H);
+  for (int i = threadIdx.x; i < H / 8; i += ROW_T) dst[i] = ok ? src[i] : make_uint4(0, 0, 0, 0);
+}
+
 // embedding_kernel that also writes the RMSNorm statistic of each row:
 // sumsq[b, t] = sum of out[b, i]^2 over i = t, t + ROW_T, ... (ROW_T groups per
 // row), which the first q|k|v kernel stages the input norm from.
@@ -107,6 +121,70 @@ __global__ void __launch_bounds__(ROW_T) add_rmsnorm_kernel(
   }
 }
 
+__device__ __forceinline__ uint32_t word4(const uint4& v, int i) {
+  return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
+}
+__device__ __forceinline__ void unpack8(const uint4& v, float (&f)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = bf_lo(word4(v, i));
+    f[2 * i + 1] = bf_hi(word4(v, i));
+  }
+}
+__device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
+  return make_uint4(pack_bf2(f[0], f[1]), pack_bf2(f[2], f[3]), pack_bf2(f[4], f[5]),
+                    pack_bf2(f[6], f[7]));
+}
+
+// add_rmsnorm_kernel for H % 8 == 0, H <= 2048 U and 16-byte aligned rows: a thread keeps U
+// pieces of 8 columns in registers and loads everything, the norm's weight included,
+// before the sum, so that a row is one round trip to memory and one barrier (the
+// column-wise loop made a trip per 256 columns).  511 rows of 1536: 7.1 -> 5.1 us.
+template <int U>
+__global__ void __launch_bounds__(ROW_T) add_rmsnorm_vec_kernel(
+    const uint16_t* x, const uint16_t* residual, uint16_t* h_out, const uint16_t* __restrict__ w,
+    uint16_t* y, int H, float eps) {
+  __shared__ float red[ROW_T / 64];
+  const int64_t row = (int64_t)blockIdx.x * H;
+  const int tid = threadIdx.x, n8 = H / 8;
+  uint4 xv[U], rv[U], wv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = 8 * min(tid + ROW_T * u, n8 - 1);
+    xv[u] = *reinterpret_cast<const uint4*>(x + row + c);
+    if (residual) rv[u] = *reinterpret_cast<const uint4*>(residual + row + c);
+    wv[u] = *reinterpret_cast<const uint4*>(w + c);
+  }
+  float h[U][8], ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    unpack8(xv[u], h[u]);
+    if (residual) {
+      float r[8];
+      unpack8(rv[u], r);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[u][e] = round_bf(h[u][e] + r[e]);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += h[u][e] * h[u][e];
+    ss += tid + ROW_T * u < n8 ? s : 0.f;
+  }
+  const float total = block_sum(ss, red);
+  const float inv = 1.f / sqrtf(total / (float)H + eps);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = tid + ROW_T * u;
+    if (c >= n8) break;
+    if (residual && h_out) *reinterpret_cast<uint4*>(h_out + row + 8 * c) = pack8(h[u]);
+    float wf[8];
+    unpack8(wv[u], wf);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wf[e] = round_bf(h[u][e] * inv) * wf[e];
+    *reinterpret_cast<uint4*>(y + row + 8 * c) = pack8(wf);
+  }
+}
+
 // RoPE (x*cos + rotate_half(x)*sin in bf16 arithmetic, transformers'
 // apply_rotary_pos_emb) on q and k of one token per sequence, then the KV
 // append of paged_kv.py:253-319 at slot context_lens[b].
@@ -147,6 +225,60 @@ __global__ void __launch_bounds__(ROW_T) rope_append_kernel(
     } else if (slot_ok) {
       const int j = i - nrot, h = j / D, d = j - h * D;
       vc[slot_base + (int64_t)h * BS * D + d] = row[nrot + j];
+    }
+  }
+}
+
+// rope_append_kernel in 16-byte pieces (D % 16 == 0, 16-byte aligned rows): a thread rotates
+// 8 pairs (d, d + D/2) or copies 8 values of v; its row's loads do not wait for the
+// position.  511 rows of 12 / 2 heads: 7.4 -> 4.7 us.
+__global__ void __launch_bounds__(ROW_T) rope_append_vec_kernel(
+    const uint16_t* __restrict__ qkv, int64_t ld, int Hq, int Hkv, int D,
+    const uint16_t* __restrict__ cos_t, const uint16_t* __restrict__ sin_t, int max_pos,
+    const int32_t* __restrict__ context_lens, uint16_t* __restrict__ q_out,
+    uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int64_t num_blocks,
+    const int32_t* __restrict__ bt, int64_t bts, int BS, int max_blocks) {
+  const int b = blockIdx.x;
+  const int pos = context_lens[b];
+  const int cpos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
+  const uint16_t* const row = qkv + (int64_t)b * ld;
+  const int half = D / 2, hc = half / 8, vc8 = D / 8;
+  const int nrot = (Hq + Hkv) * hc;
+  bool slot_ok = pos >= 0 && pos < max_blocks * BS;
+  int64_t slot_base = 0;
+  if (slot_ok) {
+    const int phys = bt[(int64_t)b * bts + pos / BS];
+    slot_ok = phys >= 0 && phys < num_blocks;
+    slot_base = ((int64_t)phys * Hkv * BS + (pos % BS)) * D;  // + h * BS * D + d
+  }
+  auto at = [](const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); };
+  for (int i = threadIdx.x; i < nrot + Hkv * vc8; i += ROW_T) {
+    if (i < nrot) {
+      const int h = i / hc, d = 8 * (i - h * hc);
+      const uint16_t* const xh = row + (int64_t)h * D + d;  // q heads then k heads
+      float x1[8], x2[8], c1[8], c2[8], s1[8], s2[8];
+      unpack8(at(xh), x1);
+      unpack8(at(xh + half), x2);
+      unpack8(at(cos_t + (int64_t)cpos * D + d), c1);
+      unpack8(at(cos_t + (int64_t)cpos * D + d + half), c2);
+      unpack8(at(sin_t + (int64_t)cpos * D + d), s1);
+      unpack8(at(sin_t + (int64_t)cpos * D + d + half), s2);
+      float lo[8], hi[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        lo[e] = round_bf(x1[e] * c1[e]) + round_bf(-x2[e] * s1[e]);
+        hi[e] = round_bf(x2[e] * c2[e]) + round_bf(x1[e] * s2[e]);
+      }
+      uint16_t* dst = h < Hq ? q_out + ((int64_t)b * Hq + h) * D + d
+                             : kc + slot_base + (int64_t)(h - Hq) * BS * D + d;
+      if (h < Hq || slot_ok) {
+        *reinterpret_cast<uint4*>(dst) = pack8(lo);
+        *reinterpret_cast<uint4*>(dst + half) = pack8(hi);
+      }
+    } else if (slot_ok) {
+      const int j = i - nrot, h = j / vc8, d = 8 * (j - h * vc8);
+      *reinterpret_cast<uint4*>(vc + slot_base + (int64_t)h * BS * D + d) =
+          at(row + (int64_t)(Hq + Hkv + h) * D + d);
     }
   }
 }
@@ -527,7 +659,9 @@ extern "C" int grpo_embedding(const int64_t* ids, const void* table, int64_t V, 
   if (B < 0 || H <= 0 || V <= 0) return einval("bad embedding dimensions");
   if (B == 0) return GRPO_OK;
   if (!ids || !table || !out) return einval("null pointer");
-  embedding_kernel<<<dim3(B), ROW_T, 0, as_stream(stream)>>>(
+  const auto kern =
+      H % 8 == 0 && aligned16(table) && aligned16(out) ? embedding_vec_kernel : embedding_kernel;
+  kern<<<dim3(B), ROW_T, 0, as_stream(stream)>>>(
       ids, static_cast<const uint16_t*>(table), V, H, static_cast<uint16_t*>(out));
   return launch_check("embedding");
 }
@@ -550,10 +684,18 @@ extern "C" int grpo_add_rmsnorm(const void* x, const void* residual, void* h_out
   if (M < 0 || H <= 0 || H > 16384) return einval("bad rmsnorm dimensions (H <= 16384)");
   if (M == 0) return GRPO_OK;
   if (!x || !weight || !y) return einval("null pointer");
-  add_rmsnorm_kernel<<<dim3(M), ROW_T, H * sizeof(float), as_stream(stream)>>>(
-      static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual),
-      static_cast<uint16_t*>(h_out), static_cast<const uint16_t*>(weight),
-      static_cast<uint16_t*>(y), H, eps);
+  auto go = [&](auto kern, size_t lds) {
+    kern<<<dim3(M), ROW_T, lds, as_stream(stream)>>>(
+        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual),
+        static_cast<uint16_t*>(h_out), static_cast<const uint16_t*>(weight),
+        static_cast<uint16_t*>(y), H, eps);
+  };
+  // (a null residual or h_out counts as aligned)
+  const bool vec = H % 8 == 0 && aligned16(x) && aligned16(residual) && aligned16(h_out) &&
+                   aligned16(weight) && aligned16(y);
+  if (vec && H <= 8 * ROW_T) go(add_rmsnorm_vec_kernel<1>, 0);
+  else if (vec && H <= 16 * ROW_T) go(add_rmsnorm_vec_kernel<2>, 0);
+  else go(add_rmsnorm_kernel, H * sizeof(float));
   return launch_check("add_rmsnorm");
 }
 
@@ -570,7 +712,11 @@ extern "C" int grpo_rope_append(const void* qkv, int64_t ld, int Hq, int Hkv, in
   if (!qkv || !cos_table || !sin_table || !context_lens || !q_out || !k_cache || !v_cache ||
       !block_tables)
     return einval("null pointer");
-  rope_append_kernel<<<dim3(B), ROW_T, 0, as_stream(stream)>>>(
+  const bool vec = D % 16 == 0 && ld % 8 == 0 && aligned16(qkv) && aligned16(cos_table) &&
+                   aligned16(sin_table) && aligned16(q_out) && aligned16(k_cache) &&
+                   aligned16(v_cache);
+  const auto kern = vec ? rope_append_vec_kernel : rope_append_kernel;
+  kern<<<dim3(B), ROW_T, 0, as_stream(stream)>>>(
       static_cast<const uint16_t*>(qkv), ld, Hq, Hkv, D, static_cast<const uint16_t*>(cos_table),
       static_cast<const uint16_t*>(sin_table), max_pos, context_lens,
       static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(k_cache),
