@@ -142,15 +142,17 @@ __global__ void __launch_bounds__(64 * CS * HW) prefill_attn_kernel(PrefillArgs 
     wait_vm<0>();  // step st has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    // the slot filled now was read a step ago: every wave is past that
-    const int nx = min(st + 1, nstep - 1);
-    if (nx / (64 / STEP_BLK) != win) {
-      win = nx / (64 / STEP_BLK);
-      tb_v = p.bt[min(64 * win + lane, p.max_blocks - 1)];
-      okm_before = okm;
-      take_table();
+    // The slot filled now was read a step ago: every wave is past that. The last step
+    // fetches nothing (the slots hold what it and the step before it read).
+    if (st + 1 < nstep) {
+      if ((st + 1) / (64 / STEP_BLK) != win) {
+        win = (st + 1) / (64 / STEP_BLK);
+        tb_v = p.bt[min(64 * win + lane, p.max_blocks - 1)];
+        okm_before = okm;
+        take_table();
+      }
+      fetch(st + 1);
     }
-    fetch(nx);
     const int t0 = STEP * st + 32 * part;
     if (t0 >= most) continue;
     const uint64_t okw = st / (64 / STEP_BLK) == win ? okm : okm_before;

@@ -42,12 +42,15 @@ def _run(dev, M, Hq, Hkv, lens, max_blocks, seed, holes=()):
     return out.float(), want, (q, k, v, table)
 
 
-# rows: within, at and past a 16-row tile; contexts: within a block, at and past the 32-
-# and 64-token halves and steps, the ring of three steps, the 64-block table windows, empty and clamped ones
+# rows: within, at and past a 16-row tile; contexts: within a block, at and past the 32-token
+# parts, the 128-token steps, the ring of two, the 64-block table windows, empty and clamped ones
 @pytest.mark.parametrize("M,Hq,Hkv,first,max_blocks", [
     (1, 1, 1, 1, 1), (17, 12, 2, 1, 2), (16, 4, 4, 17, 3), (40, 7, 1, 60, 8), (64, 28, 4, 129, 12),
     (33, 10, 2, 200, 16), (70, 8, 1, 1, 6), (512, 12, 2, 1, 32), (100, 16, 8, 4000, 260),
-    (16, 2, 1, 1009, 64), (16, 2, 1, 1020, 70), (16, 2, 1, 2040, 130)])
+    (16, 2, 1, 1009, 64), (16, 2, 1, 1020, 70), (16, 2, 1, 2040, 130),
+    # a longest row that ends with a step, which fetches nothing after it: the first,
+    # the second, the first of the second table window
+    (16, 2, 1, 113, 8), (16, 2, 1, 241, 16), (16, 12, 2, 1137, 72)])
 def test_prefill_attention(dev, M, Hq, Hkv, first, max_blocks):
     lens = [first + i for i in range(M)]
     if M > 20:
