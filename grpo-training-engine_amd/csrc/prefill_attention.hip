@@ -22,9 +22,13 @@
 //    both 16-token tiles, which is the operand P^T of the next product if its
 //    contraction index (lg, e) means token 16 (e / 4) + 4 lg + e % 4: P never leaves
 //    the lane. V's operand is read as rows and its pairs are turned with v_perm.
-// Bound by that issue and, for short contexts, by the launch and the first loads (6.5
-// us at 128 rows). 512 rows after nothing, 12 query and 2 KV heads: 11.2 us against
-// 28.0 for the decode kernel and its merge; after 2000 tokens 33 us.
+//  * A token that only some of the 16 rows attend has P = 0 in the others. Where its V is
+//    not finite (an overflow, a slot never written) it is taken out of the product and
+//    the rows that do attend it are set to NaN.
+// Bound by that issue and, for short contexts, by the launch and the first loads (7.1
+// us at 128 rows, 0.4 of them for the look at values that are not finite). 512 rows
+// after nothing, 12 query and 2 KV heads: 11.5 us against 29.1 for the decode kernel and
+// its merge; after 4000 tokens 55 us against 164.
 #include <algorithm>
 
 #include "lds_dma.hpp"
@@ -66,6 +70,31 @@ __device__ __forceinline__ int max16(int v) {
 
 __device__ __forceinline__ uint32_t word(const uint4& v, int i) {
   return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
+}
+
+__device__ __forceinline__ uint4 keep(uint32_t mask, const uint4& v) {
+  return make_uint4(v.x & mask, v.y & mask, v.z & mask, v.w & mask);
+}
+// All ones in the halves of d that are an infinity or NaN (exponent bits all set).
+__device__ __forceinline__ uint32_t inf_mask(uint32_t d) {
+  return ((d & 0x7F80u) == 0x7F80u ? 0xFFFFu : 0u) |
+         ((d & 0x7F800000u) == 0x7F800000u ? 0xFFFF0000u : 0u);
+}
+// Per half the larger of m and of v's bits in mask.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2 max_halves(u16x2 m, uint32_t mask, const uint4& v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, word(v, i) & mask));
+  return m;
+}
+// Of V's rows (a token each, 8 dims) the operand V^T of the dims 8 (..) + i.
+__device__ __forceinline__ uint4 turned(const uint4 (&v)[8], int i) {
+  const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
+  return make_uint4(perm(word(v[1], i >> 1), word(v[0], i >> 1), sel),
+                    perm(word(v[3], i >> 1), word(v[2], i >> 1), sel),
+                    perm(word(v[5], i >> 1), word(v[4], i >> 1), sel),
+                    perm(word(v[7], i >> 1), word(v[6], i >> 1), sel));
 }
 
 // HW heads per workgroup, CS parts of a step (32 tokens each): CS HW waves.
@@ -183,12 +212,37 @@ __global__ void __launch_bounds__(64 * CS * HW) prefill_attn_kernel(PrefillArgs 
     for (int e = 0; e < 8; ++e) sv[e] = s[e >> 2][e & 3] * sl2;
     if (t0 + 32 > least || !(ok0 && ok1)) {  // some row ends here, or a block is missing
       const uint32_t z[2] = {ok0 ? ~0u : 0u, ok1 ? ~0u : 0u};
+      u16x2 top{0, 0};  // largest exponent of the tokens that some row does not attend
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const bool on = t0 + 16 * (e >> 2) + 4 * lg + (e & 3) < len && z[e >> 2];
+        const int t = t0 + 16 * (e >> 2) + 4 * lg + (e & 3);
+        const bool on = t < len && z[e >> 2];
         sv[e] = on ? sv[e] : -INFINITY;
-        v[e] = make_uint4(v[e].x & z[e >> 2], v[e].y & z[e >> 2], v[e].z & z[e >> 2],
-                          v[e].w & z[e >> 2]);
+        v[e] = keep(z[e >> 2], v[e]);
+        top = max_halves(top, t < least ? 0u : 0x7F807F80u, v[e]);
+      }
+      // A value that is not finite, in a token that some row does not attend: 0 times it
+      // would be NaN. It leaves V; the rows that attend its token become NaN there.
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(max(top.x, top.y) == 0x7F80u) != 0, 0)) {
+        uint32_t one[4] = {0, 0, 0, 0};  // 1 (bf16) for the tokens that the row attends
+        uint4 w[8];                      // ... and for the values that leave V
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int t = t0 + 16 * (e >> 2) + 4 * lg + (e & 3);
+          one[e >> 1] |= t < len ? 0x3F80u << (16 * (e & 1)) : 0u;
+          const uint4 f = keep(t >= least ? ~0u : 0u,
+                               make_uint4(inf_mask(v[e].x), inf_mask(v[e].y), inf_mask(v[e].z),
+                                          inf_mask(v[e].w)));
+          w[e] = keep(0x3F803F80u, f);
+          v[e] = make_uint4(v[e].x & ~f.x, v[e].y & ~f.y, v[e].z & ~f.z, v[e].w & ~f.w);
+        }
+        const uint4 b = make_uint4(one[0], one[1], one[2], one[3]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const f32x4_t n = mfma16x16x32(turned(w, i), b, f32x4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int q = 0; q < 4; ++q) oacc[i][q] = n[q] > 0.f ? NAN : oacc[i][q];
+        }
       }
     }
 #pragma unroll
@@ -219,11 +273,7 @@ __global__ void __launch_bounds__(64 * CS * HW) prefill_attn_kernel(PrefillArgs 
     const uint4 bl = make_uint4(pl[0], pl[1], pl[2], pl[3]);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
-      const uint4 a = make_uint4(perm(word(v[1], i >> 1), word(v[0], i >> 1), sel),
-                                 perm(word(v[3], i >> 1), word(v[2], i >> 1), sel),
-                                 perm(word(v[5], i >> 1), word(v[4], i >> 1), sel),
-                                 perm(word(v[7], i >> 1), word(v[6], i >> 1), sel));
+      const uint4 a = turned(v, i);
       oacc[i] = mfma16x16x32(a, bh, oacc[i]);
       oacc[i] = mfma16x16x32(a, bl, oacc[i]);
     }

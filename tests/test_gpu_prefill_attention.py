@@ -80,3 +80,47 @@ def test_prefill_attention_against_float64(dev):
     want = torch.einsum("mht,thd->mhd", p, vv)
     # one rounding to bf16: half an ulp, 2^-9, with a little for the float32 sums
     assert float(((got - want).abs() / want.abs().clamp(min=1e-2)).max()) <= 1.05 * 2.0 ** -8
+
+
+# lens of a chunk that starts inside a block, of rows in no order, of idle rows; four parts and two
+@pytest.mark.parametrize("M,Hq,Hkv,lens", [
+    (40, 6, 1, lambda i: 101 + i), (33, 4, 4, lambda i: (37 * i) % 250),
+    (600, 14, 2, lambda i: 3 * i % 700), (530, 8, 8, lambda i: 90 + i % 50)])
+def test_prefill_attention_takes_nothing_from_tokens_past_a_context(dev, M, Hq, Hkv, lens):
+    """Infinite and NaN values of tokens that a row does not attend (later tokens of the
+    chunk, slots not written yet) do not reach it; of those it attends, they do."""
+    from grpo_mi355x import _lib
+
+    lib = _lib.device_library()
+    g = torch.Generator().manual_seed(M)
+    n = [lens(i) for i in range(M)]
+    top = max(n)
+    max_blocks = -(-top // 16)
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, k, v = rnd(M, Hq, 128), rnd(max_blocks, Hkv, 16, 128), rnd(max_blocks, Hkv, 16, 128)
+    at = lambda c, t: c[t // 16, :, t % 16]  # table: the identity
+    for i, t in enumerate(t for t in (70, 112, 113, 127, 128, 200, top - 1) if t < top):
+        at(v, t)[:, 5 * i] = (float("inf"), float("-inf"), float("nan"))[i % 3]
+    at(k, min(top - 1, 130))[:] = float("nan")
+    for t in range(top, 16 * max_blocks):  # never written
+        at(k, t)[:], at(v, t)[:] = float("nan"), float("nan")
+    table, ln = torch.arange(max_blocks, dtype=torch.int32), torch.tensor(n, dtype=torch.int32)
+    d = [t.to(dev) for t in (q, k, v, table, ln)]
+    out = torch.empty(M, Hq, 128, dtype=torch.bfloat16, device=dev)
+    print(f"prefill attention, values not finite, M={M} Hq={Hq} Hkv={Hkv}", flush=True)
+    _lib.check(lib.grpo_paged_attn_prefill(
+        d[0].data_ptr(), Hq * 128, 128, d[1].data_ptr(), d[2].data_ptr(), max_blocks,
+        d[3].data_ptr(), d[4].data_ptr(), out.data_ptr(), M, Hq, Hkv, 128, 16, max_blocks,
+        1 / math.sqrt(128), _lib.stream_handle(dev)), "prefill")
+    got = out.float().cpu()
+    kk, vv = (c.transpose(1, 2).reshape(-1, Hkv, 128).double().repeat_interleave(Hq // Hkv, 1)
+              for c in (k, v))
+    for m in range(M):
+        if n[m] == 0:
+            assert not got[m].any()
+            continue
+        s = torch.einsum("hd,thd->ht", q[m].double(), kk[:n[m]]) / math.sqrt(128)
+        want = torch.einsum("ht,thd->hd", torch.softmax(s, -1), vv[:n[m]])
+        on = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got[m]), on), (m, n[m])
+        assert ((got[m] - want).abs()[on] <= 1.05 * 2.0 ** -8 * want.abs()[on].clamp(min=1e-2)).all()
