@@ -33,8 +33,10 @@
 //    goes to the ids = x mod 8, so the row tiles of a column tile read its
 //    weights through one L2 and every XCD gets the same number of tiles.
 //
-// bf16 with K % 128 == 0, r <= 16 and blocksize >= 64 runs nf4_gemm_k2 (below) instead,
-// which was no slower at any of 45 measured shapes of 128 .. 2048 rows.
+// bf16 with K % 128 == 0, r <= 16 and blocksize >= 64 runs nf4_gemm_k2 (below) instead:
+// with the tile and slices that its time model picks it was slower at 2 of 560 measured
+// shapes of 65 .. 4096 rows (224 x 4608 x 3584 6 %, 1024 x 1536 x 8960 3 %), at the median
+// 0.77 of the time, its SiLU form 0.68 .. 0.93; profiles/nf4_gemm_wide_batches.md.
 #include <algorithm>
 #include <type_traits>
 
@@ -955,11 +957,11 @@ __global__ void __launch_bounds__(64 * WM * WN * KS, 2) nf4_gemm_k2(K2Args p) {
   }
 }
 
-// Tiles of nf4_gemm_k2 (ks K groups) and their time model in us, fitted to 430 measured
-// shapes of 128 .. 2048 rows (r.m.s. error 6 %; the tile it picks is within 7 % of the
-// best one measured, and within 2 % in 40 of 45 shapes): a round of workgroups costs
-// `fixed` and, per step, `step` alone on a CU, `more` for each further one that fits
-// (occ, occ_l with LoRA), `lora` with LoRA.
+// Tiles of nf4_gemm_k2 (ks K groups) and their time model in us: a round of workgroups
+// costs `fixed` and, per step, `step` alone on a CU, `more` for each further one that fits
+// (occ, occ_l with LoRA), `lora` with LoRA. Over 560 shapes of 65 .. 4096 rows, each
+// measured with every tile and up to 13 slice counts, its r.m.s. error is 8 %; what it
+// picks is within 1 % of the best one at 90 % of them, within 13 % at all.
 struct K2Tile {
   int bm, bn, ks, occ, occ_l;
   double fixed, step, more, lora;
@@ -975,9 +977,12 @@ constexpr bool k2_has(int tile, K2Mode mode, bool lora) {
 }
 
 // The tile for the segments' columns (SILU: I columns of half a tile each) in S K
-// slices of kss superstages, and its time in us. A split also writes float32 partial
-// sums, reads them back and launches the finish (3.2 us; 1.4 us per million sums, with
-// LoRA 3.3 us per million outputs).
+// slices of kss superstages, and its time in us. Rounds are counted on the XCD with the
+// most workgroups, ceil(tiles / 8) in every slice, over its 32 CUs: 28 tiles in 9 slices
+// are 252 workgroups, but 36 on four of the XCDs, and take two rounds (128 x 3584 x
+// 18944: 55.8 us, in 8 slices 39.2). A split also writes float32 partial sums, reads them
+// back and launches the finish (3.2 us; 1.4 us per million sums, with LoRA 3.3 us per
+// million outputs).
 int k2_tile(int M, int nseg, const int* seg_end, int kss, int S, bool lora, K2Mode mode,
             double* us) {
   int best = -1;
@@ -987,14 +992,14 @@ int k2_tile(int M, int nseg, const int* seg_end, int kss, int S, bool lora, K2Mo
     int64_t nt = 0;
     for (int s = 0, start = 0; s < nseg; start = seg_end[s], ++s)
       nt += cdiv(seg_end[s] - start, mode == K2_SILU ? c.bn / 2 : c.bn);
-    const int64_t tiles = cdiv(M, c.bm) * nt * S;
+    const int64_t tiles = cdiv(cdiv(M, c.bm) * nt, 8) * S;  // of an XCD
     const int occ = lora ? c.occ_l : c.occ;
     auto round = [&](int64_t per_cu) {
       return c.fixed + 4 * (double)cdiv(kss, c.ks) *
                            (c.step + (lora ? c.lora : 0.0) + (double)(per_cu - 1) * c.more);
     };
-    const int64_t full = tiles / (256 * occ), rem = tiles % (256 * occ);
-    double t = 3.5 + (double)full * round(occ) + (rem ? round(cdiv(rem, 256)) : 0.0);
+    const int64_t full = tiles / (32 * occ), rem = tiles % (32 * occ);
+    double t = 3.5 + (double)full * round(occ) + (rem ? round(cdiv(rem, 32)) : 0.0);
     if (S > 1) {
       const double outs = (double)M * seg_end[nseg - 1];
       t += 3.2 + outs * (S * 1.4e-6 + (lora ? 3.3e-6 : 0.0));
@@ -1338,6 +1343,24 @@ int nf4_gemm_silu_launch(const uint16_t* x, int64_t ldx, const uint8_t* w, const
 
 extern "C" int grpo_nf4_gemm_supported(int M, int N, int K, int r, int blocksize) {
   return gemm_ok(M, N, K, r, blocksize) ? 1 : 0;
+}
+
+extern "C" int grpo_nf4_gemm_tile(int M, int N, int K, int r, int blocksize, int silu, int* rows,
+                                  int* cols, int* k_groups, int* slices) {
+  const int64_t wrows = silu ? 2 * (int64_t)N : N;
+  if (!rows || !cols || !k_groups || !slices || wrows > INT32_MAX || (silu && r != 0) ||
+      !gemm_ok(M, (int)wrows, K, r, blocksize) || !k2_shape(K, r, wrows, blocksize))
+    return 0;
+  GemmPlan pl{1, (int)cdiv(K, GM_KS), 0, 0};
+  if (!silu) pl = nf4_gemm_plan(M, K, r, blocksize, 1, &N);
+  double us = 0.0;
+  const K2Tile& t = K2_TILE[k2_tile(M, 1, &N, pl.kst, pl.S, r > 0,
+                                    silu ? K2_SILU : (pl.S > 1 ? K2_PART : K2_OUT), &us)];
+  *rows = t.bm;
+  *cols = t.bn;
+  *k_groups = t.ks;
+  *slices = pl.S;
+  return 1;
 }
 
 namespace {

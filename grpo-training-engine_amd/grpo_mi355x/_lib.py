@@ -103,6 +103,7 @@ SIGNATURES = {
          _VP, _SZ, _VP],
     ),
     "grpo_nf4_gemm_supported": (_I32, [_I32, _I32, _I32, _I32, _I32]),
+    "grpo_nf4_gemm_tile": (_I32, [_I32] * 6 + [_c.POINTER(_I32)] * 4),
     "grpo_nf4_gemm": (
         _I32,
         [_VP, _I64, _VP, _VP, _VP, _I32, _VP, _VP, _VP, _I32, _F32, _VP, _I64, _I32, _I32, _I32,

@@ -299,6 +299,12 @@ int grpo_nf4_lora_linear(const void* x, int64_t ldx, const uint8_t* w, const flo
  * (ldx % 8 == 0); any M and N.  grpo_nf4_gemm_supported: 1 if the shape is
  * taken (alignment aside), else 0. */
 int grpo_nf4_gemm_supported(int M, int N, int K, int r, int blocksize);
+/* The tile (rows x weight rows), the groups of waves that share K in a workgroup and the
+ * slices of K that the NF4 GEMM's ring kernel runs a bf16 linear of this shape with
+ * (silu: the gate|up + SiLU form, N its activation columns); 1, or 0 where another
+ * kernel runs it. */
+int grpo_nf4_gemm_tile(int M, int N, int K, int r, int blocksize, int silu, int* rows,
+                       int* cols, int* k_groups, int* slices);
 int grpo_nf4_gemm(const void* x, int64_t ldx, const uint8_t* w, const float* absmax,
                   const float* code16, int blocksize, const void* bias, const void* lora_a,
                   const void* lora_b, int r, float scaling, void* y, int64_t ldy, int M, int N,
