@@ -22,8 +22,9 @@ with float16 adapters (the reference's float16 X_DTYPE / LORA_DTYPE, ``:141-143,
 take).  The backward (``:761-930``) is ``grpo_nf4_lora_train_backward``: the
 reference's gradients and rounding points, grad_x as one GEMM over the weight
 transposed in 16 bits, everything of rank r straight from x and grad_out.
-Tensors the training kernels do not take (``_train_workspace``), and a backward
-that is itself differentiated, run the same products as torch ops.
+Tensors the training kernels do not take (``_train_workspace``), a forward of many
+rows whose product is too long for its tiles (``train_forward_pays``) and a
+backward that is itself differentiated run the same products as torch ops.
 """
 
 from __future__ import annotations
@@ -155,10 +156,27 @@ def train_forward_pays(m: int, n: int, k: int, r: int, blocksize: int,
     54.8 at 1024; 256 x 1536 15.5 / 19.1 at 4096.  Shapes its older kernel takes cross
     earlier: 24.2 / 19.2 at 512 rows of 1536 x 1536, 136.6 / 106.3 at 2048 of 1536 x
     8960.  In float16 the decoding kernel does not split K: 32.9 / 17.2 (1536 x 1536) and
-    33.2 / 30.1 (8960 x 1536) at 16 rows."""
+    33.2 / 30.1 (8960 x 1536) at 16 rows; it wins where N is wide enough to fill the chip
+    at few rows over a short K (8960 x 1536 34.5 / 38.3 at 256, 48.2 / 45.5 at 512; 8960 x
+    1024 26.2 / 30.2 at 384).
+
+    Beyond ``fused_forward_rows`` the other route is the dequantized weight + library
+    GEMMs, which cut a long K over the CUs that the 256 x 256 tiles leave idle: K = 8960,
+    r = 16, that against this, 135 / 176 at 3072 rows of N 1536 (72 tiles), 177 / 208 at
+    4096 of 2048 (128), 389 / 479 at 8192 of 2560 (320: two rounds), but 249 / 243 at 8192 of
+    2048 (256) and 616 / 454 at 2048 of 8960.  At K = 18944 the library's time is uneven and
+    this one is mostly faster (3584 columns: 458 / 387 at 2048 rows, 357 / 370 at 1536).
+    Rank 32 costs the preparation more, which decides at few columns: 55.7 / 66.2 at 6144
+    rows of 512 x 3584."""
+    rows = fused_forward_rows(k)
+    if m > rows:
+        if 4096 < k <= 10240 and n <= 4096:
+            tiles = -(-m // 256) * -(-n // 256)
+            return tiles >= (0.73 if r <= 16 else 0.88) * 256 * -(-tiles // 256)
+        return not (r > 16 and n <= 1024 and 3072 <= k <= 4096)
     if dtype == torch.float16:
-        return True
-    if k % 128 == 0 and r <= 16 and blocksize >= 64 and m <= fused_forward_rows(k):
+        return not (128 <= m <= 384 and k <= 1536 and n >= 4 * k)
+    if k % 128 == 0 and r <= 16 and blocksize >= 64:
         return m * n >= 5_000_000
     return m >= (512 if k <= 4096 else 1024)
 

@@ -210,3 +210,23 @@ def test_transposed_dequant_of_strided_scales(dev):
     qs.code = qs.code.double()
     with pytest.raises(ValueError):
         layer(x)
+
+
+@pytest.mark.parametrize("m,n,k,r,dt", [(1030, 96, 4224, 16, torch.bfloat16),
+                                        (1100, 64, 4128, 32, torch.float16)])
+def test_forward_over_library_products_is_the_training_forward(dev, m, n, k, r, dt):
+    """A long K over few tiles runs the dequantized weight + library products: the same
+    rounding points as the training kernels."""
+    from grpo_mi355x.core.nf4 import Linear4bitNF4
+    from grpo_mi355x.kernels import lora_forward as L, lora_fused_forward, ops
+
+    gen = torch.Generator().manual_seed(n)
+    rnd = lambda *s, sd: (torch.randn(*s, generator=gen) * sd).to(dt).to(dev)
+    base = Linear4bitNF4.from_weight(rnd(n, k, sd=0.02).float(), rnd(n, sd=1.0))
+    x, a, b = rnd(1, m, k, sd=1.0), rnd(r, k, sd=0.05), rnd(n, r, sd=0.05)
+    qs = base.weight.quant_state
+    assert not L.train_forward_pays(m, n, k, r, qs.blocksize, dt)
+    got = lora_fused_forward(x, base_layer=base, lora_A=a, lora_B=b, scaling=1.7)
+    want = ops.nf4_lora_train_forward(x[0], base.weight.data.view(-1), qs.absmax, qs.code,
+                                      qs.blocksize, a, b, 1.7, base.bias.to(dt))
+    _close(got[0], want.double(), dt, "y")

@@ -470,3 +470,25 @@ def test_live_width_covers_every_context_of_a_graph_replay():
     none = Stand(64)  # no position bound (start not called): the table width
     DecodeEngine.run(none, 32)
     assert none.replayed == [None, None]
+
+
+@pytest.mark.parametrize("m,n,k,r,dtype,train", [
+    # beyond fused_forward_rows: a long K over few or just too many 256 x 256 tiles
+    (1024, 1536, 8960, 32, torch.bfloat16, True), (1025, 1536, 8960, 32, torch.bfloat16, False),
+    (3072, 1536, 8960, 16, torch.float16, False), (8192, 1536, 8960, 16, torch.bfloat16, True),
+    (8192, 1536, 8960, 32, torch.bfloat16, False), (8192, 2048, 8960, 32, torch.bfloat16, True),
+    (8192, 2560, 8960, 8, torch.float16, False), (2048, 8960, 8960, 16, torch.bfloat16, True),
+    (2048, 3584, 18944, 16, torch.bfloat16, True),
+    (8192, 3584, 3584, 16, torch.bfloat16, True), (8192, 512, 3584, 16, torch.bfloat16, True),
+    (6144, 512, 3584, 32, torch.bfloat16, False), (6144, 512, 1536, 32, torch.bfloat16, True),
+    # float16 at few rows of a wide, short weight
+    (127, 8960, 1536, 8, torch.float16, True), (128, 8960, 1536, 8, torch.float16, False),
+    (384, 8960, 1536, 8, torch.float16, False), (385, 8960, 1536, 8, torch.float16, True),
+    (256, 1536, 1536, 8, torch.float16, True), (256, 8960, 2048, 8, torch.float16, True),
+    # the decoding kernels' own line
+    (255, 8960, 1536, 16, torch.bfloat16, False), (1024, 8960, 1536, 16, torch.bfloat16, True)])
+def test_training_forward_route(m, n, k, r, dtype, train):
+    """Which forward the shape runs is where the measurements cross (train_forward_pays)."""
+    from grpo_mi355x.kernels.lora_forward import train_forward_pays
+
+    assert train_forward_pays(m, n, k, r, 64, dtype) is train
