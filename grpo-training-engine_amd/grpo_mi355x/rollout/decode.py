@@ -881,6 +881,8 @@ class DecodeEngine:
             self.graph.replay()
         else:
             self._step()
+        if self._pos_hi is not None:
+            self._pos_hi += 1
 
     # steps recorded in one graph for run(): one graph launch per 16 steps
     # instead of one per step (7 us per step less at config 3)
@@ -949,9 +951,9 @@ class DecodeEngine:
                     self._pos_hi += self.MULTI_STEP
                 steps -= self.MULTI_STEP
         for _ in range(steps):
+            hi = self._pos_hi
             self.step()
-            if self._pos_hi is not None:
-                self._pos_hi += 1
+            self._pos_hi = None if hi is None else hi + 1
 
     def compaction_engines(self, sizes=(24, 16, 8)) -> list:
         """Greedy engines of fewer rows (``sizes`` below this engine's) over the

@@ -492,3 +492,39 @@ def test_training_forward_route(m, n, k, r, dtype, train):
     from grpo_mi355x.kernels.lora_forward import train_forward_pays
 
     assert train_forward_pays(m, n, k, r, 64, dtype) is train
+
+
+def test_steps_outside_run_move_the_position_bound():
+    """step() advances the rows by one: a later run() plans its splits for the contexts
+    that they have reached (a narrower plan would leave out the tokens past it)."""
+    from grpo_mi355x.rollout.decode import DecodeEngine
+
+    class Graph:
+        def __init__(self, log=None, pw=None):
+            self.log, self.pw = log, pw
+
+        def replay(self):
+            if self.log is not None:
+                self.log.append(self.pw)
+
+    class Stand:
+        LIVE_WIDTH, MULTI_STEP, B, Hkv = True, 16, 8, 2
+        max_blocks, attn_splits, attn_fused, _pos_hi = 64, 8, True, None
+        pool = type("Pool", (), {"block_size": 16})
+        step, _live_width = DecodeEngine.step, DecodeEngine._live_width
+
+        def _multi_graph(self, pw=None):
+            return Graph(self.widths, pw)
+
+    s = Stand()
+    s.graph, s.widths, s._pos_hi = Graph(), [], 100
+    DecodeEngine.run(s, 16 + 3)
+    assert s._pos_hi == 119
+    for _ in range(481):
+        s.step()
+    DecodeEngine.run(s, 16)
+    assert s._pos_hi == 616 and s.widths[0] * 16 >= 116 and s.widths[1] * 16 >= 616
+    s._pos_hi = None  # unknown: the table's width, and no bound appears
+    s.step()
+    DecodeEngine.run(s, 18)
+    assert s._pos_hi is None and s.widths[2] is None
