@@ -53,6 +53,13 @@ def _vp(x) -> ctypes.c_void_p:
     return ctypes.c_void_p(x)
 
 
+def _plans_by_context(eng) -> bool:
+    """Whether the engine's attention splits are planned for the live contexts
+    (``DecodeEngine.LIVE_WIDTH``)."""
+    return (getattr(eng, "attn_fused", False) and getattr(eng, "attn_splits", 1) > 1
+            and eng.LIVE_WIDTH and eng.B * eng.Hkv * 8 <= 256)
+
+
 class DecodeEngine:
     """Static-shape decode step for ``batch`` rows over a KV pool."""
 
@@ -821,8 +828,10 @@ class DecodeEngine:
             self.pad.data_ptr(), self.append_pos.data_ptr(), self.attn_len.data_ptr(),
             self.block_tables.data_ptr(), self.max_blocks, _lib.ptr(gen),
             0 if gen is None else gen.shape[1], _lib.stream_handle(dev)), "decode_start")
-        self._pos_hi = None
-        self._pos_stale = True  # read from the device when run() first plans splits
+        # run()'s plans need a bound on the positions: read here (a host sync where they
+        # are on the device), and only where the plans depend on it
+        self._pos_hi = (int(positions.max()) if positions.numel() and _plans_by_context(self)
+                        else None)
 
     def capture(self):
         """Record one step into a HIP graph (after two warm-up steps on a side stream)."""
@@ -901,16 +910,13 @@ class DecodeEngine:
     # (config 4's 32-row engine: 8867 tok/s planned live against 8927).
     LIVE_WIDTH = True
     _pw: Optional[int] = None  # plan width of the launches being built (None: the table's)
-    # bound on every row's position (None: unknown); stale: after start(), until
-    # run() needs it (a host sync)
+    # bound on every row's position (None: unknown, or no plan depends on it)
     _pos_hi: Optional[int] = None
-    _pos_stale = False
 
     def _live_width(self, ctx: int) -> int:
         """Plan width (blocks) covering contexts of up to ``ctx`` tokens."""
         full = self.max_blocks
-        if not (self.LIVE_WIDTH and getattr(self, "attn_fused", False)
-                and getattr(self, "attn_splits", 1) > 1 and self.B * self.Hkv * 8 <= 256):
+        if not _plans_by_context(self):
             return full
         unit = max(8, -(-full // 8))
         need = -(-max(ctx, 1) // self.pool.block_size)
@@ -941,8 +947,6 @@ class DecodeEngine:
         Each replay's attention splits are planned for the contexts its steps
         can reach (every row's position advances by at most one per step)."""
         if self.graph is not None and steps >= self.MULTI_STEP:
-            if getattr(self, "_pos_stale", False):
-                self._pos_hi, self._pos_stale = int(self.pos.max()), False
             while steps >= self.MULTI_STEP:
                 pw = (self._live_width(self._pos_hi + self.MULTI_STEP)
                       if self._pos_hi is not None else None)
@@ -994,7 +998,7 @@ class DecodeEngine:
         self.generated.copy_(src.pad.view(1, 1).expand_as(self.generated))
         self.generated[:n].copy_(src.generated.index_select(0, idx))
         self._masks()
-        self._pos_hi, self._pos_stale = src._pos_hi, src._pos_stale
+        self._pos_hi = src._pos_hi
 
     def run_paged(self, sids: list, max_steps: int, chunk: Optional[int] = None,
                   check_invariants: bool = False, compact: Optional[list] = None) -> dict:
@@ -1079,7 +1083,7 @@ class DecodeEngine:
             if check_invariants:
                 pool.check_invariants()
             peak = max(peak, pool.num_blocks - pool.num_free)
-            eng._pos_hi, eng._pos_stale = max(pos), False
+            eng._pos_hi = max(pos)
             eng.run(n)
             steps += n
         for b in list(live):  # rows cut off by max_steps

@@ -41,7 +41,7 @@ def test_decode_start(dev, B, max_blocks, w, cols, kind):
     bt = torch.randint(0, 1 << 20, (B, w), dtype=torch.int32)
     DecodeEngine.start(s, tok.to(dev), pos.to(dev), bt.to(dev), lim.to(dev), cols, 5, 9)
     on = lim > 0
-    assert s.graph is None and s.graph_multi == {} and s._pos_stale and s._pos_hi is None
+    assert s.graph is None and s.graph_multi == {} and s._pos_hi is None
     assert torch.equal(s.tokens.cpu(), tok.view(B)) and int(s.eos) == 5 and int(s.pad) == 9
     assert torch.equal(s.pos.cpu(), pos.int()) and torch.equal(s.limit.cpu(), lim.int())
     assert not s.count.any() and torch.equal(s.active.cpu(), on)

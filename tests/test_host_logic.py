@@ -528,3 +528,49 @@ def test_steps_outside_run_move_the_position_bound():
     s.step()
     DecodeEngine.run(s, 18)
     assert s._pos_hi is None and s.widths[2] is None
+
+
+@pytest.mark.parametrize("rows,live,bound", [(8, True, 37), (32, True, None), (8, False, None)])
+def test_start_reads_the_position_bound_and_run_reads_nothing(monkeypatch, rows, live, bound):
+    """The bound on the positions is start()'s own work, where a plan depends on it, and
+    is not left for a later run() to read from the device."""
+    from grpo_mi355x import _lib
+    from grpo_mi355x.rollout.decode import DecodeEngine
+
+    monkeypatch.setattr(_lib, "stream_handle", lambda device=None: 0)
+
+    class Replay:
+        def replay(self):
+            pass
+
+    class Stand:
+        LIVE_WIDTH, MULTI_STEP, Hkv, attn_splits, attn_fused, _pos_hi = live, 16, 2, 8, True, None
+        max_blocks, device, graph, generated = 64, torch.device("cpu"), Replay(), None
+        pool = type("Pool", (), {"block_size": 16})
+        lib = type("Lib", (), {"grpo_decode_start": staticmethod(lambda *a: 0)})
+        step, _live_width = DecodeEngine.step, DecodeEngine._live_width
+
+        def __init__(self):
+            self.B = rows
+            for name in ("tokens", "count", "limit", "active", "eos", "pad", "append_pos",
+                         "attn_len", "block_tables"):
+                setattr(self, name, torch.zeros(1))
+
+        @property
+        def pos(self):
+            assert self.starting, "run() read the device"
+            return torch.zeros(1)
+
+        def _multi_graph(self, pw=None):
+            self.width = pw
+            return Replay()
+
+    s = Stand()
+    s.starting = True
+    pos = torch.arange(rows) % 8 + 30
+    DecodeEngine.start(s, pos, pos, torch.zeros(rows, 4, dtype=torch.int32), pos, 99, record=False)
+    assert s._pos_hi == bound
+    s.starting = False
+    DecodeEngine.run(s, 17)
+    assert s._pos_hi == (None if bound is None else bound + 17)
+    assert s.width == (None if bound is None else 8)
