@@ -1161,10 +1161,22 @@ class PrefillEngine(DecodeEngine):
         _run_chunks(self, table, prompt, n)
 
 
+def prefill_attention_pays(rows: int, kv_heads: int, tokens: int) -> bool:
+    """Whether a pass of ``rows`` rows of one sequence over contexts of up to ``tokens``
+    runs the prefill attention rather than the decode attention's row per workgroup.
+    The first walks the whole context once per 16 rows, however few those are (11 us
+    per 1000 tokens); the second's work grows with rows, KV heads and context over all
+    CUs.  Measured on MI355X, us, first / second: 128 rows x 2 KV heads after 1000 tokens
+    17.5 / 18.9, after 4000 49.0 / 46.4; 64 x 2 after 500 11.7 / 14.6, after 2000 28.1 / 22.3; 16
+    x 2 after nothing 6.3 / 7.0, after 500 11.7 / 7.8; 192 x 2 29.3 / 48.1 after 2000 and 90.9 /
+    167 after 8000."""
+    return rows * kv_heads >= 384 or tokens <= 4 * rows * kv_heads
+
+
 class GemmPrefillEngine:
     """Chunked paged prefill with wide chunks: up to ``chunk`` (default 512)
     prompt tokens of one sequence per pass, every linear on the NF4 GEMM
-    (``grpo_nf4_lora_linear`` beyond 64 rows: ``nf4_gemm_mfma``), so a
+    (``grpo_nf4_lora_linear`` beyond 64 rows: ``nf4_gemm.hip``), so a
     511-token prompt reads each NF4 weight once per row tile of one pass
     instead of once per 64-token chunk.
 
@@ -1173,17 +1185,20 @@ class GemmPrefillEngine:
     points: embedding -> per layer RMSNorm (+ the residual add of the previous
     layer's down_proj) -> q|k|v (grouped: one GEMM per projection, bias and
     LoRA in the kernel) -> RoPE + K/V append (``grpo_rope_append``) ->
-    attention over p + i + 1 tokens (``grpo_paged_attn_decode``) -> o_proj ->
+    attention over p + i + 1 tokens (``grpo_paged_attn_prefill``, or
+    ``grpo_paged_attn_decode``: ``prefill_attention_pays``) -> o_proj ->
     residual add + RMSNorm -> gate|up with SiLU*up in its epilogue
     (``grpo_nf4_gate_up_silu``) -> down_proj.  The reference
     prefills with one transformers forward and a per-token scatter of K/V
     (``paged_kv.py:547-586``).  Only the cache is filled: the last layer stops
     after its append (its attention and MLP feed nothing that is kept).  The
     pass is captured once into a HIP graph; rows past the end of a short last
-    chunk are masked (slot -1, length 0)."""
+    chunk are masked (slot -1, length 0).  ``max_tokens``: the longest prompt
+    expected (default: what the block table holds); it only steers the choice
+    of the attention."""
 
     def __init__(self, model: Qwen2ForCausalLM, pool: PagedKVPool, chunk: int, max_blocks: int,
-                 max_pos: Optional[int] = None):
+                 max_pos: Optional[int] = None, max_tokens: Optional[int] = None):
         self.lib = _lib.device_library()
         cfg = model.config
         self.model, self.pool, self.cfg = model, pool, cfg
@@ -1245,8 +1260,10 @@ class GemmPrefillEngine:
                     B, n, k, rr, nseg, self.bs)))
         # one workspace for every linear (they run one after another on one stream)
         self.ws = torch.empty(max(ws, 16), dtype=torch.uint8, device=dev)
+        tokens = max_blocks * pool.block_size
         self.attn_prefill = bool(self.lib.grpo_paged_attn_prefill_supported(
-            self.Hq, self.Hkv, D, pool.block_size))
+            self.Hq, self.Hkv, D, pool.block_size)) and prefill_attention_pays(
+                chunk, self.Hkv, tokens if max_tokens is None else min(tokens, max_tokens))
         self.ws_attn = ops.workspace("paged_attn_prefill", 1 if self.attn_prefill else max(
             ops.paged_attention_workspace_bytes(B, self.Hq, self.Hkv, D, pool.block_size,
                                                 max_blocks), 1), dev)
@@ -1405,7 +1422,7 @@ def prefill_engine(model: Qwen2ForCausalLM, pool: PagedKVPool, n: int, width: in
     ``PrefillEngine`` of ``prefill_chunk(n)`` rows."""
     if n > GEMM_PREFILL_MIN:
         chunk = min(GEMM_PREFILL_CHUNK, (n + 63) // 64 * 64)
-        return GemmPrefillEngine(model, pool, chunk, width, max_pos=max_pos)
+        return GemmPrefillEngine(model, pool, chunk, width, max_pos=max_pos, max_tokens=n)
     return PrefillEngine(model, pool, prefill_chunk(n), width, max_pos=max_pos)
 
 

@@ -96,10 +96,11 @@ def test_chunked_prefill_cache_matches_oracle(dev, chunk):
             assert e_ch <= 1e-2 and e_ch <= 2 * e_tf + 2e-3
 
 
-@pytest.mark.parametrize("chunk", [128, 192])
+@pytest.mark.parametrize("chunk", [16, 128, 192])
 def test_gemm_prefill_cache_matches_oracle(dev, chunk):
     """The wide-chunk prefill on the NF4 GEMM (``GemmPrefillEngine``): 149
-    cached tokens as 128 + 21 or in one 192-row pass.  Its cache is within the
+    cached tokens as 128 + 21, in one 192-row pass, or in passes of 16 rows, whose
+    attention is the decode kernel (``prefill_attention_pays``).  Its cache is within the
     bar of the oracle's and within twice the teacher-forced path's error plus
     2e-3; rows past the prompt and another sequence's blocks are untouched."""
     from grpo_mi355x.core.kv_pool import PagedKVPool
@@ -113,6 +114,7 @@ def test_gemm_prefill_cache_matches_oracle(dev, chunk):
     pool = PagedKVPool(layers, 3 * width, 2, 128, 16, device=dev)
     decoy = pool.allocate(width * 16)
     pre = GemmPrefillEngine(model, pool, chunk, width)
+    assert pre.attn_prefill == (chunk > 16)
     print(f"GEMM prefill: {n} tokens, chunk {chunk}", flush=True)
     sid = prefill(pre, pool, tuple(prompt), width)
     torch.cuda.synchronize()

@@ -574,3 +574,16 @@ def test_start_reads_the_position_bound_and_run_reads_nothing(monkeypatch, rows,
     DecodeEngine.run(s, 17)
     assert s._pos_hi == (None if bound is None else bound + 17)
     assert s.width == (None if bound is None else 8)
+
+
+def test_prefill_attention_choice():
+    """Wide passes and short contexts run the prefill attention; every engine that
+    prefill_engine makes (its chunk is the prompt, or 512 rows) does."""
+    from grpo_mi355x.rollout.decode import GEMM_PREFILL_CHUNK, prefill_attention_pays as pays
+
+    assert [pays(16, 2, t) for t in (16, 128, 129, 500)] == [True, True, False, False]
+    assert [pays(128, 2, t) for t in (1000, 1024, 1025, 4000)] == [True, True, False, False]
+    assert pays(192, 2, 8000) and pays(48, 8, 15000) and not pays(191, 2, 8000)
+    for n in (65, 128, 300, 511, 512, 513, 4000):
+        chunk = min(GEMM_PREFILL_CHUNK, (n + 63) // 64 * 64)
+        assert all(pays(chunk, hkv, n) for hkv in (1, 2, 4, 8))
