@@ -59,14 +59,16 @@ int g_target_waves = GRPO_TARGET_WAVES;  // launch-shape target: 8 waves per CU 
 
 // F16: float16_rne(code * absmax) instead of bf16 (the weight cast to a float16
 // grad / LoRA dtype in the reference's backward and forward).
-// Bound by memory (0.56 bytes read, 2 written per value): a thread decodes 8
-// nibbles into one 16-byte store, so a wave writes 1 KiB runs, with the byte-permute
-// lookup of the multiplying kernels; four words are in flight per thread.
-// 18944 x 3584: 27.3 us, 6.4 TB/s read and written (28.6 with 16 nibbles per thread
-// looked up in LDS and two strided stores).
-constexpr int DQ_T = 256, DQ_U = 4;
+// Bound by memory (0.56 bytes read, 2 written per value), small weights by the launch and
+// one round trip: a thread decodes 8 nibbles into one 16-byte store, so a wave writes
+// 1 KiB runs, with the byte-permute lookup of the multiplying kernels. One run per
+// thread up to 2^24 values, four in flight beyond: bf16, us, 256 x 1536 2.0 with one (2.5
+// with four; 2.1 with 16 nibbles per thread looked up in LDS and two strided stores),
+// 1536 x 1536 2.7 (3.3, 3.1), 8960 x 1536 7.3 (7.7, 8.9); 37888 x 3584 62 with four, 71 with one.
+constexpr int DQ_T = 256;
+constexpr int64_t DQ_FEW = 1 << 21;  // runs of 8 values
 
-template <bool F16, bool POW2>
+template <bool F16, bool POW2, int U>
 __global__ void __launch_bounds__(DQ_T) nf4_dequant_vec(const uint32_t* __restrict__ w,
                                                         const float* __restrict__ absmax,
                                                         const float* __restrict__ code16,
@@ -76,17 +78,17 @@ __global__ void __launch_bounds__(DQ_T) nf4_dequant_vec(const uint32_t* __restri
 #pragma unroll
   for (int j = 0; j < 16; ++j) code[j] = load_uniform(code16 + j);
   const int shift = __builtin_ctz(blocksize);
-  const int64_t i0 = (int64_t)blockIdx.x * (DQ_T * DQ_U) + threadIdx.x;
-  uint32_t wv[DQ_U];
-  float a[DQ_U];
+  const int64_t i0 = (int64_t)blockIdx.x * (DQ_T * U) + threadIdx.x;
+  uint32_t wv[U];
+  float a[U];
 #pragma unroll
-  for (int u = 0; u < DQ_U; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int64_t i = min(i0 + u * DQ_T, nvec - 1);
     wv[u] = w[i];
     a[u] = absmax[POW2 ? (8 * i) >> shift : (8 * i) / blocksize];
   }
 #pragma unroll
-  for (int u = 0; u < DQ_U; ++u) {
+  for (int u = 0; u < U; ++u) {
     const uint4 v = interleave8(decode8(wv[u], make_lut<F16>(code, a[u])));
     if (i0 + u * DQ_T < nvec) out[i0 + u * DQ_T] = v;
   }
@@ -2123,7 +2125,9 @@ int run_dequant(const uint8_t* w, const float* absmax, const float* code16, void
   if (numel == 0) return GRPO_OK;
   if (!w || !absmax || !code16 || !out) return einval("null pointer");
   hipStream_t st = as_stream(stream);
-  const int64_t nvec = numel / 8, blocks = cdiv(nvec, DQ_T * DQ_U);
+  const int64_t nvec = numel / 8;
+  const bool few = nvec <= DQ_FEW;
+  const int64_t blocks = cdiv(nvec, DQ_T * (few ? 1 : 4));
   if (numel % 8 == 0 && blocksize % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 3u) == 0 &&
       aligned16(out) && blocks < (1ll << 24)) {
     auto go = [&](auto kern) {
@@ -2131,8 +2135,9 @@ int run_dequant(const uint8_t* w, const float* absmax, const float* code16, void
                                                     code16, reinterpret_cast<uint4*>(out), nvec,
                                                     blocksize);
     };
-    if ((blocksize & (blocksize - 1)) == 0) go(nf4_dequant_vec<F16, true>);
-    else go(nf4_dequant_vec<F16, false>);
+    const bool pow2 = (blocksize & (blocksize - 1)) == 0;
+    if (few) pow2 ? go(nf4_dequant_vec<F16, true, 1>) : go(nf4_dequant_vec<F16, false, 1>);
+    else pow2 ? go(nf4_dequant_vec<F16, true, 4>) : go(nf4_dequant_vec<F16, false, 4>);
   } else {
     const int64_t blocks = std::min<int64_t>(cdiv(numel, 256), 8192);
     nf4_dequant_scalar<F16><<<dim3((unsigned)blocks), 256, 0, st>>>(

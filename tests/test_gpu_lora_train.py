@@ -130,7 +130,10 @@ def test_linear4bit_weight_layout_with_and_without_gradient(dev, m):
     _close(x.grad, g.double() @ w.double(), torch.bfloat16, "grad_x")
 
 
-@pytest.mark.parametrize("n,k,bs", [(1, 8, 8), (3, 24, 24), (65, 128, 64), (129, 1536, 4096)])
+@pytest.mark.parametrize("n,k,bs", [
+    (1, 8, 8), (3, 24, 24), (65, 128, 64), (129, 1536, 4096),
+    # one run of eight per thread up to 2^24 values, four beyond
+    (4096, 4096, 64), (4099, 4104, 64), (4097, 4104, 24)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_dequant_runs_of_eight(dev, n, k, bs, dt):
     """nf4_dequant's vector path over odd run counts and blocksizes, bit for bit with
