@@ -60,7 +60,8 @@ def test_embedding_pieces(dev, h):
 
 
 @pytest.mark.parametrize("hq,hkv,d,pad", [(12, 2, 128, 0), (28, 4, 128, 8), (1, 1, 16, 0),
-                                          (32, 8, 128, 0), (2, 1, 24, 0), (12, 2, 128, 4)])
+                                          (32, 8, 128, 0), (2, 1, 24, 0), (12, 2, 128, 4),
+                                          (2, 1, 128, 0), (6, 5, 32, 8)])
 def test_rope_append_pieces(dev, hq, hkv, d, pad):
     lib, check = _lib()
     rows, bs, blocks, cap = 37, 16, 24, 4
