@@ -202,7 +202,10 @@ class Linear4bitNF4(nn.Module):
         dt = torch.float16 if x.dtype == torch.float16 else torch.bfloat16
         w = self._dequantized_for(x, dt)
         bias = None if self.bias is None else self.bias.to(w.dtype)
-        return F.linear(x.to(w.dtype), w, bias)
+        x = x.to(w.dtype)
+        # rows that are not contiguous would make this (and its backward) a batched
+        # product over the expanded weight, one of the two with a transposed view of it
+        return F.linear(x if x.is_contiguous() else x.contiguous(), w, bias)
 
     def _dequantized_for(self, x: torch.Tensor, dt: torch.dtype) -> torch.Tensor:
         """``dequantize(dt)``, stored [in, out] where x's gradient will be asked for

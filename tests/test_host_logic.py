@@ -587,3 +587,33 @@ def test_prefill_attention_choice():
     for n in (65, 128, 300, 511, 512, 513, 4000):
         chunk = min(GEMM_PREFILL_CHUNK, (n + 63) // 64 * 64)
         assert all(pays(chunk, hkv, n) for hkv in (1, 2, 4, 8))
+
+
+@pytest.mark.parametrize("stored", ["rows", "columns"])
+def test_linear4bit_runs_no_batched_product(monkeypatch, stored):
+    """Inputs whose rows are not contiguous (transposed, sliced, expanded): forward and
+    backward stay plain products, in either layout of the weight."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from grpo_mi355x.core.nf4 import Linear4bitNF4
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.__name__.split(".")[0])
+            return func(*args, **(kwargs or {}))
+
+    w = torch.randn(32, 16).bfloat16()
+    kept = w if stored == "rows" else w.t().contiguous().t()
+    monkeypatch.setattr(Linear4bitNF4, "_dequantized_for", lambda self, x, dt: kept)
+    lin = Linear4bitNF4(16, 32, bias=False)
+    for x in (torch.randn(7, 2, 16).transpose(0, 1), torch.randn(2, 9, 16)[:, 1:8],
+              torch.randn(1, 7, 16).expand(2, 7, 16), torch.randn(2, 3, 4, 16).transpose(1, 2)):
+        x = x.bfloat16().detach().requires_grad_()
+        seen = []
+        with Seen():
+            y = lin(x)
+            y.backward(torch.ones_like(y))
+        assert "mm" in seen and not {"bmm", "baddbmm"} & set(seen)
+        assert x.grad.shape == x.shape
+        want = (x.detach().double() @ w.double().t())
+        assert torch.allclose(y.detach().double(), want, rtol=2e-2, atol=2e-2)
