@@ -5,7 +5,9 @@
 // compiler, which does not tell the ring's stages apart, would wait for all
 // outstanding loads before each LDS read. Its own waits for its own loads stay
 // correct, since loads retire in order and it only undercounts what is outstanding
-// (it then waits for more than it needs, never for less).
+// (it then waits for more than it needs, never for less). m0, which carries the LDS
+// address, is a reserved register: it cannot be named as clobbered, and the compiler sets
+// it anew before each instruction of its own that reads it.
 #pragma once
 
 #include "common.hpp"

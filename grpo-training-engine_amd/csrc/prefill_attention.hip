@@ -335,6 +335,19 @@ int go(const PrefillArgs& a, hipStream_t st) {
   return launch_check("prefill_attn");
 }
 
+// Heads per workgroup and parts of a step. Two heads in four parts while every workgroup
+// has a CU of its own (128 KiB of LDS), else up to four heads in two parts: 512 rows of
+// 12 / 2 heads 11.2 us against 14.7, of 28 / 4 heads 21.4 against 15.2 (each 0.4 more since
+// the look at values that are not finite).
+struct Form {
+  int heads, parts;
+};
+Form form_of(int M, int Hq, int Hkv) {
+  const int gq = Hq / Hkv;
+  if (cdiv(M, 16) * Hkv * cdiv(gq, 2) <= 256) return {std::min(gq, 2), 4};
+  return {gq > 2 ? 4 : gq, 2};
+}
+
 bool prefill_ok(int Hq, int Hkv, int D, int block_size) {
   return Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && D == PD && block_size == PBS &&
          (int64_t)Hq < 65536;
@@ -344,6 +357,15 @@ bool prefill_ok(int Hq, int Hkv, int D, int block_size) {
 
 extern "C" int grpo_paged_attn_prefill_supported(int Hq, int Hkv, int D, int block_size) {
   return prefill_ok(Hq, Hkv, D, block_size) ? 1 : 0;
+}
+
+extern "C" int grpo_paged_attn_prefill_plan(int M, int Hq, int Hkv, int* heads, int* parts) {
+  if (M < 1 || !heads || !parts || !prefill_ok(Hq, Hkv, PD, PBS))
+    return einval("bad attention dimensions");
+  const Form f = form_of(M, Hq, Hkv);
+  *heads = f.heads;
+  *parts = f.parts;
+  return GRPO_OK;
 }
 
 extern "C" int grpo_paged_attn_prefill(const void* q, int64_t q_stride_b, int64_t q_stride_h,
@@ -368,11 +390,8 @@ extern "C" int grpo_paged_attn_prefill(const void* q, int64_t q_stride_b, int64_
                       static_cast<const uint16_t*>(v_cache), num_blocks, block_table, lens,
                       static_cast<uint16_t*>(out), M, Hq, Hkv, max_blocks, scale};
   hipStream_t st = as_stream(stream);
-  // Two heads in four parts while every workgroup has a CU of its own (128 KiB of
-  // LDS), else up to four heads in two parts, two workgroups per CU: 512 rows of 12 / 2
-  // heads 11.2 us against 14.7, of 28 / 4 heads 21.4 against 15.2.
-  const int gq = Hq / Hkv;
-  if (cdiv(M, 16) * Hkv * cdiv(gq, 2) <= 256) return gq == 1 ? go<1, 4>(a, st) : go<2, 4>(a, st);
-  if (gq == 1) return go<1, 2>(a, st);
-  return gq == 2 ? go<2, 2>(a, st) : go<4, 2>(a, st);
+  const Form f = form_of(M, Hq, Hkv);
+  if (f.parts == 4) return f.heads == 1 ? go<1, 4>(a, st) : go<2, 4>(a, st);
+  if (f.heads == 1) return go<1, 2>(a, st);
+  return f.heads == 2 ? go<2, 2>(a, st) : go<4, 2>(a, st);
 }

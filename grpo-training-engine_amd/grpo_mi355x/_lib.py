@@ -120,6 +120,8 @@ SIGNATURES = {
          _I32, _VP, _SZ, _VP],
     ),
     "grpo_paged_attn_prefill_supported": (_I32, [_I32, _I32, _I32, _I32]),
+    "grpo_paged_attn_prefill_plan": (
+        _I32, [_I32, _I32, _I32, _c.POINTER(_I32), _c.POINTER(_I32)]),
     "grpo_paged_attn_prefill": (
         _I32,
         [_VP, _I64, _I64, _VP, _VP, _I64, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _F32,

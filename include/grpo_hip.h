@@ -870,6 +870,9 @@ int grpo_sample_advance(const void* logits, int64_t ld_logits, int M, int V, flo
  * Needs head_dim 128, block size 16 and 16-byte aligned rows and caches
  * (grpo_paged_attn_prefill_supported; alignment aside). No workspace. */
 int grpo_paged_attn_prefill_supported(int Hq, int Hkv, int D, int block_size);
+/* The form that M rows run in: query heads per workgroup and the groups of waves that
+ * share a step's tokens. */
+int grpo_paged_attn_prefill_plan(int M, int Hq, int Hkv, int* heads, int* parts);
 int grpo_paged_attn_prefill(const void* q, int64_t q_stride_b, int64_t q_stride_h,
                             const void* k_cache, const void* v_cache, int64_t num_blocks,
                             const int32_t* block_table, const int32_t* lens, void* out, int M,

@@ -3,8 +3,9 @@ pinned against the oracle (tests/test_gpu_attention.py), and against float64.
 
 Both kernels hold float32 scores, sums and P (as two bf16 terms) and round once to
 bf16; they differ in the order of the sums, so a result can fall to the other
-neighbouring bf16 value: within one ulp (2^-7 of the larger), most of them equal."""
+neighbouring bf16 value: within one ulp (2^-7 of the value at most), most of them equal."""
 
+import ctypes
 import math
 
 import pytest
@@ -42,6 +43,16 @@ def _run(dev, M, Hq, Hkv, lens, max_blocks, seed, holes=()):
     return out.float(), want, (q, k, v, table)
 
 
+def _form(M, Hq, Hkv):
+    """(heads per workgroup, parts of a step) that the launcher picks."""
+    from grpo_mi355x import _lib
+
+    h, p = ctypes.c_int(0), ctypes.c_int(0)
+    _lib.check(_lib.library().grpo_paged_attn_prefill_plan(M, Hq, Hkv, ctypes.byref(h),
+                                                           ctypes.byref(p)), "plan")
+    return h.value, p.value
+
+
 # rows: within, at and past a 16-row tile; contexts: within a block, at and past the 32-token
 # parts, the 128-token steps, the ring of two, the 64-block table windows, empty and clamped ones
 @pytest.mark.parametrize("M,Hq,Hkv,first,max_blocks", [
@@ -62,10 +73,30 @@ def test_prefill_attention(dev, M, Hq, Hkv, first, max_blocks):
         assert not got[3].any() and not got[5].any()
 
 
+# More workgroups than CUs: two parts of 32 tokens per 64-token step (a 64-block table window
+# is 16 of them), one, two and four heads per workgroup, the last with and without an idle
+# wave; contexts from one step to several windows, one that ends with a step and a window
+@pytest.mark.parametrize("M,Hq,Hkv,form", [(528, 8, 8, (1, 2)), (528, 16, 8, (2, 2)),
+                                           (512, 28, 4, (4, 2)), (530, 32, 8, (4, 2)),
+                                           (520, 6, 2, None), (1300, 6, 2, (4, 2))])
+@pytest.mark.parametrize("first,max_blocks", [(1, 40), (1000, 128), (2040, 210)])
+def test_prefill_attention_in_two_parts(dev, M, Hq, Hkv, form, first, max_blocks):
+    assert _form(M, Hq, Hkv) == (form or (2, 4))
+    lens = [first + i // 2 for i in range(M)]
+    lens[3], lens[5], lens[-1] = 0, -4, 16 * max_blocks + 50
+    lens[96:112] = [1024] * 16
+    got, want, _ = _run(dev, M, Hq, Hkv, lens, max_blocks, M + Hq)
+    assert float(((got - want).abs() / want.abs().clamp(min=1e-3)).max()) <= 2.0 ** -7
+    assert float((got == want.bfloat16().float()).float().mean()) >= 0.97
+    assert not got[3].any() and not got[5].any()
+
+
+@pytest.mark.parametrize("M,Hq,Hkv", [(50, 6, 1), (528, 8, 8), (528, 16, 8), (512, 28, 4)])
 @pytest.mark.parametrize("first,max_blocks,holes", [
     (20, 12, (1, 6)), (1000, 80, (0, 62, 63, 64, 65, 66)), (1, 3, (0, 1, 2))])
-def test_prefill_attention_skips_invalid_blocks(dev, first, max_blocks, holes):
-    got, want, _ = _run(dev, 50, 6, 1, [first + 3 * i for i in range(50)], max_blocks, 5, holes)
+def test_prefill_attention_skips_invalid_blocks(dev, first, max_blocks, holes, M, Hq, Hkv):
+    got, want, _ = _run(dev, M, Hq, Hkv, [first + 3 * (i % 50) for i in range(M)], max_blocks, 5,
+                        holes)
     assert torch.isfinite(got).all()
     assert float(((got - want).abs() / want.abs().clamp(min=1e-3)).max()) <= 2.0 ** -7
 
@@ -78,7 +109,7 @@ def test_prefill_attention_against_float64(dev):
     on = torch.arange(kk.shape[0], device=dev) < torch.arange(100, 196, device=dev)[:, None]
     p = torch.softmax(s.masked_fill(~on[:, None], -math.inf), -1)
     want = torch.einsum("mht,thd->mhd", p, vv)
-    # one rounding to bf16: half an ulp, 2^-9, with a little for the float32 sums
+    # one rounding to bf16, 2^-8 of the value at most, with a little for the float32 sums
     assert float(((got - want).abs() / want.abs().clamp(min=1e-2)).max()) <= 1.05 * 2.0 ** -8
 
 
