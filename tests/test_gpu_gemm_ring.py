@@ -15,26 +15,40 @@ import torch
 
 from conftest import rel_err, to_dev_bf16
 from oracle.bf16 import bf16_bits_to_f32
+from test_gemm_plan import plan
 from test_gpu_gemm import _check
 from test_gpu_nf4 import _code, make_linear_case, oracle_linear, run_linear
 
 pytestmark = pytest.mark.gpu
 
+# m, n, k, r, bias, blocksize, (rows, columns, K groups, K slices)
 CASES = [
-    (65, 72, 128, 16, True, 64),     # one superstage: the second K group has none
-    (66, 80, 384, 5, True, 128),     # 2 + 1 superstages, r % 8 != 0 (scalar LoRA B loads)
-    (129, 1027, 640, 1, False, 64),  # 3 + 2, N % 8 != 0 (element stores), rank 1
-    (513, 320, 256, 0, True, 256),   # an absmax block of two superstages
-    (257, 4104, 896, 12, True, 64),  # 128-row tiles with LoRA, 4 + 3 superstages
-    (1030, 2056, 128, 16, True, 64), # several rounds of workgroups, one superstage
-    (1025, 16392, 256, 0, True, 64), # 256 x 256 tiles, one row and 8 columns past them
-    (200, 528, 1920, 16, True, 64),  # K split (15 superstages)
-    (140, 96, 4224, 0, False, 64),   # K split without LoRA, 33 superstages
+    (65, 72, 128, 16, True, 64, (64, 64, 2, 1)),     # one superstage: the second K group has none
+    (66, 80, 384, 5, True, 128, (64, 64, 2, 1)),     # 2 + 1, r % 8 != 0 (scalar LoRA B loads)
+    (129, 1027, 640, 1, False, 64, (64, 64, 2, 1)),  # 3 + 2, N % 8 != 0 (element stores), rank 1
+    (513, 320, 256, 0, True, 256, (64, 64, 2, 1)),   # an absmax block of two superstages
+    (257, 4104, 896, 12, True, 64, (64, 128, 2, 1)), # 4 + 3
+    (257, 3600, 1920, 0, True, 64, (64, 128, 2, 1)),
+    (1030, 2056, 128, 16, True, 64, (128, 128, 1, 1)),   # several rounds of workgroups
+    (1025, 16392, 256, 0, True, 64, (128, 128, 1, 1)),
+    (200, 8208, 640, 16, True, 64, (128, 128, 2, 1)),
+    (200, 8208, 896, 0, False, 64, (128, 128, 2, 1)),
+    (2049, 4104, 512, 0, True, 64, (256, 256, 1, 1)),  # one row and 8 columns past the tiles
+    # K split, each tile that has it with and without LoRA
+    (200, 528, 1920, 16, True, 64, (64, 64, 2, 4)),
+    (140, 96, 4224, 0, False, 64, (64, 64, 2, 9)),
+    (65, 2064, 4224, 16, True, 64, (64, 128, 2, 6)),
+    (65, 2320, 7936, 0, True, 64, (64, 128, 2, 6)),
+    (65, 3600, 4224, 0, True, 64, (128, 128, 1, 7)),
+    (65, 6192, 3456, 16, True, 64, (128, 128, 1, 9)),
+    (65, 4112, 4224, 0, False, 64, (128, 128, 2, 6)),
+    (65, 4112, 4224, 16, True, 64, (128, 128, 2, 6)),
 ]
 
 
-@pytest.mark.parametrize("m,n,k,r,with_bias,bs", CASES)
-def test_ring_gemm_matches_oracle(dev, m, n, k, r, with_bias, bs):
+@pytest.mark.parametrize("m,n,k,r,with_bias,bs,tile", CASES)
+def test_ring_gemm_matches_oracle(dev, m, n, k, r, with_bias, bs, tile):
+    assert plan(m, n, k, r, bs) == tile  # what the case is for
     print(f"ring gemm m={m} n={n} k={k} r={r} bias={with_bias} bs={bs}", flush=True)
     c = make_linear_case(m + n + k + r, m, n, k, r, with_bias, bs=bs)
     _check(run_linear(dev, c), oracle_linear(c))
@@ -76,13 +90,16 @@ def test_ring_gemm_infinite_t_reaches_only_its_ranks(dev):
     assert np.all(np.isposinf(y))
 
 
-@pytest.mark.parametrize("m,i,k", [(65, 8, 128), (130, 1000, 384), (1030, 264, 896),
-                                   (513, 17416, 256)])
-def test_ring_gate_up_silu_matches_float32(dev, m, i, k):
+@pytest.mark.parametrize("m,i,k,tile", [
+    (65, 8, 128, (128, 128, 1, 1)), (130, 1000, 384, (128, 128, 1, 1)),
+    (1030, 264, 896, (128, 128, 2, 1)), (513, 17416, 256, (128, 128, 1, 1)),
+    (513, 8200, 384, (256, 256, 1, 1))])  # one row and 8 columns past the tiles
+def test_ring_gate_up_silu_matches_float32(dev, m, i, k, tile):
     """SiLU(gate) * up of the stacked weight against the same formula on the oracle's
     bf16 gate and up: two roundings after them, so 2^-7 of the largest output."""
     from grpo_mi355x import _lib
 
+    assert plan(m, i, k, 0, silu=1) == tile
     lib = _lib.device_library()
     c = make_linear_case(m + i + k, m, 2 * i, k, 0, False)
     gu = torch.from_numpy(bf16_bits_to_f32(oracle_linear(c)))
