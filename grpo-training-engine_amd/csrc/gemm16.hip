@@ -231,25 +231,34 @@ int go(Args a, hipStream_t st) {
   return launch_check("gemm16");
 }
 
-template <bool F16, Gemm16Mode MODE>
-int pick(const Args& a, hipStream_t st) {
-  // Microseconds per stage of each tile, measured: alone on a CU, and per tile of
-  // a full chip. The tile with the least time for its count per CU runs:
-  // 256 x 256 once the chip is full of them (1189 TFLOP/s; 837 with 128 x 128),
-  // the smaller ones where a larger tile would leave CUs without work (2092 x 1536 x
-  // 1536: 33.1, 18.1, 22.0 and 28.0 us with the four tiles; 662 rows: 31.4, 12.5, 9.5
-  // and 9.7; 256 x 1024 x 1024: 22.4, 8.9, 6.5 and 5.4).
-  static constexpr struct { int bm, bn; double alone, full; } TILE[4] = {
-      {256, 256, 0.70, 0.79}, {128, 128, 0.32, 0.281}, {64, 128, 0.198, 0.231},
-      {64, 64, 0.165, 0.136}};
+// Microseconds per stage of each tile, measured: alone on a CU, and per tile of
+// a full chip. The tile with the least time for its count per CU runs:
+// 256 x 256 once the chip is full of them (1189 TFLOP/s; 837 with 128 x 128),
+// the smaller ones where a larger tile would leave CUs without work (2092 x 1536 x
+// 1536: 33.1, 18.1, 22.0 and 28.0 us with the four tiles; 662 rows: 31.4, 12.5, 9.5
+// and 9.7; 256 x 1024 x 1024: 22.4, 8.9, 6.5 and 5.4).
+constexpr struct {
+  int bm, bn;
+  double alone, full;
+} TILE[4] = {{256, 256, 0.70, 0.79},
+             {128, 128, 0.32, 0.281},
+             {64, 128, 0.198, 0.231},
+             {64, 64, 0.165, 0.136}};
+
+int tile_of(int M, int N) {
   int best = 0;
   double least = 0.0;
   for (int i = 0; i < 4; ++i) {
-    const int64_t tiles = cdiv(a.g.M, TILE[i].bm) * cdiv(a.g.N, TILE[i].bn);
+    const int64_t tiles = cdiv(M, TILE[i].bm) * cdiv(N, TILE[i].bn);
     const double us = std::max(TILE[i].alone, TILE[i].full * (double)cdiv(tiles, 256));
     if (i == 0 || us < least) best = i, least = us;
   }
-  switch (best) {
+  return best;
+}
+
+template <bool F16, Gemm16Mode MODE>
+int pick(const Args& a, hipStream_t st) {
+  switch (tile_of(a.g.M, a.g.N)) {
     case 0: return go<F16, MODE, 8, 4, 2, 4, 4>(a, st);
     case 1: return go<F16, MODE, 4, 4, 2, 2, 8>(a, st);
     case 2: return go<F16, MODE, 2, 4, 2, 2, 8>(a, st);
@@ -282,3 +291,11 @@ int gemm16_launch(const Gemm16& g, Gemm16Mode mode, bool f16, hipStream_t st) {
 }
 
 }  // namespace grpo
+
+extern "C" int grpo_gemm16_tile(int M, int N, int* rows, int* cols) {
+  using namespace grpo;
+  if (M < 1 || N < 1 || !rows || !cols) return einval("bad GEMM dimensions");
+  *rows = TILE[tile_of(M, N)].bm;
+  *cols = TILE[tile_of(M, N)].bn;
+  return GRPO_OK;
+}

@@ -78,6 +78,7 @@ SIGNATURES = {
     "grpo_nf4_grad_x": (_I32, [_VP, _I64, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _VP, _I64, _VP,
                                 _I64, _VP]),
     "grpo_nf4_dequant_t": (_I32, [_VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _VP]),
+    "grpo_gemm16_tile": (_I32, [_I32, _I32, _c.POINTER(_I32), _c.POINTER(_I32)]),
     "grpo_nf4_lora_train_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32, _I32]),
     "grpo_nf4_lora_train_forward": (
         _I32,

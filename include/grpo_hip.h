@@ -101,6 +101,9 @@ int grpo_nf4_dequant_t(const uint8_t* w, const float* absmax, const float* code1
  * not supported: N % 32, K % 32 != 0, r outside [1, 32] or a blocksize that is
  * not a power of two >= 32).  Holds the weight in 16 bits. */
 size_t grpo_nf4_lora_train_workspace_bytes(int M, int N, int K, int r, int blocksize);
+/* The tile of rows x columns that the training linear's 16-bit GEMM takes for M rows of
+ * N outputs (forward; grad_x: M rows of K). */
+int grpo_gemm16_tile(int M, int N, int* rows, int* cols);
 
 /* The fused linear for training batches, _lora_forward_kernel (src/
  * triton_kernels/lora_forward.py:107-260) as two launches: W in dt and t = dt(x
