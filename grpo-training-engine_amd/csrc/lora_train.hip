@@ -6,8 +6,10 @@
 //   grad_A = dt(gi^T x)               grad_B = dt(dt(g * dt(s))^T xa)
 //   grad_x = dt(dt(g W) + dt(gi A))   y = dt(dt(dt(x W^T) [+ bias]) + dt(dt(t B^T) * dt(s)))
 //
-// The weight is decoded once per call, not once per row tile: at 512 rows and more
-// the two passes over N x K 16-bit values cost less than the decode repeated.
+// The weight is decoded once per call, not once per row tile: from about 5 million
+// outputs (fewer where the decoding GEMM's ring kernel does not run) the two passes over
+// N x K 16-bit values cost less than the decode repeated; the backward, which needs the
+// weight transposed, always takes them.
 // The products of rank r are bound by one read of x and g (M x K and M x N
 // 16-bit values), so they are MFMA tiles fed straight from global memory in the
 // row-major layout the caller has: no transposed or scaled copies are written.

@@ -486,8 +486,8 @@ __global__ void __launch_bounds__(256) nf4_finish_rows(LinParts o, uint16_t* __r
 //    1 KiB piece), absmax (one per row and stage) and LoRA A rows come to LDS too,
 //    into a ring of three: the one being decoded, the next and the one being fetched.
 //  * Step st multiplies stage st, decodes stage st + 2 (a thread: 8 or 16 nibbles of
-//    one row, whose codebook is built once per stage, or per two where the absmax
-//    block has 64 values or more), fetches stage st + 3 of x and a quarter of the
+//    one row, whose codebook is built once per two stages: an absmax block has 64
+//    values at least), fetches stage st + 3 of x and a quarter of the
 //    superstage after next. The decoded stages alternate between two LDS slots: the
 //    slot written in step st was read before its barrier. Every wait counts loads.
 //  * LoRA: x A^T is one more MFMA column of the tile, its rows shared out among the

@@ -212,7 +212,8 @@ class Linear4bitNF4(nn.Module):
         and out >= 2 in: grad_x = g W is then a product along contiguous rows.
         Library GEMMs, forward + backward, out 8960, in 1536 (us): 71 -> 57 at 512
         rows, 103 -> 73 at 1024; 9216 x 2048 108 -> 89 at 1024, 190 -> 196 at 2800; the
-        other way round for a wide in (1536 x 8960: 75 -> 109 at 1024)."""
+        other way round for a wide in (1536 x 8960: 75 -> 109 at 1024). Not measured for in
+        above 2048, which keeps the row-major weight."""
         n, k = self.out_features, self.in_features
         if (n >= 2 * k and 1024 <= k <= 2048 and x.requires_grad and torch.is_grad_enabled()
                 and x.numel() <= 2048 * k):
