@@ -36,7 +36,7 @@
 // bf16 with K % 128 == 0, r <= 16 and blocksize >= 64 runs nf4_gemm_k2 (below) instead:
 // with the tile and slices that its time model picks it was slower at 2 of 560 measured
 // shapes of 65 .. 4096 rows (224 x 4608 x 3584 6 %, 1024 x 1536 x 8960 3 %), at the median
-// 0.77 of the time, its SiLU form 0.68 .. 0.93; profiles/nf4_gemm_wide_batches.md.
+// 0.77 of the time, its SiLU form 0.68 .. 0.93.
 #include <algorithm>
 #include <type_traits>
 
